@@ -126,54 +126,55 @@ SCPHD_HD inline double uniform_oc(uint32_t lo, uint32_t hi) { /* (0, 1] */
  *       and cos(pi/4 t) = C(t^2) are Taylor polynomials to t^9 and t^8
  *       (|error| < 4e-8);
  *   r = sqrt(-2 log a); z0 = r cos 2 pi c, z1 = r sin 2 pi c (single
- *   precision; box_muller widens them to double). */
-/* The correctly rounded single-precision square root of x = +-0 or x in
- * [2^-96, 2^128): the hardware root (within 1 ulp for such x) moved by one
- * ulp down or up when the residual x - s'^2 of that neighbour shows it is
- * the nearer root, the same correction as the compiler's IEEE sqrt, without
- * its scaling of tiny inputs and its special cases (+-0 pass through the
- * correction unchanged: the neighbour below is a NaN, the one above gives a
- * zero residual). */
-__device__ inline float sqrt_rn_normal(float x) {
-    const float s = __builtin_amdgcn_sqrtf(x);
-    const float dn = __uint_as_float(__float_as_uint(s) - 1u);
-    const float up = __uint_as_float(__float_as_uint(s) + 1u);
-    float r = __builtin_fmaf(-dn, s, x) <= 0.0f ? dn : s;
-    r = __builtin_fmaf(-up, s, x) > 0.0f ? up : r;
-    return r;
+ *   precision; box_muller widens them to double).
+ *
+ * The kernels that draw normals are bound by VALU issue, and this is half of
+ * their instructions, so its integer work is kept short: 51 instructions a
+ * pair instead of 64 for the same bits (checked for every x0 and every
+ * x1 >> 8).
+ *   - x0 + 1 in double is exact, x0 = 2^32 - 1 included; its exponent and
+ *     leading 23 fraction bits are one alignbit away from the layout of a
+ *     float (the exponent modulo 256), and one add of 1.0's bits less those
+ *     of the smallest f moves the fractions above sqrt(2) to the next e.
+ *   - P's coefficients and ln2 carry the factor -2 (a power of two: exact).
+ *   - t = min(r, 2 - r) for r the offset in a quarter turn, a float's
+ *     fraction bits as they are.
+ *   - The quadrant's signs and the exchange of sin and cos are bits 31 and
+ *     30 of x1 and of y = x1 ^ 2 x1. */
+
+/* The correctly rounded single-precision square root of x = -0 or x in
+ * [2^-23, 89), the values of -2 log a: the hardware's 1/sqrt (within 1 ulp)
+ * and one Goldschmidt step, whose residual x - g^2 is exact.  Checked
+ * against the correctly rounded root for every a.  (x = -0 gives -0: its
+ * reciprocal root is taken of a small positive number instead.) */
+__device__ inline float sqrt_rn_log(float x) {
+    const float r = __builtin_amdgcn_rsqf(__builtin_fmaxf(x, 0x1p-64f));
+    const float g = x * r, h = 0.5f * r;
+    return __builtin_fmaf(__builtin_fmaf(-g, g, x), h, g);
 }
 
 __device__ inline void box_muller_f(uint32_t x0, uint32_t x1, float& z0, float& z1) {
 #pragma clang fp contract(off)
-    const uint32_t n = x0 + 1u; /* 0 stands for a = 1 (log a = 0) */
-    const uint32_t nn = n != 0u ? n : 1u;
-    const int lz = __clz((int)nn);
-    const uint32_t m = nn << lz; /* [2^31, 2^32) */
-    float f = __uint_as_float(0x3F800000u | ((m >> 8) & 0x7FFFFFu)); /* (m >> 8) 2^-23, in [1, 2) */
-    int e = -1 - lz;
-    if (f > 0x1.6a09e6p+0f) {
-        f *= 0.5f;
-        e += 1;
-    }
+    constexpr uint32_t F_MIN = 0x3F3504F4u; /* the smallest f: half of the first float above 0x1.6a09e6p+0 */
+    const double a = (double)x0 + 1.0;      /* a 2^32 */
+    const uint32_t ix = __builtin_amdgcn_alignbit((uint32_t)__double2hiint(a), (uint32_t)__double2loint(a), 29) +
+                        (0x00800000u + 0x3F800000u - F_MIN); /* e + 32 above bit 23 */
+    const float f = __uint_as_float((ix & 0x7FFFFFu) + F_MIN);
+    const int e = (int)(ix >> 23) - 32;
     const float sx = f - 1.0f;
-    float pl = 0x1.6626eap-4f;
-    pl = __builtin_fmaf(pl, sx, -0x1.26729ep-3f);
-    pl = __builtin_fmaf(pl, sx, 0x1.322850p-3f);
-    pl = __builtin_fmaf(pl, sx, -0x1.5329bep-3f);
-    pl = __builtin_fmaf(pl, sx, 0x1.98b80ap-3f);
-    pl = __builtin_fmaf(pl, sx, -0x1.0005a6p-2f);
-    pl = __builtin_fmaf(pl, sx, 0x1.555790p-2f);
-    pl = __builtin_fmaf(pl, sx, -0x1.fffff8p-2f);
-    pl = __builtin_fmaf(pl, sx, 1.0f);
-    const float lf = sx * pl;
-    const float L = n != 0u ? __builtin_fmaf((float)e, 0x1.62e430p-1f, lf) : 0.0f;
-    /* -2 L is -0 (a = 1) or at least 2^-23 (a <= 1 - 2^-24): correctly
-     * rounded without the tiny-input path */
-    const float r = sqrt_rn_normal(-2.0f * L);
-    const uint32_t c = x1 >> 8;
-    const uint32_t oct = c >> 21;
-    const uint32_t fr = c & 0x1FFFFFu;
-    const float t = (float)((oct & 1u) ? (0x200000u - fr) : fr) * 0x1.0p-21f;
+    float pl = -0x1.6626eap-3f;
+    pl = __builtin_fmaf(pl, sx, 0x1.26729ep-2f);
+    pl = __builtin_fmaf(pl, sx, -0x1.322850p-2f);
+    pl = __builtin_fmaf(pl, sx, 0x1.5329bep-2f);
+    pl = __builtin_fmaf(pl, sx, -0x1.98b80ap-2f);
+    pl = __builtin_fmaf(pl, sx, 0x1.0005a6p-1f);
+    pl = __builtin_fmaf(pl, sx, -0x1.555790p-1f);
+    pl = __builtin_fmaf(pl, sx, 0x1.fffff8p-1f);
+    pl = __builtin_fmaf(pl, sx, -2.0f);
+    const float r = sqrt_rn_log(__builtin_fmaf((float)e, -0x1.62e430p+0f, sx * pl));
+    const uint32_t quarter = (x1 >> 8) & 0x3FFFFFu; /* 2^22 to the quarter turn */
+    const uint32_t tri = min(quarter, 0x400000u - quarter);
+    const float t = __uint_as_float((tri << 2) + 0x3F800000u) - 1.0f;
     const float t2 = t * t;
     float ps = 0x1.507834p-22f;
     ps = __builtin_fmaf(ps, t2, -0x1.32d2ccp-15f);
@@ -188,13 +189,14 @@ __device__ inline void box_muller_f(uint32_t x0, uint32_t x1, float& z0, float& 
     pc = __builtin_fmaf(pc, t2, 1.0f);
     /* quadrant angle phi = 2 pi c - q pi/2: odd octants measure t from pi/2
      * (sin and cos exchanged), odd quadrants exchange them again, so one
-     * exchange when exactly one applies; the quadrant's signs are sign-bit
-     * flips: -cos for q = 1, 2 and -sin for q = 2, 3 */
-    const uint32_t q = oct >> 1;
-    const bool swap = ((oct ^ q) & 1u) != 0u;
+     * exchange when exactly one applies (bits 29 and 30 of x1 differ); the
+     * quadrant's signs are sign-bit flips: -cos for q = 1, 2 (bits 30 and 31
+     * differ) and -sin for q = 2, 3 (bit 31) */
+    const uint32_t y = x1 ^ (x1 << 1);
+    const bool swap = (y & 0x40000000u) != 0u;
     const float sn0 = swap ? pc : sv, cs0 = swap ? sv : pc;
-    const float sn = __uint_as_float(__float_as_uint(sn0) ^ ((q & 2u) << 30));
-    const float cs = __uint_as_float(__float_as_uint(cs0) ^ (((q + 1u) & 2u) << 30));
+    const float sn = __uint_as_float(__float_as_uint(sn0) ^ (x1 & 0x80000000u));
+    const float cs = __uint_as_float(__float_as_uint(cs0) ^ (y & 0x80000000u));
     z0 = r * cs;
     z1 = r * sn;
 }
