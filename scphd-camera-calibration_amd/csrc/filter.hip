@@ -97,74 +97,77 @@ hipError_t grow_keep(DBuf<T>& b, int64_t need, int64_t keep, hipStream_t s) {
     return hipSuccess;
 }
 
-/* One generation of sample blocks: 7 planes of float or double. */
+/* One generation of sample blocks, in SLABS slabs (Clouds). */
 struct Generation {
-    void* pl[7] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
-    size_t pbytes[7] = {};
+    void* sl[SLABS] = {};
+    size_t sbytes[SLABS] = {};
     int64_t cap_blocks = 0;
     std::vector<Block>* retired = nullptr; /* the owning handle's list */
     void release() {
-        for (int c = 0; c < 7; ++c) {
-            retire(retired, pl[c], pbytes[c]);
-            pl[c] = nullptr;
-            pbytes[c] = 0;
+        for (int c = 0; c < SLABS; ++c) {
+            retire(retired, sl[c], sbytes[c]);
+            sl[c] = nullptr;
+            sbytes[c] = 0;
         }
         cap_blocks = 0;
     }
-    /* grow to at least need blocks keeping the first keep blocks.  Planes
+    /* grow to at least need blocks keeping the first keep blocks.  Slabs
      * are replaced one at a time (allocate, copy the kept blocks, wait, hand
-     * the old plane back), so the transient is one plane, not a whole
-     * generation; if an allocation fails, every plane still holds the kept
+     * the old slab back), so the transient is one slab, not a whole
+     * generation; if an allocation fails, every slab still holds the kept
      * blocks and at least the old capacity, which stays the recorded one.
      * Keeping blocks happens only while no other stream works on the
-     * generation, so after the wait an old plane goes straight to the cache.
+     * generation, so after the wait an old slab goes straight to the cache.
      * drained: no queued work touches the generation, so with nothing to
-     * keep its planes go straight to the cache too, where the allocations
+     * keep its slabs go straight to the cache too, where the allocations
      * that follow can reuse or free them. */
     hipError_t ensure(int64_t need, int64_t keep, int S, size_t esz, hipStream_t s, bool drained = false) {
         if (need <= cap_blocks) return hipSuccess;
         const int64_t cap = std::max<int64_t>(need + need / 4, 16);
+        const size_t block = (size_t)cloud_stride(S, esz) * esz;
         if (keep <= 0 && drained) {
-            for (int c = 0; c < 7; ++c) {
-                if (pl[c]) cache_put(Block{pl[c], pbytes[c]});
-                pl[c] = nullptr;
-                pbytes[c] = 0;
+            for (int c = 0; c < SLABS; ++c) {
+                if (sl[c]) cache_put(Block{sl[c], sbytes[c]});
+                sl[c] = nullptr;
+                sbytes[c] = 0;
             }
             cap_blocks = 0;
         } else if (keep <= 0) {
             release(); /* nothing to keep: release first, then allocate */
         }
         int64_t got = INT64_MAX;
-        for (int c = 0; c < 7; ++c) {
+        for (int c = 0; c < SLABS; ++c) {
             void* np = nullptr;
-            size_t b = (size_t)cap * S * esz;
+            size_t b = (size_t)((cap + SLABS - 1) / SLABS) * block;
+            const size_t kept = (size_t)((keep - c + SLABS - 1) / SLABS) * block; /* of blocks c, c + SLABS, .. */
             hipError_t e = cache_alloc(&np, &b);
             if (e != hipSuccess) {
                 if (keep <= 0) release();
                 return e;
             }
-            if (keep > 0 && pl[c]) {
-                e = hipMemcpyAsync(np, pl[c], (size_t)keep * S * esz, hipMemcpyDeviceToDevice, s);
+            if (keep > 0 && sl[c]) {
+                e = kept ? hipMemcpyAsync(np, sl[c], kept, hipMemcpyDeviceToDevice, s) : hipSuccess;
                 if (e == hipSuccess) e = hipStreamSynchronize(s);
                 if (e != hipSuccess) {
                     retire(retired, np, b);
                     return e;
                 }
-                cache_put(Block{pl[c], pbytes[c]});
+                cache_put(Block{sl[c], sbytes[c]});
             } else {
-                retire(retired, pl[c], pbytes[c]);
+                retire(retired, sl[c], sbytes[c]);
             }
-            pl[c] = np;
-            pbytes[c] = b;
-            got = std::min<int64_t>(got, (int64_t)(b / ((size_t)S * esz)));
+            sl[c] = np;
+            sbytes[c] = b;
+            got = std::min<int64_t>(got, (int64_t)(b / block) * SLABS);
         }
         cap_blocks = got;
         return hipSuccess;
     }
     template <typename T>
-    Planes<T> planes() const {
-        Planes<T> r;
-        for (int c = 0; c < 7; ++c) r.p[c] = (T*)pl[c];
+    Clouds<T> clouds(int S) const {
+        Clouds<T> r;
+        for (int c = 0; c < SLABS; ++c) r.slab[c] = (T*)sl[c];
+        r.stride = cloud_stride(S, sizeof(T));
         return r;
     }
 };
@@ -236,11 +239,10 @@ struct scphd_filter {
     /* sample generations */
     Generation gen[2];
     int cur = 0;
-    /* every block the table references is below this index of gen[cur] */
-    int64_t blocks_used = 0;
     /* per-Gaussian intermediates */
     DBuf<double> fit, pre, lik;
     DBuf<int32_t> keep, keepscan, ndlist, holes, redo, ndfill;
+    DBuf<int32_t> wparent, wmerged; /* parent per wavefront of k_fit and of k_sample */
     /* measurements, normalisers, survivors, merge */
     DBuf<double> du, dv, eta;
     int capM = 0;
@@ -316,7 +318,7 @@ void for_each_buf(scphd_filter* f, Fn&& fn) {
     fn(f->survoff); fn(f->nmerged); fn(f->mergeoff); fn(f->outcnt); fn(f->scantmp); fn(f->sg); fn(f->sm);
     fn(f->dflag); fn(f->mcnt); fn(f->mncand); fn(f->mcand); fn(f->ngroups); fn(f->glead); fn(f->gsta);
     fn(f->gend); fn(f->gmem); fn(f->sw); fn(f->smu); fn(f->mw); fn(f->mmu); fn(f->mP); fn(f->dneff);
-    fn(f->mscratch);
+    fn(f->mscratch); fn(f->wparent); fn(f->wmerged);
 }
 
 /* hand the retired blocks to the cache: call only when no queued work on
@@ -379,12 +381,11 @@ int materialize_t(scphd_filter* f) {
     if (f->Ng == 0) return SCPHD_OK;
     const int nxt = 1 - f->cur;
     HIPTRY(f->gen[nxt].ensure(f->Ng, 0, f->S, f->esz, f->stream));
-    HIPTRY(launch_materialize<T>(f->stream, f->gen[f->cur].planes<T>(), f->gen[nxt].planes<T>(), f->gblock.p,
+    HIPTRY(launch_materialize<T>(f->stream, f->gen[f->cur].clouds<T>(f->S), f->gen[nxt].clouds<T>(f->S), f->gblock.p,
                                  f->gparent.p, f->goff.p, f->Ng, f->S, f->models.feat, f->pdt, rig_keys(f, SC_PREDICT), f->pstep,
                                  f->arith32));
     HIPTRY(launch_iota(f->stream, f->gblock.p, f->Ng));
     f->cur = nxt;
-    f->blocks_used = f->Ng;
     return SCPHD_OK;
 }
 
@@ -424,8 +425,9 @@ int update_t(scphd_filter* f, int M, int fixed) {
     const int nxt = 1 - f->cur;
     record(f, 0);
 
+    HIPTRY(f->wparent.ensure(wave_count(Ng, Np)));
     HIPTRY(launch_pose(s, f->ext.p, f->pose.p, Np, fixed, f->rig_fixed ? f->dprig.p : nullptr,
-                       f->rig_fixed ? f->dfixed.p : nullptr));
+                       f->rig_fixed ? f->dfixed.p : nullptr, f->goff.p, f->wparent.p));
     HIPTRY(f->keepscan.ensure(Ng + 1));
     HIPTRY(f->scantmp.ensure(scan_tmp_size(std::max<int64_t>(Ng, Np) + 1) + 16));
     if (Ng > 0) {
@@ -441,7 +443,7 @@ int update_t(scphd_filter* f, int M, int fixed) {
         if (f->gen[nxt].cap_blocks < Ng + hint) {
             /* the other generation holds nothing the next map needs, and
              * between updates only the parent prediction is queued (the
-             * second stream is idle): once that has run, its planes can be
+             * second stream is idle): once that has run, its slabs can be
              * handed back before the larger ones are allocated */
             HIPTRY(hipStreamSynchronize(s));
             flush_retired(f);
@@ -471,9 +473,12 @@ int update_t(scphd_filter* f, int M, int fixed) {
         fa.feat = f->models.feat;
         fa.pending = f->pending ? 1 : 0;
         fa.dt = f->pdt;
+        fa.motion = NoisyMotion(fa.feat, fa.dt);
         fa.key = rig_keys(f, SC_PREDICT); /* the landmark prediction deferred from predict */
         fa.pstep = f->pstep;
         fa.min_weight = P.min_weight;
+        fa.wave_parent = f->wparent.p;
+        fa.n_waves = (int)wave_count(Ng, Np);
         fa.fit = f->fit.p;
         fa.keep = f->keep.p;
         fa.redo = f->redo.p;
@@ -484,20 +489,15 @@ int update_t(scphd_filter* f, int M, int fixed) {
         HIPTRY(hipMemsetAsync(fa.ndfill_n, 0, sizeof(int32_t), s));
         fa.nd_base = 0;
         fa.gpd = f->hint_ok ? f->gpd.p : nullptr;
-        /* 32-bit byte offsets when every block read (below blocks_used of
-         * the current generation) and written (non-detection clouds below
-         * Ng of the next) lies below 4 GiB */
-        fa.off32 = std::max(f->blocks_used, Ng) * (int64_t)S * (int64_t)f->esz <
-                   (int64_t)0xFFFFFFFFll - 64 * (int64_t)f->esz;
         fa.arith32 = f->arith32 ? 1 : 0;
         record(f, 6);
-        HIPTRY(launch_fit<T>(s, fa, f->gen[f->cur].planes<T>(), f->gen[nxt].planes<T>()));
+        HIPTRY(launch_fit<T>(s, fa, f->gen[f->cur].clouds<T>(f->S), f->gen[nxt].clouds<T>(f->S)));
         record(f, 7);
         HIPTRY(hipEventRecord(f->ev_fit, s));
         HIPTRY(hipStreamWaitEvent(f->side, f->ev_fit, 0));
-        HIPTRY(launch_nd_fill<T>(f->side, fa, f->gen[f->cur].planes<T>(), f->gen[nxt].planes<T>()));
+        HIPTRY(launch_nd_fill<T>(f->side, fa, f->gen[f->cur].clouds<T>(f->S), f->gen[nxt].clouds<T>(f->S)));
         HIPTRY(hipEventRecord(f->ev_nd, f->side));
-        HIPTRY(launch_fit_fix<T>(s, fa, f->gen[f->cur].planes<T>(), f->gen[nxt].planes<T>()));
+        HIPTRY(launch_fit_fix<T>(s, fa, f->gen[f->cur].clouds<T>(f->S), f->gen[nxt].clouds<T>(f->S)));
         HIPTRY(launch_precompute(s, f->fit.p, f->gw.p, Ng, P.std_u * P.std_u, P.std_v * P.std_v, f->pre.p,
                                  f->lik.p));
     }
@@ -635,7 +635,8 @@ int update_t(scphd_filter* f, int M, int fixed) {
         HIPTRY(launch_scan(s, f->keep.p, f->keepscan.p, Ng, f->scantmp.p));
     else
         HIPTRY(hipMemsetAsync(f->keepscan.p, 0, sizeof(int32_t), s));
-    HIPTRY(launch_outcount(s, f->nmerged.p, f->goff.p, f->keepscan.p, Np, f->outcnt.p));
+    HIPTRY(f->wmerged.ensure(wave_count(Stot, Np)));
+    HIPTRY(launch_outcount(s, f->nmerged.p, f->goff.p, f->keepscan.p, Np, f->outcnt.p, f->mergeoff.p, f->wmerged.p));
     HIPTRY(launch_scan(s, f->outcnt.p, f->goff2.p, Np, f->scantmp.p));
     /* the non-detection clouds in [0, Ng) of the next generation are
      * complete before any return or growth of the generation (which copies
@@ -672,14 +673,14 @@ int update_t(scphd_filter* f, int M, int fixed) {
     pa.rig_meas = f->ensemble ? f->dmeas.p : nullptr;
     pa.key = rig_keys(f, SC_UPDATE);
     pa.ustep = (uint64_t)f->n_update;
+    pa.wave_parent = f->wmerged.p;
+    pa.n_waves = (int)wave_count(Kt, Np);
     pa.post_base = Ng;
     pa.holes = f->holes.p;
     pa.nholes = nholes;
-    /* 32-bit byte offsets while every destination block lies below 4 GiB */
-    pa.off32 = (Ng + over) * (int64_t)S * (int64_t)f->esz < (int64_t)0xFFFFFFFFll - 64 * (int64_t)f->esz;
     pa.arith32 = f->arith32 ? 1 : 0;
     record(f, 8);
-    HIPTRY(launch_sample<T>(s, pa, f->gen[nxt].planes<T>()));
+    HIPTRY(launch_sample<T>(s, pa, f->gen[nxt].clouds<T>(f->S)));
     record(f, 9);
     record(f, 4);
 
@@ -719,7 +720,6 @@ int update_t(scphd_filter* f, int M, int fixed) {
     f->hint_ok = true;
     f->cur = nxt;
     f->Ng = Nout;
-    f->blocks_used = Ng + over; /* non-detection clouds and posteriors in holes below Ng, the rest from Ng */
     f->n_update++;
 
     f->stats.n_meas = f->ensemble ? f->ens_meas : M;
@@ -1458,9 +1458,9 @@ int scphd_get_maps(scphd_t* f, int32_t* gcount, double* wg, double* samples) {
         size_t db = (size_t)n * 7 * sizeof(double);
         HIPTRY(cache_alloc(&dv, &db));
         double* d = (double*)dv;
-        hipError_t e = f->esz == 8 ? launch_extract<double>(s, f->gen[f->cur].planes<double>(), f->gblock.p, f->Ng,
+        hipError_t e = f->esz == 8 ? launch_extract<double>(s, f->gen[f->cur].clouds<double>(f->S), f->gblock.p, f->Ng,
                                                             f->S, d)
-                                   : launch_extract<float>(s, f->gen[f->cur].planes<float>(), f->gblock.p, f->Ng,
+                                   : launch_extract<float>(s, f->gen[f->cur].clouds<float>(f->S), f->gblock.p, f->Ng,
                                                            f->S, d);
         if (e == hipSuccess)
             e = hipMemcpyAsync(samples, d, (size_t)n * 7 * sizeof(double), hipMemcpyDeviceToHost, s);
@@ -1511,8 +1511,8 @@ int scphd_set_state(scphd_t* f, const double* states, const double* weights, con
         double* d = (double*)dv;
         hipError_t e = hipMemcpyAsync(d, samples, (size_t)n * 7 * sizeof(double), hipMemcpyHostToDevice, s);
         if (e == hipSuccess)
-            e = f->esz == 8 ? launch_inject<double>(s, d, Ng, S, f->gen[f->cur].planes<double>())
-                            : launch_inject<float>(s, d, Ng, S, f->gen[f->cur].planes<float>());
+            e = f->esz == 8 ? launch_inject<double>(s, d, Ng, S, f->gen[f->cur].clouds<double>(f->S))
+                            : launch_inject<float>(s, d, Ng, S, f->gen[f->cur].clouds<float>(f->S));
         if (e == hipSuccess) e = hipStreamSynchronize(s);
         retire(&f->retired, dv, db);
         if (e != hipSuccess) return hipfail(f, e, "set_state");
@@ -1520,7 +1520,6 @@ int scphd_set_state(scphd_t* f, const double* states, const double* weights, con
     HIPTRY(hipStreamSynchronize(s));
     flush_retired(f);
     f->Ng = Ng;
-    f->blocks_used = Ng;
     f->n_predict = n_predict;
     f->n_update = n_update;
     f->n_resample = n_resample;
@@ -1683,11 +1682,10 @@ template <typename T>
 int compact_map(scphd_filter* f) {
     const int nxt = 1 - f->cur;
     HIPTRY(f->gen[nxt].ensure(f->Ng, 0, f->S, f->esz, f->stream, true));
-    HIPTRY(launch_gather<T>(f->stream, f->gen[f->cur].planes<T>(), f->gen[nxt].planes<T>(), f->gblock.p, f->Ng,
+    HIPTRY(launch_gather<T>(f->stream, f->gen[f->cur].clouds<T>(f->S), f->gen[nxt].clouds<T>(f->S), f->gblock.p, f->Ng,
                             f->S));
     HIPTRY(launch_iota(f->stream, f->gblock.p, f->Ng));
     f->cur = nxt;
-    f->blocks_used = f->Ng;
     return SCPHD_OK;
 }
 
@@ -1718,7 +1716,7 @@ int scphd_compact(scphd_t* f) {
     for (auto* b : {&f->fit, &f->pre, &f->lik, &f->eta, &f->sw, &f->smu, &f->mw, &f->mmu, &f->mP}) b->release();
     for (auto* b : {&f->keep, &f->keepscan, &f->ndlist, &f->holes, &f->redo, &f->ndfill, &f->mcnt, &f->mncand, &f->mcand, &f->sg,
                     &f->sm, &f->glead, &f->gsta, &f->gend, &f->gmem, &f->gparent2, &f->gblock2, &f->nsurv,
-                    &f->survoff, &f->nmerged, &f->mergeoff, &f->outcnt, &f->ngroups})
+                    &f->survoff, &f->nmerged, &f->mergeoff, &f->outcnt, &f->ngroups, &f->wparent, &f->wmerged})
         b->release();
     f->gw2.release();
     f->gpd2.release();
@@ -1749,6 +1747,8 @@ int scphd_reserve(scphd_t* f, int64_t n_gaussians, int32_t max_meas) {
     HIPTRY(f->ndfill.ensure(G + 1));
     HIPTRY(f->ndlist.ensure(G));
     HIPTRY(f->holes.ensure(G));
+    HIPTRY(f->wparent.ensure(wave_count(G, (int)Np)));
+    HIPTRY(f->wmerged.ensure(wave_count(G + 1, (int)Np)));
     HIPTRY(f->scantmp.ensure(scan_tmp_size(std::max<int64_t>(G, Np) + 1) + 16));
     /* the successor table, and the current one keeping its entries, so that
      * the table swaps of later updates and resamplings find both sized */
@@ -1790,7 +1790,7 @@ int scphd_get_memory(scphd_t* f, int64_t* bytes) {
     int64_t b = 0;
     for_each_buf(f, [&b](auto& d) { b += (int64_t)d.bytes; });
     for (const auto& g : f->gen)
-        for (size_t x : g.pbytes) b += (int64_t)x;
+        for (size_t x : g.sbytes) b += (int64_t)x;
     *bytes = b;
     return SCPHD_OK;
 }

@@ -10,10 +10,11 @@
  *   map table one entry per Gaussian in canonical order (parent ascending):
  *             goff[Np+1] offsets, gparent[Ng], gblock[Ng] sample block,
  *             gw[Ng] Gaussian weight (FP64).
- *   samples   a generation buffer of 7 planes (x y z vx vy vz w) of T
- *             (float or double); block b holds samples [b*S, (b+1)*S).
- *             Blocks may be shared by several table entries after
- *             resampling; kernels never write a block they read.
+ *   samples   a generation of blocks, one cloud of S samples each, the 7
+ *             values (x y z vx vy vz w) of T (float or double) of all its
+ *             samples together (Clouds below).  Blocks may be shared by
+ *             several table entries after resampling; kernels never write a
+ *             block they read.
  */
 #ifndef SCPHD_KERNELS_H
 #define SCPHD_KERNELS_H
@@ -71,10 +72,50 @@ enum PrePlane {
  * log(det S) / 2 and 1 when the updated covariance is PD, else 0 */
 enum LikField { LK_MUU = 0, LK_MUV, LK_S0, LK_S12, LK_S3, LK_C, LK_H, LK_OK, LK_COUNT = 8 };
 
+/* A generation's sample blocks.  Block b lies in slab b % SLABS at place
+ * b / SLABS, `stride` elements a block (cloud_stride).  Inside a block the
+ * samples go in steps of 16 (what a 16-lane row handles at once; the last
+ * step may be narrower), the seven values of a step in turn.
+ *
+ * Why one block and not seven planes: the kernels that stream clouds are
+ * bound by memory, and with seven planes in and seven out, 64 B of each at a
+ * time, it gave 2.7-3.4 TB/s (4.8 reads alone); with a cloud in one place it
+ * gives 4.7-5.0 TB/s (5.8-6.3), S = 200, half of the clouds written back.
+ * (Groups of 64 samples with 16-byte accesses a lane gave 4.9-5.2, but four
+ * times the registers in flight.)  Why slabs: a generation that grows
+ * replaces them one at a time, so that it never needs twice its memory. */
+static constexpr int SLABS = 8;
 template <typename T>
-struct Planes {
-    T* p[7];
+struct Clouds {
+    T* slab[SLABS];
+    int64_t stride;
+    /* the slab chosen bit by bit: the pointers are kernel arguments, and an
+     * indexed read of those is a load from host memory or a select over all */
+    __device__ T* block(int64_t b) const {
+        static_assert(SLABS == 8);
+        const bool b0 = b & 1, b1 = b & 2, b2 = b & 4;
+        T* const x0 = b0 ? slab[1] : slab[0];
+        T* const x1 = b0 ? slab[3] : slab[2];
+        T* const x2 = b0 ? slab[5] : slab[4];
+        T* const x3 = b0 ? slab[7] : slab[6];
+        T* const y0 = b1 ? x1 : x0;
+        T* const y1 = b1 ? x3 : x2;
+        return (b2 ? y1 : y0) + (b / SLABS) * stride;
+    }
 };
+
+/* element of value c of sample s in a block of S samples */
+SCPHD_HD inline int cloud_at(int S, int s, int c) {
+    const int q = s & ~15, w = S - q < 16 ? S - q : 16;
+    return 7 * q + c * w + (s & 15);
+}
+
+/* elements from one block to the next: whole 128 B lines where that costs at
+ * most 1/32 more memory, else 16 B */
+inline int64_t cloud_stride(int S, size_t esz) {
+    const int64_t b = (int64_t)7 * S * (int64_t)esz, l = (b + 127) / 128 * 128;
+    return (l <= b + b / 32 ? l : (b + 15) / 16 * 16) / (int64_t)esz;
+}
 
 struct FilterModels {
     DisparityMeasurementModel meas;
@@ -98,16 +139,34 @@ hipError_t launch_prior(hipStream_t s, double* ext, double* pw, int Np, const do
                         NoiseKey key);
 /* rfixed (ensembles, may be null): per rig, the fixed camera for that rig
  * (rig of parent p: prig[p]); else `fixed` for every parent */
-hipError_t launch_pose(hipStream_t s, const double* ext, double* pose, int Np, int fixed,
-                       const int32_t* prig = nullptr, const int32_t* rfixed = nullptr);
+/* goff, wave_parent (wave_count(goff[Np], Np) entries, written): the map
+ * table's parent per wavefront of k_fit */
+hipError_t launch_pose(hipStream_t s, const double* ext, double* pose, int Np, int fixed, const int32_t* prig,
+                       const int32_t* rfixed, const int32_t* goff, int32_t* wave_parent);
+/* wavefronts (of four rows) that take n table entries of Np parents, none of
+ * them two parents' */
+int64_t wave_count(int64_t n, int Np);
 
 /* Apply a deferred sample prediction, writing every table entry to its own
  * block (block id = table index) of the destination generation. */
 template <typename T>
-hipError_t launch_materialize(hipStream_t s, Planes<T> src, Planes<T> dst, const int32_t* gblock,
+hipError_t launch_materialize(hipStream_t s, Clouds<T> src, Clouds<T> dst, const int32_t* gblock,
                               const int32_t* gparent, const int32_t* goff, int64_t Ng, int S,
                               LinearCVMotionModel3D feat, double dt, RigKeys key, uint64_t step,
                               bool arith32 = false);
+
+/* the landmark prediction's constants: dt, and per axis std dt^2 / 2 and std dt */
+struct NoisyMotion {
+    double dt = 0.0, sh[3] = {}, sd[3] = {};
+    NoisyMotion() = default;
+    SCPHD_HD NoisyMotion(const LinearCVMotionModel3D& m, double t) : dt(t) {
+        const double h = 0.5 * t * t, std[3] = {m.std_ax(), m.std_ay(), m.std_az()};
+        for (int i = 0; i < 3; ++i) {
+            sh[i] = std[i] * h;
+            sd[i] = std[i] * t;
+        }
+    }
+};
 
 /* ---- update ---- */
 struct FitArgs {
@@ -121,11 +180,14 @@ struct FitArgs {
     DisparityMeasurementModel meas;
     const DisparityMeasurementModel* rig_meas = nullptr; /* ensemble: per rig (rigs may differ), else null */
     LinearCVMotionModel3D feat;
+    NoisyMotion motion; /* of feat over dt */
     int pending;
     double dt;
     RigKeys key;
     uint64_t pstep;
     double min_weight;
+    const int32_t* wave_parent; /* parent per wavefront of k_fit, -1: none */
+    int n_waves;
     double* fit;     /* FP_COUNT planes */
     int32_t* keep;   /* non-detection term kept */
     int32_t* redo;     /* Gaussians whose sample weights were all zero, refitted by k_fit_fix */
@@ -134,18 +196,17 @@ struct FitArgs {
     int32_t* ndfill_n; /* their number; zero before k_fit */
     int64_t nd_base; /* destination block of the non-detection cloud of entry g: nd_base + g */
     const float* gpd = nullptr; /* per entry: pd_g of its source term at the last update (1: posterior term) */
-    int off32;       /* every source and destination plane is below 4 GiB: 32-bit byte offsets */
     int arith32 = 0; /* per-sample arithmetic in single precision (FP32 storage only) */
 };
 
 /* k_fit: the streaming sweep; k_fit_fix: the rare cases it lists in redo[];
  * k_nd_fill: the non-detection clouds it lists in ndfill[] */
 template <typename T>
-hipError_t launch_fit(hipStream_t s, const FitArgs& a, Planes<T> src, Planes<T> dst);
+hipError_t launch_fit(hipStream_t s, const FitArgs& a, Clouds<T> src, Clouds<T> dst);
 template <typename T>
-hipError_t launch_fit_fix(hipStream_t s, const FitArgs& a, Planes<T> src, Planes<T> dst);
+hipError_t launch_fit_fix(hipStream_t s, const FitArgs& a, Clouds<T> src, Clouds<T> dst);
 template <typename T>
-hipError_t launch_nd_fill(hipStream_t s, const FitArgs& a, Planes<T> src, Planes<T> dst);
+hipError_t launch_nd_fill(hipStream_t s, const FitArgs& a, Clouds<T> src, Clouds<T> dst);
 
 hipError_t launch_precompute(hipStream_t s, const double* fit, const double* gw, int64_t Ng, double var_u,
                              double var_v, double* pre, double* lik);
@@ -282,19 +343,22 @@ struct SampleArgs {
     const DisparityMeasurementModel* rig_meas = nullptr; /* ensemble: per rig, else null */
     RigKeys key;
     uint64_t ustep;
+    const int32_t* wave_parent; /* parent per wavefront, -1: none */
+    int n_waves;
     int64_t post_base;
     /* merged Gaussian gm's block: holes[gm] while gm < nholes (the blocks
      * of dropped non-detection terms), else post_base + gm - nholes */
     const int32_t* holes = nullptr;
     int64_t nholes = 0;
-    int off32; /* every destination offset is below 4 GiB: 32-bit byte offsets */
     int arith32 = 0; /* draws and disparity -> world in single precision (FP32 storage only) */
 };
 template <typename T>
-hipError_t launch_sample(hipStream_t s, const SampleArgs& a, Planes<T> dst);
+hipError_t launch_sample(hipStream_t s, const SampleArgs& a, Clouds<T> dst);
 
+/* mergeoff, wave_parent (wave_count(mergeoff[Np], Np) entries, written): the
+ * posterior terms' parent per wavefront of k_sample */
 hipError_t launch_outcount(hipStream_t s, const int32_t* nmerged, const int32_t* goff, const int32_t* keepscan,
-                           int Np, int32_t* outcnt);
+                           int Np, int32_t* outcnt, const int32_t* mergeoff, int32_t* wave_parent);
 /* ndlist[keepscan[g]] = g for the kept entries; with holes, also
  * holes[g - keepscan[g]] = g for the dropped ones */
 hipError_t launch_ndlist(hipStream_t s, const int32_t* keep, const int32_t* keepscan, int64_t Ng, int32_t* ndlist,
@@ -359,12 +423,12 @@ hipError_t launch_table_resample(hipStream_t s, const int32_t* anc, const int32_
 
 /* ---- read-back ---- */
 template <typename T>
-hipError_t launch_extract(hipStream_t s, Planes<T> src, const int32_t* gblock, int64_t Ng, int S, double* out);
+hipError_t launch_extract(hipStream_t s, Clouds<T> src, const int32_t* gblock, int64_t Ng, int S, double* out);
 /* the clouds of the Ng map entries into blocks 0 .. Ng-1 of dst */
 template <typename T>
-hipError_t launch_gather(hipStream_t s, Planes<T> src, Planes<T> dst, const int32_t* gblock, int64_t Ng, int S);
+hipError_t launch_gather(hipStream_t s, Clouds<T> src, Clouds<T> dst, const int32_t* gblock, int64_t Ng, int S);
 template <typename T>
-hipError_t launch_inject(hipStream_t s, const double* in, int64_t Ng, int S, Planes<T> dst);
+hipError_t launch_inject(hipStream_t s, const double* in, int64_t Ng, int S, Clouds<T> dst);
 
 /* ---- scan ---- */
 /* out[0..n] = exclusive prefix sums of in[0..n), out[n] = total.

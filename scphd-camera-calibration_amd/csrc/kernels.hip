@@ -171,12 +171,29 @@ __global__ void k_scale(double* x, int64_t n, double a) {
     if (i < n) x[i] *= a;
 }
 
+/* One wavefront's share of writing the table that gives the streaming kernels
+ * their parents: table entries off[p] .. off[p + 1] - 1 are parent p's, four
+ * to a wavefront (a 16-lane row each), and wavefront w of the kernel takes
+ * those from off[p] + 4 (w - first_wave(off, p)) on for p = wave_parent[w].
+ * Wavefronts never straddle parents, so that a parent's camera, model and
+ * noise key are scalar; one that has no entry of its parent holds -1 (at most
+ * one a parent). */
+__device__ inline int first_wave(int off_p, int p) { return off_p / 4 + p; }
+
+__device__ inline void write_wave_parents(int off0, int off1, int p, int lane, int32_t* wave_parent) {
+    const int w0 = first_wave(off0, p), n = first_wave(off1, p + 1) - w0, used = (off1 - off0 + 3) / 4;
+    for (int i = lane; i < n; i += 64) wave_parent[w0 + i] = i < used ? p : -1;
+}
+
 /* Camera used by an update: the parent's extrinsics, or all-zero extrinsics
- * for the fixed camera (src/scphdcameracalibration.cu:1167-1176). */
-__global__ void k_pose(const double* ext, double* pose, int Np, int fixed, const int32_t* prig,
-                       const int32_t* rfixed) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
+ * for the fixed camera (src/scphdcameracalibration.cu:1167-1176); and the map
+ * table's wave_parent.  One wavefront per parent. */
+__global__ __launch_bounds__(256) void k_pose(const double* ext, double* pose, int Np, int fixed, const int32_t* prig,
+                                              const int32_t* rfixed, const int32_t* goff, int32_t* wave_parent) {
+    const int p = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (p >= Np) return;
+    write_wave_parents(goff[p], goff[p + 1], p, lane, wave_parent);
+    if (lane != 0) return;
     if (rfixed) fixed = rfixed[prig[p]];
     CameraPose c;
     if (fixed) {
@@ -204,41 +221,43 @@ __device__ inline CameraPose load_pose(const double* pose, int p) {
 /* Landmark sample prediction (predict_features functor,
  * src/scphdcameracalibration.cu:154-178): the constant-velocity step with
  * acceleration draws a[i] * std_i (LinearCVMotionModel3D::computeNoisyMotion),
- * x + v dt + a std dt^2 / 2 and v + a std dt, the products std dt^2 / 2 and
- * std dt formed once per kernel (loop invariants) instead of per sample. */
-__device__ inline EuclideanPoint noisy_motion(EuclideanPoint x, const LinearCVMotionModel3D& feat, double dt,
-                                              const double a[3]) {
-    const double h = 0.5 * dt * dt;
-    x.x = fma(a[0], feat.std_ax() * h, fma(x.vx, dt, x.x));
-    x.y = fma(a[1], feat.std_ay() * h, fma(x.vy, dt, x.y));
-    x.z = fma(a[2], feat.std_az() * h, fma(x.vz, dt, x.z));
-    x.vx = fma(a[0], feat.std_ax() * dt, x.vx);
-    x.vy = fma(a[1], feat.std_ay() * dt, x.vy);
-    x.vz = fma(a[2], feat.std_az() * dt, x.vz);
+ * x + v dt + a std dt^2 / 2 and v + a std dt. */
+__device__ inline EuclideanPoint noisy_motion(EuclideanPoint x, const NoisyMotion& m, const double a[3]) {
+    x.x = fma(a[0], m.sh[0], fma(x.vx, m.dt, x.x));
+    x.y = fma(a[1], m.sh[1], fma(x.vy, m.dt, x.y));
+    x.z = fma(a[2], m.sh[2], fma(x.vz, m.dt, x.z));
+    x.vx = fma(a[0], m.sd[0], x.vx);
+    x.vy = fma(a[1], m.sd[1], x.vy);
+    x.vz = fma(a[2], m.sd[2], x.vz);
     return x;
 }
 
 /* the prediction of the sample (p, k, s) */
 template <typename Key>
-__device__ inline EuclideanPoint predict_sample(EuclideanPoint x, const LinearCVMotionModel3D& feat, double dt,
-                                                Key key, uint64_t step, uint32_t p, uint32_t k, uint32_t s) {
+__device__ inline EuclideanPoint predict_sample(EuclideanPoint x, const NoisyMotion& m, Key key, uint64_t step, uint32_t p, uint32_t k, uint32_t s) {
     double a[3];
     feature_normals(key, step, p, k, s, a);
-    return noisy_motion(x, feat, dt, a);
+    return noisy_motion(x, m, a);
 }
 
 /* the same for the members of a noise group in order (phase = member) */
 template <typename Key>
-__device__ inline EuclideanPoint predict_sample_seq(EuclideanPoint x, const LinearCVMotionModel3D& feat, double dt,
-                                                    Key key, uint64_t step, uint32_t p, uint32_t k, uint32_t s,
+__device__ inline EuclideanPoint predict_sample_seq(EuclideanPoint x, const NoisyMotion& m, Key key, uint64_t step, uint32_t p, uint32_t k, uint32_t s,
                                                     uint32_t phase, FeatureCarry& c) {
     double a[3];
     feature_normals_seq(key, step, p, k, s, phase, c, a);
-    return noisy_motion(x, feat, dt, a);
+    return noisy_motion(x, m, a);
+}
+
+/* the seven values of sample s of a block of S samples */
+template <typename T>
+__device__ inline void load_sample(const T* block, int S, int s, T r[7]) {
+#pragma unroll
+    for (int c = 0; c < 7; ++c) r[c] = block[cloud_at(S, s, c)];
 }
 
 template <typename T>
-__global__ void k_materialize(Planes<T> src, Planes<T> dst, const int32_t* gblock, const int32_t* gparent,
+__global__ void k_materialize(Clouds<T> src, Clouds<T> dst, const int32_t* gblock, const int32_t* gparent,
                               const int32_t* goff, int64_t Ng, int S, LinearCVMotionModel3D feat, double dt,
                               RigKeys rk, uint64_t step, int arith32) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -247,12 +266,14 @@ __global__ void k_materialize(Planes<T> src, Planes<T> dst, const int32_t* gbloc
     const int s = (int)(i - g * S);
     const int p = gparent[g];
     const int k = (int)(g - goff[p]);
-    const int64_t si = (int64_t)gblock[g] * S + s;
-    const int64_t di = g * S + s;
+    T r[7];
+    load_sample<T>(src.block(gblock[g]), S, s, r);
+    T* const db = dst.block(g);
+    auto put = [&](int c, T v) { db[cloud_at(S, s, c)] = v; };
     if (arith32) { /* the single-precision prediction of the FP32-arithmetic variant */
         float x[6], n[3];
 #pragma unroll
-        for (int c = 0; c < 6; ++c) x[c] = (float)src.p[c][si];
+        for (int c = 0; c < 6; ++c) x[c] = (float)r[c];
         if (!rk.keys) {
             feature_normals(rk.key, step, (uint32_t)p, (uint32_t)k, (uint32_t)s, n);
         } else {
@@ -262,22 +283,25 @@ __global__ void k_materialize(Planes<T> src, Planes<T> dst, const int32_t* gbloc
         }
         predict_f(x, motion_f(feat, dt), n);
 #pragma unroll
-        for (int c = 0; c < 6; ++c) dst.p[c][di] = (T)x[c];
-        dst.p[6][di] = src.p[6][si];
+        for (int c = 0; c < 6; ++c) put(c, (T)x[c]);
+        put(6, r[6]);
         return;
     }
-    EuclideanPoint x{(double)src.p[0][si], (double)src.p[1][si], (double)src.p[2][si],
-                     (double)src.p[3][si], (double)src.p[4][si], (double)src.p[5][si]};
+    EuclideanPoint x{(double)r[0], (double)r[1], (double)r[2], (double)r[3], (double)r[4], (double)r[5]};
     if (!rk.keys) { /* one rig: the key stays in scalar registers */
-        x = predict_sample(x, feat, dt, rk.key, step, (uint32_t)p, (uint32_t)k, (uint32_t)s);
+        x = predict_sample(x, NoisyMotion(feat, dt), rk.key, step, (uint32_t)p, (uint32_t)k, (uint32_t)s);
     } else {
         int pl;
         const LaneKey key = rk.of(p, pl);
-        x = predict_sample(x, feat, dt, key, step, (uint32_t)pl, (uint32_t)k, (uint32_t)s);
+        x = predict_sample(x, NoisyMotion(feat, dt), key, step, (uint32_t)pl, (uint32_t)k, (uint32_t)s);
     }
-    dst.p[0][di] = (T)x.x; dst.p[1][di] = (T)x.y; dst.p[2][di] = (T)x.z;
-    dst.p[3][di] = (T)x.vx; dst.p[4][di] = (T)x.vy; dst.p[5][di] = (T)x.vz;
-    dst.p[6][di] = src.p[6][si];
+    put(0, (T)x.x);
+    put(1, (T)x.y);
+    put(2, (T)x.z);
+    put(3, (T)x.vx);
+    put(4, (T)x.vy);
+    put(5, (T)x.vz);
+    put(6, r[6]);
 }
 
 /* ------------------------------------------------------- reproject + fit */
@@ -299,41 +323,29 @@ __device__ inline float row_sum16(float x) {
     return x;
 }
 
-/* One sample of a Gaussian's cloud: the deferred prediction applied, its
- * disparity-space point, its field-of-view flag and stored weight. */
-/* Plane element at byte offset `off` from a uniform plane base.  With a
- * 32-bit offset the address is a scalar base plus one per-lane offset
- * register (the global_load saddr form); 64-bit offsets serve planes of
- * 4 GiB and more. */
-template <typename T, typename Off>
-__device__ inline T& at(T* base, Off off) {
-    return *(T*)((char*)base + off);
-}
-
-template <typename T, typename Off>
-__device__ inline void load_sample_off(const Planes<T>& src, Off off, T r[7]) {
+/* The lane's sample of one step of a cloud, from the step's place `p` in its
+ * block, w samples wide: 16 or more, fewer in the last step, whose lanes
+ * without a sample read its last one, or none after it (nothing is read). */
+template <typename T>
+__device__ inline void load_full_step(const T* p, int lane, T r[7]) {
 #pragma unroll
-    for (int c = 0; c < 7; ++c) r[c] = at(src.p[c], off);
-}
-
-template <typename T, typename Off>
-__device__ inline void write_nd_off(const DisparityMeasurementModel& meas, Planes<T>& dst, Off off,
-                                    const EuclideanPoint& x, bool in) {
-    at(dst.p[0], off) = (T)x.x;
-    at(dst.p[1], off) = (T)x.y;
-    at(dst.p[2], off) = (T)x.z;
-    at(dst.p[3], off) = (T)x.vx;
-    at(dst.p[4], off) = (T)x.vy;
-    at(dst.p[5], off) = (T)x.vz;
-    at(dst.p[6], off) = (T)(1.0 - (in ? meas.pd() : 0.0));
+    for (int c = 0; c < 7; ++c) r[c] = p[c * 16 + lane];
 }
 
 template <typename T>
-__device__ inline void load_sample(const Planes<T>& src, int64_t si, T r[7]) {
+__device__ inline void load_step(const T* p, int w, int lane, T r[7]) {
+    if (w >= 16) {
+        load_full_step(p, lane, r);
+    } else if (w > 0) {
+        int l = min(lane, w - 1);
+        asm volatile("" : "+v"(l)); /* this branch's addresses are formed in it */
 #pragma unroll
-    for (int c = 0; c < 7; ++c) r[c] = src.p[c][si];
+        for (int c = 0; c < 7; ++c) r[c] = p[c * w + l];
+    }
 }
 
+/* One sample of a Gaussian's cloud: the deferred prediction applied, its
+ * disparity-space point, its field-of-view flag and stored weight. */
 template <typename T, typename Key>
 __device__ inline void eval_sample(const FitArgs& a, const DisparityMeasurementModel& meas, const T r[7], Key kk,
                                    int pl, int k, int s, const CameraPose& pose, EuclideanPoint& x, DisparityPoint& d,
@@ -342,21 +354,12 @@ __device__ inline void eval_sample(const FitArgs& a, const DisparityMeasurementM
     w = (double)r[6];
     if (a.pending) {
         if (fc)
-            x = predict_sample_seq(x, a.feat, a.dt, kk, a.pstep, (uint32_t)pl, (uint32_t)k, (uint32_t)s, phase, *fc);
+            x = predict_sample_seq(x, a.motion, kk, a.pstep, (uint32_t)pl, (uint32_t)k, (uint32_t)s, phase, *fc);
         else
-            x = predict_sample(x, a.feat, a.dt, kk, a.pstep, (uint32_t)pl, (uint32_t)k, (uint32_t)s);
+            x = predict_sample(x, a.motion, kk, a.pstep, (uint32_t)pl, (uint32_t)k, (uint32_t)s);
     }
     d = disparity_fast(meas, pose, x);
     in = meas.inRange(d);
-}
-
-template <typename T, typename Key>
-__device__ inline void fit_sample(const FitArgs& a, const DisparityMeasurementModel& meas, const Planes<T>& src,
-                                  int64_t si, Key kk, int pl, int k, int s, const CameraPose& pose,
-                                  EuclideanPoint& x, DisparityPoint& d, bool& in, double& w) {
-    T r[7];
-    load_sample(src, si, r);
-    eval_sample(a, meas, r, kk, pl, k, s, pose, x, d, in, w);
 }
 
 /* The FP32-arithmetic form of eval_sample: the sample's world point x (after
@@ -385,14 +388,6 @@ __device__ inline void eval_sample_f(const FitArgs& a, const SampleCtxF& cx, con
     }
     disparity_f(cx.m, cx.pose, x, q);
     in = in_range_f(cx.m, q);
-}
-
-template <typename T, typename Off>
-__device__ inline void write_nd_off_f(const DisparityMeasurementModel& meas, Planes<T>& dst, Off off, const float x[6],
-                                      bool in) {
-#pragma unroll
-    for (int c = 0; c < 6; ++c) at(dst.p[c], off) = (T)x[c];
-    at(dst.p[6], off) = (T)(1.0 - (in ? meas.pd() : 0.0));
 }
 
 __device__ inline void write_fit(const FitArgs& a, int64_t g, int lane, const double* mu, const double* P, double pdg) {
@@ -468,40 +463,128 @@ struct RowMeas<true> {
         : m(per_rig[rk.prig[p]]) {}
 };
 
-/* waves per SIMD the fit kernel is compiled for (register budget 512 / n) */
+/* Per-parent data read through the constant address space: with a parent
+ * that is the same in every active lane, the loads are scalar and the values
+ * stay in scalar registers, where FP64 instructions take them as operands. */
+typedef __attribute__((address_space(4))) const double cdouble_t;
+typedef __attribute__((address_space(4))) const int32_t cint_t;
+typedef __attribute__((address_space(4))) const uint32_t cuint_t;
+
+__device__ inline CameraPose scalar_pose(const double* pose, int p) {
+    cdouble_t* o = (cdouble_t*)(pose + (int64_t)p * 12);
+    CameraPose c;
+#pragma unroll
+    for (int i = 0; i < 9; ++i) c.R[i] = o[i];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) c.t[i] = o[9 + i];
+    return c;
+}
+
+/* What a wavefront needs of one parent: its camera, its rig's measurement
+ * model, noise key and step counter, and its index in the rig. */
+struct ParentCtx {
+    CameraPose pose;
+    DisparityMeasurementModel meas;
+    NoiseKey key;
+    uint64_t step;
+    int pl;
+    __device__ ParentCtx(const double* poses, const DisparityMeasurementModel& one,
+                         const DisparityMeasurementModel* per_rig, const RigKeys& rk, uint64_t handle_step, int p)
+        : pose(scalar_pose(poses, p)), meas(one), key(rk.key), step(handle_step), pl(p) {
+        if (!rk.keys) return;
+        const int r = ((cint_t*)rk.prig)[p];
+        pl = p - ((cint_t*)rk.poff)[r];
+        cuint_t* k = (cuint_t*)(rk.keys + r);
+        key.k0 = k[0];
+        key.k1 = k[1];
+        /* the counter a filter of the rig's own would use */
+        if (rk.sbase) step = (uint32_t)handle_step - ((cuint_t*)rk.sbase)[SC_COUNT * r + rk.which];
+        constexpr int ND = sizeof(DisparityMeasurementModel) / sizeof(double);
+        static_assert(sizeof(NoiseKey) == 2 * sizeof(uint32_t) && ND * sizeof(double) == sizeof(meas));
+        double v[ND];
+#pragma unroll
+        for (int i = 0; i < ND; ++i) v[i] = ((cdouble_t*)(per_rig + r))[i];
+        __builtin_memcpy(&meas, v, sizeof(meas));
+    }
+};
+
+/* waves per SIMD the fit kernel is compiled for (register budget 512 / n).
+ * Bound: VALU issue (0.87 ms of 491,572 Gaussians x 200 samples without any
+ * memory access at 3 waves, 0.98 at 2) and memory (0.90 ms without the
+ * normals), which overlap only in part.  At 4096 parents, 200 landmarks: 7.6
+ * ms a frame with seven planes, the camera in vector registers and 2 waves;
+ * 7.1 with clouds in blocks and the camera scalar; 6.2 with 3 waves, which
+ * wavefronts of one parent leave the registers for. */
 #ifndef SCPHD_FIT_WAVES
-#define SCPHD_FIT_WAVES 2
+#define SCPHD_FIT_WAVES 3
 #endif
 
-/* A, the arithmetic type of the per-sample work: double, or float for the
+/* LDS accesses of one wavefront's lanes before and after it, in that order */
+__device__ inline void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+/* the kernel's first argument, read here and not before: pointers that only
+ * a kernel's end needs are not held in scalar registers over its sweep */
+template <typename S>
+__device__ inline const S& kernarg_late() {
+    typedef __attribute__((address_space(4))) const char* cptr_t;
+    cptr_t k = (cptr_t)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(k));
+    return *(const S*)k;
+}
+
+/* k_fit's and k_sample's arguments */
+template <typename T>
+struct FitKernArgs {
+    FitArgs a;
+    Clouds<T> src, dst;
+};
+template <typename T>
+struct SampleKernArgs {
+    SampleArgs a;
+    Clouds<T> dst;
+};
+
+/* one row's share of k_fit's LDS; 17: lanes a value apart use other banks */
+template <typename A>
+struct FitShared {
+    A part[16 * 17];
+    double tot[32], K[6];
+};
+
+/* Sixteen row sums: lane l of the row gets the sum over its lanes of v[l],
+ * added up as row_sum16 does (neighbours, pairs of them, halves, the row). */
+template <typename A>
+__device__ inline double row_total(A* part, const A (&v)[16], int lane) {
+    wave_lds_fence();
+#pragma unroll
+    for (int e = 0; e < 16; ++e) part[e * 17 + lane] = v[e];
+    wave_lds_fence();
+    A x[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) x[i] = part[lane * 17 + i];
+#pragma unroll
+    for (int w = 1; w < 16; w *= 2)
+#pragma unroll
+        for (int i = 0; i < 16; i += 2 * w) x[i] += x[i + w];
+    return (double)x[0];
+}
+
+/* One row of k_fit, its Gaussian g of parent p (the same for every row of
+ * the wavefront).
+ * A, the arithmetic type of the per-sample work: double, or float for the
  * FP32-arithmetic variant (FP32 storage), whose moment sums are single
  * precision up to the row sums and whose in-view count is an integer. */
-template <typename T, typename Off, bool RG, typename A = double>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SCPHD_FIT_WAVES, SCPHD_FIT_WAVES))) void k_fit(
-    FitArgs a, Planes<T> src, Planes<T> dst) {
+template <typename T, typename A>
+__device__ inline void fit_row(const FitArgs& a, const ParentCtx& pc, int64_t g, int k, const T* from, T* to,
+                               FitShared<A>& sh) {
     constexpr bool F32 = std::is_same_v<A, float>;
     static_assert(!F32 || std::is_same_v<T, float>, "single-precision arithmetic needs FP32 storage");
-    /* the rows' camera poses are staged through LDS once and then held in
-     * registers for the whole sweep */
-    __shared__ double s_pose[16 * 12];
-    const int lane = threadIdx.x & 15, row = threadIdx.x >> 4;
-    const int64_t g = (int64_t)blockIdx.x * 16 + row;
-    const bool act = g < a.Ng;
-    const int p = act ? a.gparent[g] : 0;
-    if (act && lane < 12) s_pose[row * 12 + lane] = a.pose[(int64_t)p * 12 + lane];
-    __syncthreads();
-    if (!act) return; /* whole rows; rows never exchange data */
-    CameraPose pose;
-#pragma unroll
-    for (int i = 0; i < 9; ++i) pose.R[i] = s_pose[row * 12 + i];
-#pragma unroll
-    for (int i = 0; i < 3; ++i) pose.t[i] = s_pose[row * 12 + 9 + i];
-    const int k = (int)(g - a.goff[p]);
-    int pl;
-    const auto kk = row_key<RG>(a.key, p, pl); /* the rig's key, p's index in its rig */
-    const RowMeas<RG> rm(a.meas, a.rig_meas, a.key, p);
-    const DisparityMeasurementModel& meas = rm.m;
-    const int64_t b0 = (int64_t)a.gblock[g] * a.S;
+    const int lane = threadIdx.x & 15;
+    const DisparityMeasurementModel& meas = pc.meas;
+    const CameraPose& pose = pc.pose;
     const int S = a.S;
     const double wg = a.gw[g];
     const double Pd = meas.pd();
@@ -511,7 +594,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SCPHD_FIT_W
      * (a non-detection term's cloud moves little in one step): a guess that
      * costs only the write of a cloud nothing references if it proves wrong */
     const bool nd_write = nd_sure || (a.gpd && wg * (1.0 - (double)a.gpd[g]) >= a.min_weight);
-    const int64_t d0 = (a.nd_base + g) * (int64_t)S;
     SampleCtxF cx;
     if constexpr (F32) cx = SampleCtxF{meas_f(meas), pose_f(pose), motion_f(a.feat, a.dt)};
     const A PdA = (A)Pd;
@@ -525,45 +607,71 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SCPHD_FIT_W
     for (int c = 0; c < 6; ++c) m1[c] = 0.0;
 #pragma unroll
     for (int e = 0; e < 21; ++e) m2[e] = 0.0;
-    /* three sample buffers: a step consumes one and loads the step two
-     * ahead into the one its predecessor consumed.  Full steps go in groups
-     * of three with the buffers in place, so no register copy waits on a
-     * load in flight; the last steps (fewer than three, or a partial one)
-     * rotate the buffers.  Full steps carry no per-lane sample guard. */
-    T bA[7], bB[7], bC[7];
-    Off sof = (Off)((b0 + lane) * (int64_t)sizeof(T)); /* byte offsets, advanced 16 samples a step */
-    Off dof = (Off)((d0 + lane) * (int64_t)sizeof(T));
-    const Off last = (Off)((b0 + S - 1) * (int64_t)sizeof(T)); /* the cloud's last sample */
-    if (lane < S) load_sample_off(src, sof, bA);
-    sof += (Off)(16 * sizeof(T));
-    if (lane + 16 < S) load_sample_off(src, sof, bB);
-    /* one step of 16 samples, s0 .. s0 + 15, from `cur`, loading the step
-     * two ahead into `fill`; FULL: all of them exist.  That load is
-     * unconditional (no branch in the loop): past the end of the cloud it
-     * reads the last sample again. */
-    auto step = [&](auto full, const T(&cur)[7], T(&fill)[7], int s0) {
+    /* two sample buffers, used in place: a step takes its samples out of one
+     * and at once loads the step two ahead into it.  Steps go in groups of
+     * four, the noise group, so that a step's place in it (which normals it
+     * draws and which it carries) is fixed. */
+    T buf[2][7];
+    load_step(from, S, lane, buf[0]);
+    load_step(from + 112, S - 16, lane, buf[1]);
+    /* one step of 16 samples, s0 .. s0 + 15, member J of its noise group;
+     * FULL: all of them exist */
+    auto step = [&](auto full, auto member, int s0) {
         constexpr bool FULL = decltype(full)::value;
+        constexpr int J = decltype(member)::value;
+        T(&b)[7] = buf[J & 1];
         const int s = s0 + lane;
         const bool valid = FULL || s < S;
-        sof += (Off)(16 * sizeof(T));
-        load_sample_off(src, s + 32 < S ? sof : last, fill);
+        const int width = FULL ? 16 : min(S - s0, 16);
+        T* const o = to + 7 * s0 + lane;
+        float n[3] = {0.0f, 0.0f, 0.0f};
+        NoiseKey key = pc.key; /* its round keys are formed anew, not held over the sweep */
+        asm volatile("" : "+s"(key.k0), "+s"(key.k1));
+        if (a.pending && valid)
+            feature_normals_seq(key, pc.step, (uint32_t)pc.pl, (uint32_t)k, (uint32_t)s, (uint32_t)J, fc, n);
+        A x[6];
+#pragma unroll
+        for (int c = 0; c < 6; ++c) x[c] = (A)b[c];
+        A w = (A)b[6];
+        /* out of the buffer before the loads into it */
+        asm volatile("" : "+v"(w));
+#pragma unroll
+        for (int c = 0; c < 6; ++c) asm volatile("" : "+v"(x[c]));
+        if (FULL && J < 2) /* in the same group, which is whole */
+            load_full_step(from + 7 * (s0 + 32), lane, b);
+        else
+            load_step(from + 7 * (s0 + 32), S - s0 - 32, lane, b);
+        if (a.pending && valid) {
+            if constexpr (F32) {
+                predict_f(x, cx.mo, n);
+            } else {
+                const double an[3] = {(double)n[0], (double)n[1], (double)n[2]};
+                const EuclideanPoint e =
+                    noisy_motion(EuclideanPoint{x[0], x[1], x[2], x[3], x[4], x[5]}, a.motion, an);
+                x[0] = e.x; x[1] = e.y; x[2] = e.z; x[3] = e.vx; x[4] = e.vy; x[5] = e.vz;
+            }
+        }
+        if (nd_write && valid) {
+#pragma unroll
+            for (int c = 0; c < 6; ++c) o[c * width] = (T)x[c];
+        }
         A q[6] = {0, 0, 0, 0, 0, 0};
         bool in = false;
-        A w = 0;
-        [[maybe_unused]] EuclideanPoint x;
-        [[maybe_unused]] float xf[6];
-        if constexpr (F32) {
-            if (valid) eval_sample_f(a, cx, cur, kk, pl, k, s, xf, q, in, w, &fc, (uint32_t)(s0 >> 4) & 3u);
-        } else {
-            DisparityPoint d;
-            if (valid) {
-                eval_sample(a, meas, cur, kk, pl, k, s, pose, x, d, in, w, &fc, (uint32_t)(s0 >> 4) & 3u);
+        if (valid) {
+            if constexpr (F32) {
+                disparity_f(cx.m, cx.pose, x, q);
+                in = in_range_f(cx.m, q);
+            } else {
+                const DisparityPoint d =
+                    disparity_fast(meas, pose, EuclideanPoint{x[0], x[1], x[2], x[3], x[4], x[5]});
+                in = meas.inRange(d);
                 q[0] = d.u; q[1] = d.v; q[2] = d.d; q[3] = d.vu; q[4] = d.vv; q[5] = d.vd;
             }
         }
+        if (nd_write && valid) o[6 * width] = (T)(1.0 - (in ? Pd : 0.0));
         const A pd = in ? PdA : (A)0;
         const A wp = valid ? w * pd : (A)0;
-        if (s0 == 0) {
+        if (J == 0 && s0 == 0) {
             /* shift: the Gaussian's first sample, broadcast along the row
              * (the fit of a cloud with no weighted sample) */
 #pragma unroll
@@ -598,70 +706,111 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SCPHD_FIT_W
         for (int r = 0; r < 6; ++r)
 #pragma unroll
             for (int c = 0; c <= r; ++c) m2[pidx(r, c)] += wp * dv[r] * dv[c];
-        if (nd_write && valid) {
-            if constexpr (F32)
-                write_nd_off_f(meas, dst, dof, xf, in);
-            else
-                write_nd_off(meas, dst, dof, x, in);
-        }
-        dof += (Off)(16 * sizeof(T));
+        /* the sums stay in this step: left alone, the compiler moves all four
+         * steps' to the group's end, and their points wait in registers */
+        asm volatile("" : "+v"(sw), "+v"(sw2));
+        if constexpr (F32)
+            asm volatile("" : "+v"(nin));
+        else
+            asm volatile("" : "+v"(spd));
+#pragma unroll
+        for (int c = 0; c < 6; ++c) asm volatile("" : "+v"(m1[c]));
+#pragma unroll
+        for (int e = 0; e < 21; ++e) asm volatile("" : "+v"(m2[e]));
     };
     const std::integral_constant<bool, true> full;
-    const std::integral_constant<bool, false> guarded;
+    const std::integral_constant<bool, false> part;
+    const std::integral_constant<int, 0> j0;
+    const std::integral_constant<int, 1> j1;
+    const std::integral_constant<int, 2> j2;
+    const std::integral_constant<int, 3> j3;
     int s0 = 0;
-    for (; s0 + 48 <= S; s0 += 48) { /* three full steps, buffers in place */
-        step(full, bA, bC, s0);
-        step(full, bB, bA, s0 + 16);
-        step(full, bC, bB, s0 + 32);
+    for (; s0 + 64 <= S; s0 += 64) {
+        step(full, j0, s0);
+        step(full, j1, s0 + 16);
+        step(full, j2, s0 + 32);
+        step(full, j3, s0 + 48);
     }
-    for (; s0 < S; s0 += 16) { /* the last steps: buffers rotate */
-        step(guarded, bA, bC, s0);
+    if (s0 < S) { /* the last group: fewer steps, the last of them partial */
+        step(part, j0, s0);
+        if (s0 + 16 < S) step(part, j1, s0 + 16);
+        if (s0 + 32 < S) step(part, j2, s0 + 32);
+        if (s0 + 48 < S) step(part, j3, s0 + 48);
+    }
+    /* The row sums: sixteen values at a time, every lane's part of them
+     * through LDS, each lane adding up the value of its own number -- m1 and
+     * m2 at their fit planes, then sum pd_i (or the in-view count), sw, sw2.
+     * The rest of the fit goes on a value a lane.  (Row sums by DPP with the
+     * rest in every lane took 600 instructions a Gaussian, a seventh of the
+     * kernel at S = 200 and a quarter at S = 100; this takes about 170.) */
+    A v0[16], v1[16];
 #pragma unroll
-        for (int c = 0; c < 7; ++c) {
-            bA[c] = bB[c];
-            bB[c] = bC[c];
-        }
-    }
-    /* the row sums, then the rest in double */
+    for (int c = 0; c < 6; ++c) v0[c] = m1[c];
+#pragma unroll
+    for (int e = 0; e < 10; ++e) v0[6 + e] = m2[e];
+#pragma unroll
+    for (int e = 10; e < 21; ++e) v1[e - 10] = m2[e];
     if constexpr (F32)
-        spd = (double)row_sum16(nin) * Pd;
+        v1[11] = nin;
     else
-        spd = row_sum16(spd);
-    const double sw_r = (double)row_sum16(sw);
-    const double sw2_r = (double)row_sum16(sw2);
-    double m1r[6], m2r[21];
+        v1[11] = spd;
+    v1[12] = sw;
+    v1[13] = sw2;
+    v1[14] = v1[15] = 0;
+    const FitArgs& o = kernarg_late<FitArgs>();
+    const double t0 = row_total(sh.part, v0, lane), t1 = row_total(sh.part, v1, lane);
+    sh.tot[lane] = t0;
+    sh.tot[16 + lane] = t1;
+    if (lane == 0) {
 #pragma unroll
-    for (int c = 0; c < 6; ++c) m1r[c] = (double)row_sum16(m1[c]);
-#pragma unroll
-    for (int e = 0; e < 21; ++e) m2r[e] = (double)row_sum16(m2[e]);
-    const double pdg = spd / S;
+        for (int c = 0; c < 6; ++c) sh.K[c] = (double)K[c];
+    }
+    wave_lds_fence();
+    const double sum_pd = F32 ? sh.tot[FP_PD] * Pd : sh.tot[FP_PD], sw_r = sh.tot[28], sw2_r = sh.tot[29];
+    const double pdg = sum_pd / S;
 
     /* normalised weights w'_i / sum w': mean K + sum w (q - K); centred
      * covariance sum w (q - K)(q - K)^T - (2 - W) dm dm^T with W = sum w */
     const double r = sw_r > 0 ? 1.0 / sw_r : 0.0;
     const double W = sw_r * r, W2 = sw2_r * r * r;
-    double mu[6], dm[6], P[21];
-#pragma unroll
-    for (int c = 0; c < 6; ++c) {
-        dm[c] = m1r[c] * r;
-        mu[c] = (double)K[c] + dm[c];
-    }
     /* W = 0: with pd_g = 0 the fit is the first sample with zero covariance
      * (its detection terms have weight 0); with pd_g > 0 (possible only when
      * Pd = 1) k_fit_fix refits it with unit weights, as the reference does */
     const double scale = W > 0 ? (W * W + W2) / W : 0.0;
-#pragma unroll
-    for (int i = 0; i < 6; ++i)
-#pragma unroll
-        for (int j = 0; j <= i; ++j) P[pidx(i, j)] = (m2r[pidx(i, j)] * r - (2.0 - W) * dm[i] * dm[j]) * scale;
-    write_fit(a, g, lane, mu, P, pdg);
-
-    const bool keep = wg * (1 - pdg) >= a.min_weight;
+    auto cov = [&](int e, double t) { /* packed entry e of the covariance */
+        const int i = (e >= 1) + (e >= 3) + (e >= 6) + (e >= 10) + (e >= 15), j = e - i * (i + 1) / 2;
+        const double di = sh.tot[i] * r, dj = sh.tot[j] * r;
+        return (t * r - (2.0 - W) * di * dj) * scale;
+    };
+    const double f0 = lane < 6 ? sh.K[lane < 6 ? lane : 0] + t0 * r : cov(max(lane - 6, 0), t0);
+    const double f1 = lane < 11 ? cov(min(lane + 10, 20), t1) : pdg;
+    o.fit[(int64_t)lane * o.Ng + g] = f0;
+    if (lane < 12) o.fit[(int64_t)(lane + 16) * o.Ng + g] = f1;
+    const bool keep = wg * (1 - pdg) >= o.min_weight;
     if (lane == 0) {
-        a.keep[g] = keep ? 1 : 0;
-        if (sw_r == 0 && spd != 0.0) a.redo[atomicAdd(a.redo_n, 1)] = (int32_t)g;
-        if (keep && !nd_write) a.ndfill[atomicAdd(a.ndfill_n, 1)] = (int32_t)g;
+        o.keep[g] = keep ? 1 : 0;
+        if (sw_r == 0 && sum_pd != 0.0) o.redo[atomicAdd(o.redo_n, 1)] = (int32_t)g;
+        if (keep && !nd_write) o.ndfill[atomicAdd(o.ndfill_n, 1)] = (int32_t)g;
     }
+}
+
+template <typename T, typename A = double>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SCPHD_FIT_WAVES, SCPHD_FIT_WAVES))) void k_fit(
+    FitKernArgs<T> ka) {
+    __shared__ FitShared<A> sh[16];
+    const int w = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
+    if (w >= ka.a.n_waves) return;
+    const int p = ((cint_t*)ka.a.wave_parent)[w];
+    if (p < 0) return;
+    cint_t* off = (cint_t*)ka.a.goff + p;
+    const int k = 4 * (w - first_wave(off[0], p)) + ((threadIdx.x & 63) >> 4);
+    if (k >= off[1] - off[0]) return; /* whole rows; rows never exchange data */
+    const int64_t g = off[0] + k;
+    const T* const from = ka.src.block(ka.a.gblock[g]);
+    T* const to = ka.dst.block(ka.a.nd_base + g);
+    const FitArgs& a = kernarg_late<FitArgs>();
+    const ParentCtx pc(a.pose, a.meas, a.rig_meas, a.key, a.pstep, p);
+    fit_row<T, A>(a, pc, g, k, from, to, sh[threadIdx.x >> 4]);
 }
 
 /* The non-detection clouds of the terms k_fit decided only after its sweep
@@ -669,8 +818,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SCPHD_FIT_W
  * weights 1 - pd_i, computed by the same code as in the sweep.  One 16-lane
  * row per listed term; workgroups stride over the list (its length is read
  * on the device). */
-template <typename T, typename Off, bool RG, typename A = double>
-__global__ __launch_bounds__(256) void k_nd_fill(FitArgs a, Planes<T> src, Planes<T> dst) {
+template <typename T, bool RG, typename A = double>
+__global__ __launch_bounds__(256) void k_nd_fill(FitArgs a, Clouds<T> src, Clouds<T> dst) {
     constexpr bool F32 = std::is_same_v<A, float>;
     const int lane = threadIdx.x & 15;
     const int n = *a.ndfill_n;
@@ -683,8 +832,8 @@ __global__ __launch_bounds__(256) void k_nd_fill(FitArgs a, Planes<T> src, Plane
         const auto kk = row_key<RG>(a.key, p, pl);
         const RowMeas<RG> rm(a.meas, a.rig_meas, a.key, p);
         const DisparityMeasurementModel& meas = rm.m;
-        const int64_t b0 = (int64_t)a.gblock[g] * a.S;
-        const int64_t d0 = (a.nd_base + g) * (int64_t)a.S;
+        const T* from = src.block(a.gblock[g]);
+        T* to = dst.block(a.nd_base + g);
         const CameraPose pose = load_pose(a.pose, p);
         SampleCtxF cx;
         if constexpr (F32) cx = SampleCtxF{meas_f(meas), pose_f(pose), motion_f(a.feat, a.dt)};
@@ -694,26 +843,29 @@ __global__ __launch_bounds__(256) void k_nd_fill(FitArgs a, Planes<T> src, Plane
         for (int s0 = 0; s0 < a.S; s0 += 64) {
             T r[4][7];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int s = s0 + 16 * j + lane;
-                if (s < a.S) load_sample_off(src, (Off)((b0 + s) * (int64_t)sizeof(T)), r[j]);
-            }
+            for (int j = 0; j < 4; ++j) load_step(from + 7 * (s0 + 16 * j), a.S - s0 - 16 * j, lane, r[j]);
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const int s = s0 + 16 * j + lane;
                 if (s < a.S) {
+                    T* const o = to + 7 * (s - lane) + lane;
+                    const int w = min(a.S - s0 - 16 * j, 16);
                     bool in;
                     if constexpr (F32) {
-                        float x[6], q[6], w;
-                        eval_sample_f(a, cx, r[j], kk, pl, k, s, x, q, in, w, &fc, (uint32_t)j);
-                        write_nd_off_f(meas, dst, (Off)((d0 + s) * (int64_t)sizeof(T)), x, in);
+                        float x[6], q[6], sw;
+                        eval_sample_f(a, cx, r[j], kk, pl, k, s, x, q, in, sw, &fc, (uint32_t)j);
+#pragma unroll
+                        for (int c = 0; c < 6; ++c) o[c * w] = (T)x[c];
                     } else {
                         EuclideanPoint x;
                         DisparityPoint d;
-                        double w;
-                        eval_sample(a, meas, r[j], kk, pl, k, s, pose, x, d, in, w, &fc, (uint32_t)j);
-                        write_nd_off(meas, dst, (Off)((d0 + s) * (int64_t)sizeof(T)), x, in);
+                        double sw;
+                        eval_sample(a, meas, r[j], kk, pl, k, s, pose, x, d, in, sw, &fc, (uint32_t)j);
+                        const double xs[6] = {x.x, x.y, x.z, x.vx, x.vy, x.vz};
+#pragma unroll
+                        for (int c = 0; c < 6; ++c) o[c * w] = (T)xs[c];
                     }
+                    o[6 * w] = (T)(1.0 - (in ? meas.pd() : 0.0));
                 }
             }
         }
@@ -726,7 +878,7 @@ __global__ __launch_bounds__(256) void k_nd_fill(FitArgs a, Planes<T> src, Plane
  * gives).  Workgroups stride over the list (its length is read on the
  * device). */
 template <typename T, bool RG, typename A = double>
-__global__ __launch_bounds__(256) void k_fit_fix(FitArgs a, Planes<T> src, Planes<T> dst) {
+__global__ __launch_bounds__(256) void k_fit_fix(FitArgs a, Clouds<T> src, Clouds<T> dst) {
     constexpr bool F32 = std::is_same_v<A, float>;
     const int lane = threadIdx.x & 15;
     const int nredo = *a.redo_n;
@@ -739,15 +891,15 @@ __global__ __launch_bounds__(256) void k_fit_fix(FitArgs a, Planes<T> src, Plane
         const auto kk = row_key<RG>(a.key, p, pl);
         const RowMeas<RG> rm(a.meas, a.rig_meas, a.key, p);
         const DisparityMeasurementModel& meas = rm.m;
-        const int64_t b0 = (int64_t)a.gblock[g] * S;
+        const T* from = src.block(a.gblock[g]);
         const CameraPose pose = load_pose(a.pose, p);
         SampleCtxF cx;
         if constexpr (F32) cx = SampleCtxF{meas_f(meas), pose_f(pose), motion_f(a.feat, a.dt)};
         /* the sample's disparity-space point in the arithmetic type */
         auto point = [&](int s, A q[6]) {
+            T r[7];
+            load_sample<T>(from, S, s, r);
             if constexpr (F32) {
-                T r[7];
-                load_sample(src, b0 + s, r);
                 float x[6], w;
                 bool in;
                 eval_sample_f(a, cx, r, kk, pl, k, s, x, q, in, w);
@@ -756,7 +908,7 @@ __global__ __launch_bounds__(256) void k_fit_fix(FitArgs a, Planes<T> src, Plane
                 DisparityPoint d;
                 bool in;
                 double w;
-                fit_sample(a, meas, src, b0 + s, kk, pl, k, s, pose, x, d, in, w);
+                eval_sample(a, meas, r, kk, pl, k, s, pose, x, d, in, w);
                 q[0] = d.u; q[1] = d.v; q[2] = d.d; q[3] = d.vu; q[4] = d.vv; q[5] = d.vd;
             }
         };
@@ -2154,47 +2306,42 @@ __device__ inline int64_t posterior_block(const int32_t* holes, int64_t nholes, 
  * to the world by the parent's camera (disparityToWorldKernel,
  * src/kernels.cu:49-80), sample weight 1/S (:2009-2010).  Merged Gaussian
  * gm's cloud goes to the block of a dropped non-detection term while there
- * are any (holes), else after them (posterior_block).  Destination
- * addresses are byte offsets from the plane bases (32-bit while every
- * destination lies below 4 GiB). */
-template <typename T, typename Off, bool RG, typename A = double>
-__global__ __launch_bounds__(256) void k_sample(SampleArgs a, Planes<T> dst) {
+ * are any (holes), else after them (posterior_block).  The parent is the same
+ * for every row, its data in scalar registers. */
+template <typename T, typename A>
+__device__ inline void sample_row(const SampleArgs& a, const ParentCtx& pc, int64_t rec, int k, T* to) {
     constexpr bool F32 = std::is_same_v<A, float>;
     const int lane = threadIdx.x & 15;
-    const int64_t gm = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4);
-    if (gm >= a.Kt) return; /* whole rows */
-    const int p = upper_parent(a.mergeoff, a.Np, gm);
-    const int k = (int)(gm - a.mergeoff[p]);
-    int pl;
-    const auto key = row_key<RG>(a.key, p, pl);
-    const RowMeas<RG> rm(a.meas, a.rig_meas, a.key, p);
-    const DisparityMeasurementModel& meas = rm.m;
-    const int64_t rec = (int64_t)a.survoff[p] + k;
     double mu[6], P[21], L[21];
 #pragma unroll
     for (int c = 0; c < 6; ++c) mu[c] = a.mmu[c * a.scap + rec];
 #pragma unroll
     for (int e = 0; e < 21; ++e) P[e] = a.mP[e * a.scap + rec];
     chol6(P, L);
-    const CameraPose pose = load_pose(a.pose, p);
-    const T w = (T)(1.0 / a.S);
-    Off off = (Off)((posterior_block(a.holes, a.nholes, a.post_base, gm) * (int64_t)a.S + lane) * (int64_t)sizeof(T));
-    PosteriorCarry pc; /* normals carried between the two steps of a noise group */
+    /* the FP32-arithmetic variant: the factor and mean rounded to single
+     * precision once, each draw and its unprojection in single precision */
+    MeasF mf;
+    PoseF pf;
+    A Lf[21], muf[6];
     if constexpr (F32) {
-        /* the FP32-arithmetic variant: the factor and mean rounded to
-         * single precision once, each draw and its unprojection in single
-         * precision */
-        const MeasF mf = meas_f(meas);
-        const PoseF pf = pose_f(pose);
-        float Lf[21], muf[6];
+        mf = meas_f(pc.meas);
+        pf = pose_f(pc.pose);
+    }
 #pragma unroll
-        for (int e = 0; e < 21; ++e) Lf[e] = (float)L[e];
+    for (int e = 0; e < 21; ++e) Lf[e] = (A)L[e];
 #pragma unroll
-        for (int c = 0; c < 6; ++c) muf[c] = (float)mu[c];
-        for (int s = lane; s < a.S; s += 16) {
-            float z[6], q[6], x[6];
-            posterior_normals_seq(key, a.ustep, (uint32_t)pl, (uint32_t)k, (uint32_t)s, (uint32_t)(s >> 4) & 1u, pc,
-                                  z);
+    for (int c = 0; c < 6; ++c) muf[c] = (A)mu[c];
+    const T w = (T)(1.0 / a.S);
+    PosteriorCarry carry; /* normals carried between the two steps of a noise group */
+    /* the lane's sample s, member J of its noise group */
+    auto draw = [&](int s, auto member, T x[6]) {
+        constexpr uint32_t J = decltype(member)::value;
+        A z[6];
+        NoiseKey key = pc.key; /* its round keys are formed anew, not held over the sweep */
+        asm volatile("" : "+s"(key.k0), "+s"(key.k1));
+        posterior_normals_seq(key, pc.step, (uint32_t)pc.pl, (uint32_t)k, (uint32_t)s, J, carry, z);
+        if constexpr (F32) {
+            float q[6], xf[6];
 #pragma unroll
             for (int r = 0; r < 6; ++r) {
                 float acc = muf[r];
@@ -2202,44 +2349,69 @@ __global__ __launch_bounds__(256) void k_sample(SampleArgs a, Planes<T> dst) {
                 for (int c = 0; c <= r; ++c) acc = __builtin_fmaf(Lf[pidx(r, c)], z[c], acc);
                 q[r] = acc;
             }
-            world_from_disparity_f(mf, pf, q, x);
+            world_from_disparity_f(mf, pf, q, xf);
 #pragma unroll
-            for (int c = 0; c < 6; ++c) at(dst.p[c], off) = (T)x[c];
-            at(dst.p[6], off) = w;
-            off += (Off)(16 * sizeof(T));
+            for (int c = 0; c < 6; ++c) x[c] = (T)xf[c];
+        } else {
+            double q[6];
+#pragma unroll
+            for (int r = 0; r < 6; ++r) {
+                double acc = 0.0;
+#pragma unroll
+                for (int c = 0; c <= r; ++c) acc += Lf[pidx(r, c)] * z[c];
+                q[r] = acc + muf[r];
+            }
+            const DisparityPoint d{q[0], q[1], q[2], q[3], q[4], q[5]};
+            const EuclideanPoint e = world_from_disparity_fast(pc.meas, pc.pose, d);
+            x[0] = (T)e.x; x[1] = (T)e.y; x[2] = (T)e.z; x[3] = (T)e.vx; x[4] = (T)e.vy; x[5] = (T)e.vz;
         }
-        return;
-    }
-    for (int s = lane; s < a.S; s += 16) {
-        double z[6];
-        posterior_normals_seq(key, a.ustep, (uint32_t)pl, (uint32_t)k, (uint32_t)s, (uint32_t)(s >> 4) & 1u, pc, z);
-        double q[6];
+    };
+    auto put = [&](int s0, const T x[6]) {
+        T* const o = to + 7 * s0 + lane;
+        const int wd = min(a.S - s0, 16);
 #pragma unroll
-        for (int r = 0; r < 6; ++r) {
-            double acc = 0.0;
-#pragma unroll
-            for (int c = 0; c <= r; ++c) acc += L[pidx(r, c)] * z[c];
-            q[r] = acc + mu[r];
+        for (int c = 0; c < 6; ++c) __builtin_nontemporal_store(x[c], &o[c * wd]); /* next read in the next update */
+        __builtin_nontemporal_store(w, &o[6 * wd]);
+    };
+    for (int s0 = 0; s0 < a.S; s0 += 32) { /* a pair of steps is a noise group */
+        T x[6];
+        if (s0 + lane < a.S) {
+            draw(s0 + lane, std::integral_constant<uint32_t, 0>(), x);
+            put(s0, x);
         }
-        const DisparityPoint d{q[0], q[1], q[2], q[3], q[4], q[5]};
-        const EuclideanPoint x = world_from_disparity_fast(meas, pose, d);
-        at(dst.p[0], off) = (T)x.x;
-        at(dst.p[1], off) = (T)x.y;
-        at(dst.p[2], off) = (T)x.z;
-        at(dst.p[3], off) = (T)x.vx;
-        at(dst.p[4], off) = (T)x.vy;
-        at(dst.p[5], off) = (T)x.vz;
-        at(dst.p[6], off) = w;
-        off += (Off)(16 * sizeof(T));
+        if (s0 + 16 + lane < a.S) {
+            draw(s0 + 16 + lane, std::integral_constant<uint32_t, 1>(), x);
+            put(s0 + 16, x);
+        }
     }
 }
 
+template <typename T, typename A = double>
+__global__ __launch_bounds__(256) void k_sample(SampleKernArgs<T> ka) {
+    const int w = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
+    if (w >= ka.a.n_waves) return;
+    const int p = ((cint_t*)ka.a.wave_parent)[w];
+    if (p < 0) return;
+    cint_t* off = (cint_t*)ka.a.mergeoff + p;
+    const int k = 4 * (w - first_wave(off[0], p)) + ((threadIdx.x & 63) >> 4);
+    if (k >= off[1] - off[0]) return; /* whole rows */
+    T* const to = ka.dst.block(posterior_block(ka.a.holes, ka.a.nholes, ka.a.post_base, off[0] + k));
+    const SampleArgs& a = kernarg_late<SampleArgs>();
+    const ParentCtx pc(a.pose, a.meas, a.rig_meas, a.key, a.ustep, p);
+    const int64_t rec = (int64_t)((cint_t*)a.survoff)[p] + k;
+    sample_row<T, A>(a, pc, rec, k, to);
+}
+
 /* -------------------------------------------------------- map assembly */
-__global__ void k_outcount(const int32_t* nmerged, const int32_t* goff, const int32_t* keepscan, int Np,
-                           int32_t* outcnt) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
+/* Map sizes after the update, and the posterior terms' wave_parent.  One
+ * wavefront per parent. */
+__global__ __launch_bounds__(256) void k_outcount(const int32_t* nmerged, const int32_t* goff, const int32_t* keepscan,
+                                                  int Np, int32_t* outcnt, const int32_t* mergeoff,
+                                                  int32_t* wave_parent) {
+    const int p = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (p >= Np) return;
-    outcnt[p] = nmerged[p] + (keepscan[goff[p + 1]] - keepscan[goff[p]]);
+    write_wave_parents(mergeoff[p], mergeoff[p + 1], p, lane, wave_parent);
+    if (lane == 0) outcnt[p] = nmerged[p] + (keepscan[goff[p + 1]] - keepscan[goff[p]]);
 }
 
 __global__ void k_ndlist(const int32_t* keep, const int32_t* keepscan, int64_t Ng, int32_t* ndlist,
@@ -2472,35 +2644,39 @@ __global__ void k_table_resample(const int32_t* anc, const int32_t* goff_old, co
 
 /* ------------------------------------------------------------ read-back */
 /* The map's clouds into consecutive blocks: block g of dst <- block
- * gblock[g] of src, every plane. */
+ * gblock[g] of src. */
 template <typename T>
-__global__ void k_gather(Planes<T> src, Planes<T> dst, const int32_t* gblock, int64_t Ng, int S) {
+__global__ void k_gather(Clouds<T> src, Clouds<T> dst, const int32_t* gblock, int64_t Ng, int S) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= Ng * S) return;
-    const int64_t g = i / S;
-    const int64_t si = (int64_t)gblock[g] * S + (i - g * S);
-#pragma unroll
-    for (int c = 0; c < 7; ++c) dst.p[c][i] = src.p[c][si];
+    const int n = 7 * S;
+    if (i >= Ng * n) return;
+    const int64_t g = i / n;
+    const int e = (int)(i - g * n);
+    dst.block(g)[e] = src.block(gblock[g])[e];
 }
 
 template <typename T>
-__global__ void k_extract(Planes<T> src, const int32_t* gblock, int64_t Ng, int S, double* out) {
+__global__ void k_extract(Clouds<T> src, const int32_t* gblock, int64_t Ng, int S, double* out) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int64_t n = Ng * S;
     if (i >= n) return;
     const int64_t g = i / S;
-    const int64_t si = (int64_t)gblock[g] * S + (i - g * S);
+    T r[7];
+    load_sample<T>(src.block(gblock[g]), S, (int)(i - g * S), r);
 #pragma unroll
-    for (int c = 0; c < 7; ++c) out[c * n + i] = (double)src.p[c][si];
+    for (int c = 0; c < 7; ++c) out[c * n + i] = (double)r[c];
 }
 
 template <typename T>
-__global__ void k_inject(const double* in, int64_t Ng, int S, Planes<T> dst) {
+__global__ void k_inject(const double* in, int64_t Ng, int S, Clouds<T> dst) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int64_t n = Ng * S;
     if (i >= n) return;
+    const int64_t g = i / S;
+    const int s = (int)(i - g * S);
+    T* const b = dst.block(g);
 #pragma unroll
-    for (int c = 0; c < 7; ++c) dst.p[c][i] = (T)in[c * n + i];
+    for (int c = 0; c < 7; ++c) b[cloud_at(S, s, c)] = (T)in[c * n + i];
 }
 
 /* ----------------------------------------------------------------- scan */
@@ -2573,15 +2749,17 @@ hipError_t launch_scale(hipStream_t s, double* x, int64_t n, double a) {
     LAUNCH_CHECK();
 }
 
+int64_t wave_count(int64_t n, int Np) { return n / 4 + Np; }
+
 hipError_t launch_pose(hipStream_t s, const double* ext, double* pose, int Np, int fixed, const int32_t* prig,
-                       const int32_t* rfixed) {
+                       const int32_t* rfixed, const int32_t* goff, int32_t* wave_parent) {
     if (rfixed && !prig) return hipErrorInvalidValue;
-    k_pose<<<nblocks(Np, 256), 256, 0, s>>>(ext, pose, Np, fixed, prig, rfixed);
+    k_pose<<<nblocks(Np, 4), 256, 0, s>>>(ext, pose, Np, fixed, prig, rfixed, goff, wave_parent);
     LAUNCH_CHECK();
 }
 
 template <typename T>
-hipError_t launch_materialize(hipStream_t s, Planes<T> src, Planes<T> dst, const int32_t* gblock,
+hipError_t launch_materialize(hipStream_t s, Clouds<T> src, Clouds<T> dst, const int32_t* gblock,
                               const int32_t* gparent, const int32_t* goff, int64_t Ng, int S,
                               LinearCVMotionModel3D feat, double dt, RigKeys key, uint64_t step, bool arith32) {
     if (Ng <= 0) return hipSuccess;
@@ -2592,39 +2770,23 @@ hipError_t launch_materialize(hipStream_t s, Planes<T> src, Planes<T> dst, const
 }
 
 template <typename T>
-hipError_t launch_fit(hipStream_t s, const FitArgs& a, Planes<T> src, Planes<T> dst) {
+hipError_t launch_fit(hipStream_t s, const FitArgs& a, Clouds<T> src, Clouds<T> dst) {
     if (a.Ng <= 0) return hipSuccess;
-    const unsigned nb = nblocks(a.Ng, 16);
+    const unsigned nb = nblocks(a.n_waves, 4);
     if constexpr (std::is_same_v<T, float>) {
         if (a.arith32) {
-            if (a.rig_meas) {
-                if (a.off32)
-                    k_fit<T, uint32_t, true, float><<<nb, 256, 0, s>>>(a, src, dst);
-                else
-                    k_fit<T, uint64_t, true, float><<<nb, 256, 0, s>>>(a, src, dst);
-            } else if (a.off32)
-                k_fit<T, uint32_t, false, float><<<nb, 256, 0, s>>>(a, src, dst);
-            else
-                k_fit<T, uint64_t, false, float><<<nb, 256, 0, s>>>(a, src, dst);
+            k_fit<T, float><<<nb, 256, 0, s>>>(FitKernArgs<T>{a, src, dst});
             LAUNCH_CHECK();
         }
     } else if (a.arith32) {
         return hipErrorInvalidValue;
     }
-    if (a.rig_meas) {
-        if (a.off32)
-            k_fit<T, uint32_t, true><<<nb, 256, 0, s>>>(a, src, dst);
-        else
-            k_fit<T, uint64_t, true><<<nb, 256, 0, s>>>(a, src, dst);
-    } else if (a.off32)
-        k_fit<T, uint32_t, false><<<nb, 256, 0, s>>>(a, src, dst);
-    else
-        k_fit<T, uint64_t, false><<<nb, 256, 0, s>>>(a, src, dst);
+    k_fit<T><<<nb, 256, 0, s>>>(FitKernArgs<T>{a, src, dst});
     LAUNCH_CHECK();
 }
 
 template <typename T>
-hipError_t launch_fit_fix(hipStream_t s, const FitArgs& a, Planes<T> src, Planes<T> dst) {
+hipError_t launch_fit_fix(hipStream_t s, const FitArgs& a, Clouds<T> src, Clouds<T> dst) {
     if (a.Ng <= 0) return hipSuccess;
     const unsigned nb = (unsigned)std::min<int64_t>(nblocks(a.Ng, 16), 256);
     if constexpr (std::is_same_v<T, float>) {
@@ -2646,34 +2808,24 @@ hipError_t launch_fit_fix(hipStream_t s, const FitArgs& a, Planes<T> src, Planes
 }
 
 template <typename T>
-hipError_t launch_nd_fill(hipStream_t s, const FitArgs& a, Planes<T> src, Planes<T> dst) {
+hipError_t launch_nd_fill(hipStream_t s, const FitArgs& a, Clouds<T> src, Clouds<T> dst) {
     if (a.Ng <= 0) return hipSuccess;
     const int64_t blocks = std::min<int64_t>(nblocks(a.Ng, 16), 2048); /* the list is at most Ng long */
     if constexpr (std::is_same_v<T, float>) {
         if (a.arith32) {
-            if (a.rig_meas) {
-                if (a.off32)
-                    k_nd_fill<T, uint32_t, true, float><<<blocks, 256, 0, s>>>(a, src, dst);
-                else
-                    k_nd_fill<T, uint64_t, true, float><<<blocks, 256, 0, s>>>(a, src, dst);
-            } else if (a.off32)
-                k_nd_fill<T, uint32_t, false, float><<<blocks, 256, 0, s>>>(a, src, dst);
+            if (a.rig_meas)
+                k_nd_fill<T, true, float><<<blocks, 256, 0, s>>>(a, src, dst);
             else
-                k_nd_fill<T, uint64_t, false, float><<<blocks, 256, 0, s>>>(a, src, dst);
+                k_nd_fill<T, false, float><<<blocks, 256, 0, s>>>(a, src, dst);
             LAUNCH_CHECK();
         }
     } else if (a.arith32) {
         return hipErrorInvalidValue;
     }
-    if (a.rig_meas) {
-        if (a.off32)
-            k_nd_fill<T, uint32_t, true><<<blocks, 256, 0, s>>>(a, src, dst);
-        else
-            k_nd_fill<T, uint64_t, true><<<blocks, 256, 0, s>>>(a, src, dst);
-    } else if (a.off32)
-        k_nd_fill<T, uint32_t, false><<<blocks, 256, 0, s>>>(a, src, dst);
+    if (a.rig_meas)
+        k_nd_fill<T, true><<<blocks, 256, 0, s>>>(a, src, dst);
     else
-        k_nd_fill<T, uint64_t, false><<<blocks, 256, 0, s>>>(a, src, dst);
+        k_nd_fill<T, false><<<blocks, 256, 0, s>>>(a, src, dst);
     LAUNCH_CHECK();
 }
 
@@ -2725,40 +2877,24 @@ hipError_t launch_estimate(hipStream_t s, const double* ext, const double* pw, c
 }
 
 template <typename T>
-hipError_t launch_sample(hipStream_t s, const SampleArgs& a, Planes<T> dst) {
+hipError_t launch_sample(hipStream_t s, const SampleArgs& a, Clouds<T> dst) {
     if (a.Kt <= 0) return hipSuccess;
-    const unsigned nb = nblocks(a.Kt, 16);
+    const unsigned nb = nblocks(a.n_waves, 4);
     if constexpr (std::is_same_v<T, float>) {
         if (a.arith32) {
-            if (a.rig_meas) {
-                if (a.off32)
-                    k_sample<T, uint32_t, true, float><<<nb, 256, 0, s>>>(a, dst);
-                else
-                    k_sample<T, uint64_t, true, float><<<nb, 256, 0, s>>>(a, dst);
-            } else if (a.off32)
-                k_sample<T, uint32_t, false, float><<<nb, 256, 0, s>>>(a, dst);
-            else
-                k_sample<T, uint64_t, false, float><<<nb, 256, 0, s>>>(a, dst);
+            k_sample<T, float><<<nb, 256, 0, s>>>(SampleKernArgs<T>{a, dst});
             LAUNCH_CHECK();
         }
     } else if (a.arith32) {
         return hipErrorInvalidValue;
     }
-    if (a.rig_meas) {
-        if (a.off32)
-            k_sample<T, uint32_t, true><<<nb, 256, 0, s>>>(a, dst);
-        else
-            k_sample<T, uint64_t, true><<<nb, 256, 0, s>>>(a, dst);
-    } else if (a.off32)
-        k_sample<T, uint32_t, false><<<nb, 256, 0, s>>>(a, dst);
-    else
-        k_sample<T, uint64_t, false><<<nb, 256, 0, s>>>(a, dst);
+    k_sample<T><<<nb, 256, 0, s>>>(SampleKernArgs<T>{a, dst});
     LAUNCH_CHECK();
 }
 
 hipError_t launch_outcount(hipStream_t s, const int32_t* nmerged, const int32_t* goff, const int32_t* keepscan,
-                           int Np, int32_t* outcnt) {
-    k_outcount<<<nblocks(Np, 256), 256, 0, s>>>(nmerged, goff, keepscan, Np, outcnt);
+                           int Np, int32_t* outcnt, const int32_t* mergeoff, int32_t* wave_parent) {
+    k_outcount<<<nblocks(Np, 4), 256, 0, s>>>(nmerged, goff, keepscan, Np, outcnt, mergeoff, wave_parent);
     LAUNCH_CHECK();
 }
 
@@ -2916,21 +3052,21 @@ hipError_t launch_table_resample(hipStream_t s, const int32_t* anc, const int32_
 }
 
 template <typename T>
-hipError_t launch_gather(hipStream_t s, Planes<T> src, Planes<T> dst, const int32_t* gblock, int64_t Ng, int S) {
+hipError_t launch_gather(hipStream_t s, Clouds<T> src, Clouds<T> dst, const int32_t* gblock, int64_t Ng, int S) {
     if (Ng <= 0) return hipSuccess;
-    k_gather<T><<<nblocks(Ng * S, 256), 256, 0, s>>>(src, dst, gblock, Ng, S);
+    k_gather<T><<<nblocks(Ng * 7 * S, 256), 256, 0, s>>>(src, dst, gblock, Ng, S);
     LAUNCH_CHECK();
 }
 
 template <typename T>
-hipError_t launch_extract(hipStream_t s, Planes<T> src, const int32_t* gblock, int64_t Ng, int S, double* out) {
+hipError_t launch_extract(hipStream_t s, Clouds<T> src, const int32_t* gblock, int64_t Ng, int S, double* out) {
     if (Ng <= 0) return hipSuccess;
     k_extract<T><<<nblocks(Ng * S, 256), 256, 0, s>>>(src, gblock, Ng, S, out);
     LAUNCH_CHECK();
 }
 
 template <typename T>
-hipError_t launch_inject(hipStream_t s, const double* in, int64_t Ng, int S, Planes<T> dst) {
+hipError_t launch_inject(hipStream_t s, const double* in, int64_t Ng, int S, Clouds<T> dst) {
     if (Ng <= 0) return hipSuccess;
     k_inject<T><<<nblocks(Ng * S, 256), 256, 0, s>>>(in, Ng, S, dst);
     LAUNCH_CHECK();
@@ -2947,26 +3083,26 @@ hipError_t launch_scan(hipStream_t s, const int32_t* in, int32_t* out, int64_t n
 }
 
 /* explicit instantiations */
-template hipError_t launch_materialize<float>(hipStream_t, Planes<float>, Planes<float>, const int32_t*,
+template hipError_t launch_materialize<float>(hipStream_t, Clouds<float>, Clouds<float>, const int32_t*,
                                               const int32_t*, const int32_t*, int64_t, int, LinearCVMotionModel3D,
                                               double, RigKeys, uint64_t, bool);
-template hipError_t launch_materialize<double>(hipStream_t, Planes<double>, Planes<double>, const int32_t*,
+template hipError_t launch_materialize<double>(hipStream_t, Clouds<double>, Clouds<double>, const int32_t*,
                                                const int32_t*, const int32_t*, int64_t, int, LinearCVMotionModel3D,
                                                double, RigKeys, uint64_t, bool);
-template hipError_t launch_fit<float>(hipStream_t, const FitArgs&, Planes<float>, Planes<float>);
-template hipError_t launch_fit<double>(hipStream_t, const FitArgs&, Planes<double>, Planes<double>);
-template hipError_t launch_fit_fix<float>(hipStream_t, const FitArgs&, Planes<float>, Planes<float>);
-template hipError_t launch_fit_fix<double>(hipStream_t, const FitArgs&, Planes<double>, Planes<double>);
-template hipError_t launch_nd_fill<float>(hipStream_t, const FitArgs&, Planes<float>, Planes<float>);
-template hipError_t launch_nd_fill<double>(hipStream_t, const FitArgs&, Planes<double>, Planes<double>);
-template hipError_t launch_sample<float>(hipStream_t, const SampleArgs&, Planes<float>);
-template hipError_t launch_sample<double>(hipStream_t, const SampleArgs&, Planes<double>);
-template hipError_t launch_gather<float>(hipStream_t, Planes<float>, Planes<float>, const int32_t*, int64_t, int);
-template hipError_t launch_gather<double>(hipStream_t, Planes<double>, Planes<double>, const int32_t*, int64_t,
+template hipError_t launch_fit<float>(hipStream_t, const FitArgs&, Clouds<float>, Clouds<float>);
+template hipError_t launch_fit<double>(hipStream_t, const FitArgs&, Clouds<double>, Clouds<double>);
+template hipError_t launch_fit_fix<float>(hipStream_t, const FitArgs&, Clouds<float>, Clouds<float>);
+template hipError_t launch_fit_fix<double>(hipStream_t, const FitArgs&, Clouds<double>, Clouds<double>);
+template hipError_t launch_nd_fill<float>(hipStream_t, const FitArgs&, Clouds<float>, Clouds<float>);
+template hipError_t launch_nd_fill<double>(hipStream_t, const FitArgs&, Clouds<double>, Clouds<double>);
+template hipError_t launch_sample<float>(hipStream_t, const SampleArgs&, Clouds<float>);
+template hipError_t launch_sample<double>(hipStream_t, const SampleArgs&, Clouds<double>);
+template hipError_t launch_gather<float>(hipStream_t, Clouds<float>, Clouds<float>, const int32_t*, int64_t, int);
+template hipError_t launch_gather<double>(hipStream_t, Clouds<double>, Clouds<double>, const int32_t*, int64_t,
                                           int);
-template hipError_t launch_extract<float>(hipStream_t, Planes<float>, const int32_t*, int64_t, int, double*);
-template hipError_t launch_extract<double>(hipStream_t, Planes<double>, const int32_t*, int64_t, int, double*);
-template hipError_t launch_inject<float>(hipStream_t, const double*, int64_t, int, Planes<float>);
-template hipError_t launch_inject<double>(hipStream_t, const double*, int64_t, int, Planes<double>);
+template hipError_t launch_extract<float>(hipStream_t, Clouds<float>, const int32_t*, int64_t, int, double*);
+template hipError_t launch_extract<double>(hipStream_t, Clouds<double>, const int32_t*, int64_t, int, double*);
+template hipError_t launch_inject<float>(hipStream_t, const double*, int64_t, int, Clouds<float>);
+template hipError_t launch_inject<double>(hipStream_t, const double*, int64_t, int, Clouds<double>);
 
 }  // namespace scphd
