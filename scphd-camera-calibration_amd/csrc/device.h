@@ -454,12 +454,39 @@ __device__ inline double rcp_nr(double x) {
     return __builtin_fma(r, e, r);
 }
 
+/* CameraPose::worldToCamera with the order of its sums given: y, x, z, or x,
+ * y, z for the position where `xy` (uniform over a wavefront) says so.  A
+ * cloud whose points the camera sees in a line has a covariance of rounding
+ * errors, which the samples drawn from it show: the same order, the same
+ * samples. */
+__device__ inline EuclideanPoint world_to_camera(const CameraPose& c, const EuclideanPoint& p, bool xy) {
+    const double dx = p.x - c.t[0], dy = p.y - c.t[1], dz = p.z - c.t[2];
+    double a[3];
+    if (xy) {
+#pragma unroll
+        for (int i = 0; i < 3; ++i) a[i] = __builtin_fma(c.R[3 + i], dy, c.R[i] * dx);
+        asm volatile("" : "+v"(a[0]), "+v"(a[1]), "+v"(a[2])); /* a branch, not both */
+    } else {
+#pragma unroll
+        for (int i = 0; i < 3; ++i) a[i] = __builtin_fma(c.R[i], dx, c.R[3 + i] * dy);
+        asm volatile("" : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]));
+    }
+    EuclideanPoint q;
+    q.x = __builtin_fma(c.R[6], dz, a[0]);
+    q.y = __builtin_fma(c.R[7], dz, a[1]);
+    q.z = __builtin_fma(c.R[8], dz, a[2]);
+    q.vx = __builtin_fma(c.R[6], p.vz, __builtin_fma(c.R[0], p.vx, c.R[3] * p.vy));
+    q.vy = __builtin_fma(c.R[7], p.vz, __builtin_fma(c.R[1], p.vx, c.R[4] * p.vy));
+    q.vz = __builtin_fma(c.R[8], p.vz, __builtin_fma(c.R[2], p.vx, c.R[5] * p.vy));
+    return q;
+}
+
 /* DisparityMeasurementModel::computeMeasurement of a world point seen by
  * camera c, with the three quotients fx/z, fy/z, 1/z^2 taken from one
  * reciprocal 1/z (within a few ulps of the divisions). */
 __device__ inline DisparityPoint disparity_fast(const DisparityMeasurementModel& m, const CameraPose& c,
-                                                const EuclideanPoint& pw) {
-    const EuclideanPoint p = c.worldToCamera(pw);
+                                                const EuclideanPoint& pw, bool xy = false) {
+    const EuclideanPoint p = world_to_camera(c, pw, xy);
     const double iz = rcp_nr(p.z);
     const double fz = m.fx() * iz, gz = m.fy() * iz, iz2 = iz * iz;
     DisparityPoint q;

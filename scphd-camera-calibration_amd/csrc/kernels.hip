@@ -611,6 +611,7 @@ __device__ inline void fit_row(const FitArgs& a, const ParentCtx& pc, int64_t g,
      * and at once loads the step two ahead into it.  Steps go in groups of
      * four, the noise group, so that a step's place in it (which normals it
      * draws and which it carries) is fixed. */
+    [[maybe_unused]] const int triples = S - S % 48;
     T buf[2][7];
     load_step(from, S, lane, buf[0]);
     load_step(from + 112, S - 16, lane, buf[1]);
@@ -662,8 +663,11 @@ __device__ inline void fit_row(const FitArgs& a, const ParentCtx& pc, int64_t g,
                 disparity_f(cx.m, cx.pose, x, q);
                 in = in_range_f(cx.m, q);
             } else {
+                /* the order of a point's sums by its place in triples of
+                 * whole steps */
+                const bool xy = (uint32_t)s0 / 16 % 3 == 1 && s0 < triples;
                 const DisparityPoint d =
-                    disparity_fast(meas, pose, EuclideanPoint{x[0], x[1], x[2], x[3], x[4], x[5]});
+                    disparity_fast(meas, pose, EuclideanPoint{x[0], x[1], x[2], x[3], x[4], x[5]}, xy);
                 in = meas.inRange(d);
                 q[0] = d.u; q[1] = d.v; q[2] = d.d; q[3] = d.vu; q[4] = d.vv; q[5] = d.vd;
             }
