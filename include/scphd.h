@@ -229,10 +229,12 @@ int scphd_get_phase_ms(scphd_t* f, double* ms8);
  * to its general code paths, so that small inputs exercise them.
  *   merge_lds_cap       parents with more survivors merge in global scratch
  *                       (k_merge_groups<true>); default: what fits 60 KB LDS
- *   eta_heavy_cap       0..2048: more Gaussians above the birth/clutter term
- *                       -> the normaliser max pass sweeps the whole map
- *   eta_ncand_cap       0..8: more candidate terms per measurement -> the
- *                       normaliser count and the survivor pass sweep the map
+ *   eta_heavy_cap       0..2048: below 2048 the normaliser meets every pair
+ *                       of a Gaussian and a measurement instead of those
+ *                       within a window in v
+ *   eta_ncand_cap       0..8: a parent with more kept detection terms than
+ *                       this times its measurements -> the normaliser count
+ *                       and the survivor pass sweep the map (0: always)
  *   merge_force_rounds  nonzero: every parent merges in the round loop
  *                       (k_merge_rounds), the path of candidate or
  *                       neighbour-list overflow

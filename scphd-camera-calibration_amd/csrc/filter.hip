@@ -246,9 +246,9 @@ struct scphd_filter {
     /* measurements, normalisers, survivors, merge */
     DBuf<double> du, dv, eta;
     int capM = 0;
-    DBuf<int32_t> nsurv, survoff, nmerged, mergeoff, outcnt, scantmp, sg, sm, dflag, mcnt, mncand, mcand;
+    DBuf<int32_t> nsurv, survoff, nmerged, mergeoff, outcnt, scantmp, sg, sm, dflag, mcnt, knum, kjm;
     DBuf<int32_t> ngroups, glead, gsta, gend, gmem;
-    DBuf<double> sw, smu, mw, mmu, mP, dneff;
+    DBuf<double> sw, smu, mw, mmu, mP, dneff, kw;
     DBuf<char> mscratch;
     /* mapped host memory the device writes read-back values into: int32
      * [0, 16) for k_readout and k_nan_count, an FP64 pair count at byte
@@ -270,6 +270,7 @@ struct scphd_filter {
     scphd_update_stats stats{};
     int64_t last_M = 0;
     int64_t kt_hint = 0; /* blocks the last update's posterior clouds took beyond the dropped terms' */
+    int max_map = 0; /* no parent's map is larger */
     bool has_outputs = false; /* the last update's per-parent outputs are held (scphd_compact releases them) */
     bool timing = false;
     hipEvent_t ev[10] = {};  /* 0..5 phase boundaries, 6..7 fit kernel, 8..9 sample kernel */
@@ -316,7 +317,7 @@ void for_each_buf(scphd_filter* f, Fn&& fn) {
     fn(f->gblock2); fn(f->gw2); fn(f->gpd); fn(f->gpd2); fn(f->fit); fn(f->pre); fn(f->lik); fn(f->keep);
     fn(f->keepscan); fn(f->ndlist); fn(f->holes); fn(f->redo); fn(f->ndfill); fn(f->du); fn(f->dv); fn(f->eta); fn(f->nsurv);
     fn(f->survoff); fn(f->nmerged); fn(f->mergeoff); fn(f->outcnt); fn(f->scantmp); fn(f->sg); fn(f->sm);
-    fn(f->dflag); fn(f->mcnt); fn(f->mncand); fn(f->mcand); fn(f->ngroups); fn(f->glead); fn(f->gsta);
+    fn(f->dflag); fn(f->mcnt); fn(f->knum); fn(f->kjm); fn(f->kw); fn(f->ngroups); fn(f->glead); fn(f->gsta);
     fn(f->gend); fn(f->gmem); fn(f->sw); fn(f->smu); fn(f->mw); fn(f->mmu); fn(f->mP); fn(f->dneff);
     fn(f->mscratch); fn(f->wparent); fn(f->wmerged);
 }
@@ -537,15 +538,22 @@ int update_t(scphd_filter* f, int M, int fixed) {
     ea.loglik = f->loglik.p;
     ea.nsurv = f->nsurv.p;
     HIPTRY(f->mcnt.ensure((int64_t)Np * std::max(M, 1)));
-    HIPTRY(f->mncand.ensure((int64_t)Np * std::max(M, 1)));
-    HIPTRY(f->mcand.ensure((int64_t)Np * std::max(M, 1) * ETA_NCAND));
+    /* room for the kept terms: ETA_NCAND a measurement, on average over a
+     * parent's measurements */
+    ea.kcap = (int64_t)(f->dbg_ncand >= 0 ? std::min(f->dbg_ncand, ETA_NCAND) : ETA_NCAND) * M;
+    ea.no_lists = ea.kcap == 0;
+    HIPTRY(f->knum.ensure(Np));
+    HIPTRY(f->kw.ensure(Np * std::max<int64_t>(ea.kcap, 1)));
+    HIPTRY(f->kjm.ensure(2 * Np * std::max<int64_t>(ea.kcap, 1)));
     ea.mcnt = f->mcnt.p;
-    ea.mncand = f->mncand.p;
-    ea.mcand = f->mcand.p;
+    ea.knum = f->knum.p;
+    ea.kw = f->kw.p;
+    ea.kjm = f->kjm.p;
     ea.lw_gate = P.min_weight > 0 ? std::log(P.min_weight) - 1e-3 : -INFINITY;
-    ea.heavy_cap = f->dbg_heavy >= 0 ? std::min(f->dbg_heavy, ETA_HEAVY) : ETA_HEAVY;
-    ea.ncand_cap = f->dbg_ncand >= 0 ? std::min(f->dbg_ncand, ETA_NCAND) : ETA_NCAND;
-    HIPTRY(launch_eta(s, ea));
+    ea.sweep = f->dbg_heavy >= 0 && f->dbg_heavy < ETA_HEAVY;
+    ea.img_height = f->models.meas.img_height();
+    ea.rig_meas = f->ensemble ? f->dmeas.p : nullptr;
+    HIPTRY(launch_eta(s, ea, f->max_map));
     HIPTRY(launch_scan(s, f->nsurv.p, f->survoff.p, Np, f->scantmp.p));
     HIPTRY(launch_readout(s, f->survoff.p, Np, 0, nullptr, nullptr, f->dmap));
     HIPTRY(hipStreamSynchronize(s));
@@ -647,6 +655,7 @@ int update_t(scphd_filter* f, int M, int fixed) {
     flush_retired(f); /* both streams have drained */
     const int64_t Nout = f->hmap[0];
     const int64_t Kt = f->hmap[3];
+    const int max_map = f->hmap[1];
     if (f->hmap[4] != 0) return fail(f, SCPHD_ERR_STATE, "survivor count mismatch between passes");
     const int64_t capx = f->hmap[2];
     f->stats.cap_exceeded = capx;
@@ -720,6 +729,7 @@ int update_t(scphd_filter* f, int M, int fixed) {
     f->hint_ok = true;
     f->cur = nxt;
     f->Ng = Nout;
+    f->max_map = max_map;
     f->n_update++;
 
     f->stats.n_meas = f->ensemble ? f->ens_meas : M;
@@ -1520,6 +1530,7 @@ int scphd_set_state(scphd_t* f, const double* states, const double* weights, con
     HIPTRY(hipStreamSynchronize(s));
     flush_retired(f);
     f->Ng = Ng;
+    f->max_map = *std::max_element(gcount, gcount + Np);
     f->n_predict = n_predict;
     f->n_update = n_update;
     f->n_resample = n_resample;
@@ -1713,8 +1724,8 @@ int scphd_compact(scphd_t* f) {
      * (each update sizes them again); the debug outputs of the last update
      * go with them */
     f->gen[1 - f->cur].release();
-    for (auto* b : {&f->fit, &f->pre, &f->lik, &f->eta, &f->sw, &f->smu, &f->mw, &f->mmu, &f->mP}) b->release();
-    for (auto* b : {&f->keep, &f->keepscan, &f->ndlist, &f->holes, &f->redo, &f->ndfill, &f->mcnt, &f->mncand, &f->mcand, &f->sg,
+    for (auto* b : {&f->fit, &f->pre, &f->lik, &f->eta, &f->sw, &f->smu, &f->mw, &f->mmu, &f->mP, &f->kw}) b->release();
+    for (auto* b : {&f->keep, &f->keepscan, &f->ndlist, &f->holes, &f->redo, &f->ndfill, &f->mcnt, &f->knum, &f->kjm, &f->sg,
                     &f->sm, &f->glead, &f->gsta, &f->gend, &f->gmem, &f->gparent2, &f->gblock2, &f->nsurv,
                     &f->survoff, &f->nmerged, &f->mergeoff, &f->outcnt, &f->ngroups, &f->wparent, &f->wmerged})
         b->release();
@@ -1776,8 +1787,9 @@ int scphd_reserve(scphd_t* f, int64_t n_gaussians, int32_t max_meas) {
     /* per (parent, measurement) and the measurement sets */
     HIPTRY(f->eta.ensure(Np * M));
     HIPTRY(f->mcnt.ensure(Np * M));
-    HIPTRY(f->mncand.ensure(Np * M));
-    HIPTRY(f->mcand.ensure(Np * M * ETA_NCAND));
+    HIPTRY(f->knum.ensure(Np));
+    HIPTRY(f->kw.ensure(Np * M * ETA_NCAND));
+    HIPTRY(f->kjm.ensure(2 * Np * M * ETA_NCAND));
     HIPTRY(f->du.ensure((int64_t)f->n_rigs * M));
     HIPTRY(f->dv.ensure((int64_t)f->n_rigs * M));
     HIPTRY(hipStreamSynchronize(f->stream));

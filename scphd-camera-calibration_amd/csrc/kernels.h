@@ -231,15 +231,24 @@ struct EtaArgs {
     double* loglik;    /* Np   */
     int32_t* nsurv;    /* Np   */
     int32_t* mcnt;     /* Np*M detection terms kept per (parent, measurement) */
-    int32_t* mncand;   /* Np*M candidates per (parent, measurement): terms that may be kept */
-    int32_t* mcand;    /* Np*M*ETA_NCAND their map indices (ascending), when at most ETA_NCAND */
+    /* the kept detection terms of a parent in pack order, at kcap p + i:
+     * weight, (map index, measurement); knum[p] of them, -1 when there are
+     * more than kcap or k_eta made no list */
+    int32_t* knum;
+    double* kw;
+    int32_t* kjm;
+    int64_t kcap;
     double lw_gate;    /* log(min_weight) - 1e-3: below it exp() < min_weight for certain */
-    int heavy_cap;     /* at most ETA_HEAVY: more Gaussians above bpc than this -> whole-map max pass */
-    int ncand_cap;     /* at most ETA_NCAND: more candidates than this -> whole-map sweeps */
+    int no_lists;      /* nonzero: no lists of the kept terms, whole-map sweeps (verification) */
+    double img_height; /* of the camera; in an ensemble rig_meas[r]'s (null for one rig) */
+    const DisparityMeasurementModel* rig_meas = nullptr;
+    int sweep = 0;     /* nonzero: every pair is evaluated, no windows (verification) */
+    int mask_stride = 0; /* set by launch_eta */
 };
-static constexpr int ETA_NCAND = 8;
-static constexpr int ETA_HEAVY = 2048; /* LDS list of the Gaussians that can exceed bpc */
-hipError_t launch_eta(hipStream_t s, const EtaArgs& a);
+static constexpr int ETA_NCAND = 8; /* kept detection terms a measurement that the lists have room for */
+static constexpr int ETA_HEAVY = 2048; /* the normal value of scphd_debug_set_limits' eta_heavy_cap */
+/* max_map: at least the largest parent's map size (any larger number serves) */
+hipError_t launch_eta(hipStream_t s, EtaArgs a, int max_map);
 
 struct SurvArgs {
     EtaArgs e;

@@ -1042,37 +1042,20 @@ __device__ inline Lik4 load_lik4(const double* lik, int64_t g) {
     return x;
 }
 
-__device__ inline double det_lw(const double* r, double zu, double zv);
-
-/* One record through the scalar path (its index the same in every lane). */
-__device__ inline double det_lw(lik_t* r, double zu, double zv) {
-    double v[LK_COUNT];
-#pragma unroll
-    for (int q = 0; q < LK_COUNT; ++q) v[q] = r[q];
-    return det_lw((const double*)v, zu, zv);
-}
-
-__device__ inline lik_t* lik_rec(const double* lik, int64_t g) { return (lik_t*)(lik + g * LK_COUNT); }
-
 /* log weight of the detection term of Gaussian record r and measurement
  * (zu, zv): log pd + log w - dist/2 - log 2 pi - log det / 2
  * (src/kernels.cu:527-539); log(0) when the updated covariance is not PD
- * (:597-598). */
+ * (:597-598).  The fused multiply-adds are written out, so that every place
+ * that evaluates a term gets the same bits. */
+static constexpr double LOG_2PI = 1.8378770664093453;
 __device__ inline double det_lw(const double* r, double zu, double zv) {
     const double i0 = zu - r[LK_MUU], i1 = zv - r[LK_MUV];
-    const double dist = i0 * i0 * r[LK_S0] + i0 * i1 * r[LK_S12] + i1 * i1 * r[LK_S3];
-    const double lw = r[LK_C] - 0.5 * dist - 1.8378770664093453 - r[LK_H];
+    /* one order of the three products in every kernel: a weight that is the
+     * same to the last bit sorts the same */
+    const double dist = fma(i1 * i1, r[LK_S3], fma(i0 * i0, r[LK_S0], i0 * i1 * r[LK_S12]));
+    const double lw = fma(-0.5, dist, r[LK_C]) - LOG_2PI - r[LK_H];
     return r[LK_OK] != 0.0 ? lw : SCPHD_LOG0;
 }
-
-/* Per parent: eta_{p,m} = log( sum_g exp(lw_{g,m}) + M w0 + kappa ) for
- * every measurement (normaliser reduce_by_key + log_sum_exp,
- * src/scphdcameracalibration.cu:1729-1768, exact per-parent segments), the
- * single-cluster log-likelihood sum_m eta + sum_g w_g (:1813-1849) and the
- * number of detection/birth terms whose normalised weight reaches
- * min_weight (updateKernel's prune flag, src/kernels.cu:608-659).
- * One workgroup per parent, one thread per measurement, the Gaussians'
- * likelihood records read by scalar loads. */
 
 /* e^x for -746 < x <= 0, the normaliser's terms (within 1 ulp of a
  * correctly rounded exp): x = k ln2 + r with |r| <= ln2/2 by Cody and
@@ -1100,16 +1083,79 @@ __device__ inline double exp_nonpos(double x) {
     return ldexp(p, (int)k);
 }
 
-__global__ __launch_bounds__(NT) void k_eta(EtaArgs a) {
+/* order-preserving map of a double to unsigned (for LDS atomic maxima) */
+__device__ inline unsigned long long max_key(double x) {
+    const unsigned long long b = (unsigned long long)__double_as_longlong(x);
+    return b >> 63 ? ~b : b | (1ull << 63);
+}
+__device__ inline double max_val(unsigned long long k) {
+    return __longlong_as_double((long long)(k >> 63 ? k & ~(1ull << 63) : ~k));
+}
+
+/* Per parent: eta_{p,m} = log( sum_g exp(lw_{g,m}) + M w0 + kappa ) for
+ * every measurement (normaliser reduce_by_key + log_sum_exp,
+ * src/scphdcameracalibration.cu:1729-1768, exact per-parent segments), the
+ * single-cluster log-likelihood sum_m eta + sum_g w_g (:1813-1849), and the
+ * detection terms whose normalised weight reaches min_weight, listed in pack
+ * order and counted with the birth terms that reach it (updateKernel's prune
+ * flag, src/kernels.cu:608-659).
+ *
+ * One workgroup per parent; 256 measurements a round.  A term matters to a
+ * measurement only within a few standard deviations of it: with
+ * l <= C - log 2 pi - H - dist/2 and dist >= dv^2 / S_vv (the marginal of
+ * the quadratic form), l > L needs dv^2 <= 2 (C - log 2 pi - H - L) S_vv.
+ * So the round's measurements are put in bins of v (a measurement's place is
+ * its rank by bin), and a Gaussian meets those of the bins its window covers:
+ *   1. l > bpc (L = bpc; no other term can move the maximum off bpc): few
+ *      Gaussians and few measurements each, a Gaussian a lane, an atomic
+ *      maximum per measurement;
+ *   2. l > max - 60 (L = bpc - 60; all terms below exp(-60) of the largest
+ *      together are 1e-7 of an ulp of eta): about 30 measurements a
+ *      Gaussian, but all of them for a few, so a wavefront takes a Gaussian
+ *      at a time against its measurements in blocks of 64, held in registers,
+ *      and collects a word of the measurements' masks, 32 Gaussians, in
+ *      registers too;
+ *   3. the masks' terms (about 20 a measurement, up to 130) are listed by
+ *      measurement and then map index, evaluated a lane each, and summed per
+ *      measurement in that order, ascending in g: the oracle's.  Terms that
+ *      can no longer be kept leave the mask;
+ *   4. the rest are listed, evaluated against eta, and those kept written
+ *      in list order, which is the pack order.
+ * Gaussians go in chunks of the mask's 2048 bits in 2 and 3; a map of more
+ * than one chunk makes no list (4), and k_survivors sweeps it.
+ *
+ * Bound: latency (LDS and the records' gathers), which is why the lists
+ * spread the uneven terms over all lanes.  Ten frames of 4096 parents, 200
+ * landmarks: 18.0 ms when every pair was evaluated twice and measurements
+ * with more than eight candidate terms (one in seven) swept the map again. */
+static constexpr int ETA_BINS = 128, ETA_CHUNK = 2048, ETA_LIST = 1024;
+static constexpr double ETA_DROP = 60.0;
+
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_eta(EtaArgs a) {
+    constexpr int REC = 6; /* of a record, what step 2 needs */
     __shared__ double red[16];
     __shared__ int sh[8];
-    __shared__ int s_heavy[ETA_HEAVY];
+    __shared__ double s_zu[NT], s_zv[NT];    /* the round's measurements by place */
+    __shared__ uint16_t s_m[NT];             /* the measurement at a place */
+    __shared__ unsigned long long s_max[NT]; /* per measurement: its maximum's key; then eta's bits */
+    __shared__ unsigned long long s_any[NT]; /* per place: its mask's non-zero words */
+    __shared__ int s_cnt[NT];                /* per measurement: terms kept */
+    __shared__ int s_off[ETA_BINS + 1], s_cur[ETA_BINS];
+    __shared__ union {
+        double rec[NT / 64][32 * REC];       /* per wavefront: the records of a word of Gaussians */
+        struct {
+            double e[ETA_LIST];              /* a list's terms: exp(l - max) */
+            uint32_t pair[ETA_LIST];         /* place << 16 | map index in the chunk */
+        } l;
+    } u;
+    extern __shared__ uint32_t s_mask[];     /* per place, a.mask_stride words */
     const int p = blockIdx.x;
-    const int t = threadIdx.x;
+    const int t = threadIdx.x, lane = t & 63;
     const int64_t g0 = a.goff[p];
     const int G = a.goff[p + 1] - a.goff[p];
+    const bool lists = !a.no_lists && G <= ETA_CHUNK;
     double eta_sum = 0.0;
-    int cnt = 0;
+    int cnt = 0, kept = 0;
     /* this parent's measurement set: its rig's in an ensemble */
     const int rig = a.moff ? a.prig[p] : 0;
     const int M = a.moff ? a.moff[rig + 1] - a.moff[rig] : a.M;
@@ -1118,125 +1164,277 @@ __global__ __launch_bounds__(NT) void k_eta(EtaArgs a) {
     const double logw0 = a.births[rig].logw0;
     const bool birth_ok = a.births[rig].pd_ok != 0;
     const int rounds = (M + NT - 1) / NT;
-    /* Only a Gaussian with l > bpc can move the maximum off bpc, and
-     * l <= C - log 2 pi - H (the value at dist = 0; the computed quadratic
-     * form is never below -1e-9 of its scale), so the max pass visits only
-     * those whose bound exceeds bpc (with a 1e-6 relative margin), in
-     * ascending order: the same first maximum.  More than heavy_cap (at most
-     * ETA_HEAVY) of them: the whole map. */
-    int nheavy = 0;
-    for (int j0 = 0; j0 < G; j0 += NT) {
-        const int j = j0 + t;
-        bool h = false;
-        if (j < G) {
-            const double* rec = a.lik + (g0 + j) * LK_COUNT;
-            const double ub = rec[LK_C] - 1.8378770664093453 - rec[LK_H];
-            h = rec[LK_OK] != 0.0 && ub + 1e-6 * (1.0 + fabs(ub)) > bpc;
+    const double bin_scale = ETA_BINS / fabs(a.rig_meas ? a.rig_meas[rig].img_height() : a.img_height);
+    /* candidates: terms with l - max above the gate (less 1e-6), the only
+     * ones that can pass it against eta >= max */
+    const double cgate = a.lw_gate - 1e-6;
+    const double drop = fmax(ETA_DROP, -cgate); /* no candidate is dropped */
+    /* monotone in v, a NaN's the first */
+    auto bin = [&](double v) { return (int)fmin(fmax(v * bin_scale, 0.0), (double)(ETA_BINS - 1)); };
+    /* the places [q0, q1) of the measurements that Gaussian record r may give
+     * l > L; the margins cover the rounding of l and of the window */
+    auto window = [&](const double* r, double L, int& q0, int& q1) {
+        q0 = q1 = 0;
+        if (r[LK_OK] == 0.0) return;
+        const double ub = r[LK_C] - LOG_2PI - r[LK_H], over = ub - L + 1e-6 * (1.0 + fabs(ub));
+        if (!(over > 0.0)) return;
+        const double c = 0.5 * r[LK_S12], det = r[LK_S0] * r[LK_S3] - c * c;
+        const double hw = sqrt(2.000002 * over * (r[LK_S0] / det)) * 1.000001 + 1e-12 * fabs(r[LK_MUV]);
+        if (a.sweep || !(det > 1e-9 * r[LK_S0] * r[LK_S3]) || !(hw < 1e300) || r[LK_MUV] != r[LK_MUV]) {
+            q1 = s_off[ETA_BINS]; /* near singular: every measurement */
+        } else {
+            q0 = s_off[bin(r[LK_MUV] - hw)];
+            q1 = s_off[bin(r[LK_MUV] + hw) + 1];
         }
-        int tot;
-        const int pos = nheavy + block_exscan(h ? 1 : 0, sh, &tot);
-        if (h && pos < ETA_HEAVY) s_heavy[pos] = j;
-        nheavy += tot;
-    }
-    __syncthreads();
-    const bool listed = nheavy <= a.heavy_cap;
+    };
+    auto load_rec = [&](int j, double* r) {
+        const double* rec = a.lik + (g0 + j) * LK_COUNT;
+#pragma unroll
+        for (int q = 0; q < LK_COUNT; ++q) r[q] = rec[q];
+    };
     for (int r = 0; r < rounds; ++r) {
         const int m = r * NT + t;
         const bool valid = m < M;
         const double zu = valid ? a.zu[zb + m] : 0.0, zv = valid ? a.zv[zb + m] : 0.0;
+        const int64_t pm = (int64_t)p * a.M + m;
+        /* the round's measurements by bin */
+        __syncthreads();
+        if (t < ETA_BINS) s_cur[t] = 0;
+        s_max[t] = max_key(bpc);
+        s_cnt[t] = 0;
+        __syncthreads();
+        const int mb = bin(zv);
+        int place = 0;
+        if (valid) atomicAdd(&s_cur[mb], 1);
+        __syncthreads();
+        if (t < 64) { /* exclusive offsets, two bins a lane */
+            const int c0 = s_cur[2 * t], c1 = s_cur[2 * t + 1];
+            int x = c0 + c1;
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                const int y = __shfl_up(x, o, 64);
+                if (t >= o) x += y;
+            }
+            s_off[2 * t] = s_cur[2 * t] = x - c0 - c1;
+            s_off[2 * t + 1] = s_cur[2 * t + 1] = x - c1;
+            if (t == 63) s_off[ETA_BINS] = x;
+        }
+        __syncthreads();
+        if (valid) {
+            place = atomicAdd(&s_cur[mb], 1);
+            s_zu[place] = zu;
+            s_zv[place] = zv;
+            s_m[place] = (uint16_t)t;
+        }
+        __syncthreads();
+        /* 1. maxima */
+        for (int j = t; j < G; j += NT) {
+            double rec[LK_COUNT];
+            load_rec(j, rec);
+            int q, q1;
+            for (window(rec, bpc, q, q1); q < q1; ++q) {
+                const double l = det_lw(rec, s_zu[q], s_zv[q]);
+                if (l > bpc) atomicMax(&s_max[s_m[q]], max_key(l));
+            }
+        }
+        __syncthreads();
         /* eta = mx + log1p(sum of the other terms' exp(l - mx)), mx the
          * first maximum of (bpc, l_0, ...), terms summed g ascending then
          * bpc: the normaliser definition the oracle uses bit for bit */
-        double mx = bpc;
-        int am = -1;
+        const double mx = max_val(s_max[t]);
+        bool met = !(mx > bpc); /* the maximum's own term (1, not summed) */
         double T = 0.0;
-        int mcnt = 0;
-        /* candidates: terms with l - mx above the gate (less 1e-6), the only
-         * ones that can pass it against eta >= mx; the first ETA_NCAND kept */
-        int nc = 0, cc[ETA_NCAND];
-#pragma unroll
-        for (int q = 0; q < ETA_NCAND; ++q) cc[q] = 0;
-        const double cgate = a.lw_gate - 1e-6;
-        if (valid) {
-            if (listed) {
-                for (int q = 0; q < nheavy; ++q) {
-                    const int j = __builtin_amdgcn_readfirstlane(s_heavy[q]);
-                    const double l = det_lw(lik_rec(a.lik, g0 + j), zu, zv);
-                    if (l > mx) {
-                        mx = l;
-                        am = j;
-                    }
+        const int nq = s_off[ETA_BINS];
+        /* the terms in this thread's row of the masks from (words, bits) on,
+         * ascending: fills the list's places up to ETA_LIST from `pos` on */
+        unsigned long long words_left = 0;
+        uint32_t bits_left = 0;
+        int word = 0;
+        auto row_begin = [&]() { /* and their number */
+            words_left = valid ? s_any[place] : 0;
+            bits_left = 0;
+            int n = 0;
+            for (unsigned long long w = words_left; w; w &= w - 1)
+                n += __popc(s_mask[place * a.mask_stride + __builtin_ctzll(w)]);
+            return n;
+        };
+        auto row_list = [&](int& pos, int end) {
+            while (pos < end) {
+                if (!bits_left) {
+                    if (!words_left) return;
+                    word = __builtin_ctzll(words_left);
+                    words_left &= words_left - 1;
+                    bits_left = s_mask[place * a.mask_stride + word];
+                    continue;
                 }
-            } else {
-                for (int j0 = 0; j0 < G; j0 += 4) {
-                    const Lik4 R = load_lik4(a.lik, g0 + j0);
+                u.l.pair[pos & (ETA_LIST - 1)] =
+                    (uint32_t)place << 16 | (uint32_t)(32 * word + __builtin_ctz(bits_left));
+                bits_left &= bits_left - 1;
+                ++pos;
+            }
+        };
+        for (int c0 = 0; c0 < G; c0 += ETA_CHUNK) {
+            const int cn = min(ETA_CHUNK, G - c0), words = (cn + 31) / 32;
+            s_any[t] = 0;
+            /* 2. block k: the measurements at places 64 k + lane; a pair hits
+             * when 2 ub - dist > lim (never at a place without one) */
+            double bu[4], bv[4], lim[4];
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const double l = det_lw(R.v[q], zu, zv);
-                        if (j0 + q < G && l > mx) {
-                            mx = l;
-                            am = j0 + q;
+            for (int k = 0; k < 4; ++k) {
+                const int q = 64 * k + lane;
+                bu[k] = bv[k] = 0.0;
+                lim[k] = INFINITY;
+                if (q < nq) {
+                    bu[k] = s_zu[q];
+                    bv[k] = s_zv[q];
+                    lim[k] = 2.0 * (max_val(s_max[s_m[q]]) - drop);
+                }
+            }
+            __syncthreads();
+            for (int w = __builtin_amdgcn_readfirstlane(t >> 6); w < words; w += NT / 64) {
+                const int jw = c0 + 32 * w, n = min(32, c0 + cn - jw);
+                double* const wr = u.rec[t >> 6];
+                /* the word's windows, a Gaussian a lane: blocks met */
+                int blocks = 0;
+                if (lane < n) {
+                    double rec[LK_COUNT];
+                    load_rec(jw + lane, rec);
+                    int q0, q1;
+                    window(rec, bpc - drop, q0, q1);
+                    if (q0 < q1) blocks = (2 << ((q1 - 1) >> 6)) - (1 << (q0 >> 6));
+                    const double ub = rec[LK_C] - LOG_2PI - rec[LK_H];
+                    wr[lane * REC] = rec[LK_MUU];
+                    wr[lane * REC + 1] = rec[LK_MUV];
+                    wr[lane * REC + 2] = rec[LK_S0];
+                    wr[lane * REC + 3] = rec[LK_S12];
+                    wr[lane * REC + 4] = rec[LK_S3];
+                    wr[lane * REC + 5] = 2.0 * ub + 2e-6 * (1.0 + fabs(ub));
+                }
+                wave_lds_fence();
+                uint32_t bits[4] = {0, 0, 0, 0};
+#pragma unroll 4
+                for (int b = 0; b < n; ++b) {
+                    const int met_blocks = __builtin_amdgcn_readlane(blocks, b);
+                    double rec[REC];
+#pragma unroll
+                    for (int q = 0; q < REC; ++q) rec[q] = wr[b * REC + q];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k)
+                        if (met_blocks >> k & 1) {
+                            const double i0 = bu[k] - rec[0], i1 = bv[k] - rec[1];
+                            const double dist = fma(i1 * i1, rec[4], fma(i0 * i1, rec[3], i0 * i0 * rec[2]));
+                            if (rec[5] - dist > lim[k]) bits[k] |= 1u << b;
                         }
+                }
+                wave_lds_fence();
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const int q = 64 * k + lane;
+                    if (q < nq) {
+                        s_mask[q * a.mask_stride + w] = bits[k];
+                        if (bits[k]) atomicOr(&s_any[q], 1ull << w);
                     }
                 }
             }
-            /* terms that cannot change T are skipped, which changes no bit:
-             * exp(x) is +0 for x <= -746, and for T in [2^(e-1), 2^e) a term
-             * below 2^(e-55), a quarter ulp, leaves T + exp(x) == T */
-            double thr = -746.0;
+            __syncthreads();
+            /* 3. the terms' values, and their sum */
+            int total, n = row_begin();
+            const int first = block_exscan(n, sh, &total);
+            int pos = first;
+            for (int l0 = 0; l0 < total; l0 += ETA_LIST) {
+                row_list(pos, l0 + ETA_LIST);
+                __syncthreads();
+                const int ln = min(ETA_LIST, total - l0);
+                for (int q = t; q < ln; q += NT) {
+                    const uint32_t pr = u.l.pair[q];
+                    const int pl = (int)(pr >> 16), j = (int)(pr & 0xFFFFu);
+                    double rec[LK_COUNT];
+                    load_rec(c0 + j, rec);
+                    const double x = det_lw(rec, s_zu[pl], s_zv[pl]) - max_val(s_max[s_m[pl]]);
+                    u.l.e[q] = x > -746.0 ? exp_nonpos(x) : 0.0;
+                    if (!(x > cgate)) atomicAnd(&s_mask[pl * a.mask_stride + (j >> 5)], ~(1u << (j & 31)));
+                }
+                __syncthreads();
+                const int q1 = min(first + n - l0, ln);
+                for (int q = max(first - l0, 0); q < q1; ++q) {
+                    const double e = u.l.e[q];
+                    if (!met && e == 1.0)
+                        met = true;
+                    else
+                        T += e;
+                }
+                __syncthreads();
+            }
+        }
+        if (mx > bpc) T += exp(bpc - mx);
+        const double eta = mx + log1p(T);
+        s_max[t] = (unsigned long long)__double_as_longlong(eta);
+        if (valid) {
+            a.eta[pm] = eta;
+            eta_sum += eta;
+            const double w = exp(logw0 - eta);
+            cnt += (w >= a.min_weight && birth_ok) ? 1 : 0;
+        }
+        /* 4. the kept terms */
+        if (lists && G > 0) {
+            int total, n = row_begin();
+            int pos = block_exscan(n, sh, &total);
+            for (int l0 = 0; l0 < total; l0 += ETA_LIST) {
+                row_list(pos, l0 + ETA_LIST);
+                __syncthreads();
+                constexpr int E = ETA_LIST / NT; /* consecutive terms of a thread */
+                double w[E];
+                int mine = 0;
+#pragma unroll
+                for (int i = 0; i < E; ++i) {
+                    const int q = E * t + i;
+                    w[i] = -1.0; /* not kept */
+                    if (l0 + q >= total) continue;
+                    const uint32_t pr = u.l.pair[q];
+                    const int pl = (int)(pr >> 16), sl = s_m[pl];
+                    double rec[LK_COUNT];
+                    load_rec((int)(pr & 0xFFFFu), rec);
+                    const double x = det_lw(rec, s_zu[pl], s_zv[pl]) - __longlong_as_double((long long)s_max[sl]);
+                    if (!(x > a.lw_gate)) continue;
+                    const double wx = exp(x);
+                    if (!(wx >= a.min_weight)) continue;
+                    w[i] = wx;
+                    ++mine;
+                    atomicAdd(&s_cnt[sl], 1);
+                }
+                int k, kn;
+                k = kept + block_exscan(mine, sh, &kn);
+#pragma unroll
+                for (int i = 0; i < E; ++i)
+                    if (w[i] >= 0.0) {
+                        if (k < a.kcap) {
+                            const uint32_t pr = u.l.pair[E * t + i];
+                            a.kw[p * a.kcap + k] = w[i];
+                            *(int2*)(a.kjm + 2 * (p * a.kcap + k)) =
+                                int2{(int)(pr & 0xFFFFu), r * NT + s_m[pr >> 16]};
+                        }
+                        ++k;
+                    }
+                kept += kn;
+                __syncthreads();
+            }
+            __syncthreads();
+            if (valid) {
+                a.mcnt[pm] = s_cnt[t];
+                cnt += s_cnt[t];
+            }
+        } else if (valid) { /* no list: sweep the map */
+            int mcnt = 0;
             for (int j0 = 0; j0 < G; j0 += 4) {
                 const Lik4 R = load_lik4(a.lik, g0 + j0);
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
-                    const double x = det_lw(R.v[q], zu, zv) - mx;
-                    if (j0 + q < G && j0 + q != am && x > thr) {
-                        T += exp_nonpos(x);
-                        /* the bound holds only once T > 0: a term that
-                         * underflowed to +0 leaves the threshold at -746 */
-                        thr = T > 0.0 ? fmax(-746.0, (double)(__builtin_amdgcn_frexp_exp(T) - 55) * 0.6931471805599453)
-                                      : -746.0;
-                    }
-                    if (j0 + q < G && x > cgate && R.v[q][LK_OK] != 0.0) {
-                        const int j = j0 + q;
-#pragma unroll
-                        for (int e = 0; e < ETA_NCAND; ++e) cc[e] = nc == e ? j : cc[e];
-                        ++nc;
-                    }
+                    const double x = det_lw(R.v[q], zu, zv) - eta;
+                    if (j0 + q < G && x > a.lw_gate && R.v[q][LK_OK] != 0.0) mcnt += exp(x) >= a.min_weight ? 1 : 0;
                 }
             }
-        }
-        if (am >= 0) T += exp(bpc - mx);
-        const double eta = mx + log1p(T);
-        if (valid) {
-            const int64_t pm = (int64_t)p * a.M + m;
-            a.eta[pm] = eta;
-            eta_sum += eta;
-            if (nc <= a.ncand_cap) { /* the candidates alone */
-#pragma unroll
-                for (int k = 0; k < ETA_NCAND; ++k) {
-                    if (k >= nc) break;
-                    const int j = cc[k];
-                    const double* rec = a.lik + (g0 + j) * LK_COUNT;
-                    const double x = det_lw(rec, zu, zv) - eta;
-                    if (x > a.lw_gate && rec[LK_OK] != 0.0) mcnt += exp(x) >= a.min_weight ? 1 : 0;
-                    a.mcand[pm * ETA_NCAND + k] = j;
-                }
-            } else {
-                for (int j0 = 0; j0 < G; j0 += 4) {
-                    const Lik4 R = load_lik4(a.lik, g0 + j0);
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const double x = det_lw(R.v[q], zu, zv) - eta;
-                        if (j0 + q < G && x > a.lw_gate && R.v[q][LK_OK] != 0.0)
-                            mcnt += exp(x) >= a.min_weight ? 1 : 0;
-                    }
-                }
-            }
-            a.mncand[pm] = nc;
             a.mcnt[pm] = mcnt;
             cnt += mcnt;
-            const double w = exp(logw0 - eta);
-            cnt += (w >= a.min_weight && birth_ok) ? 1 : 0;
         }
     }
     double swg = 0.0;
@@ -1247,13 +1445,19 @@ __global__ __launch_bounds__(NT) void k_eta(EtaArgs a) {
     if (t == 0) {
         a.loglik[p] = se + sg;
         a.nsurv[p] = (int32_t)sc;
+        a.knum[p] = lists && kept <= a.kcap ? kept : -1;
     }
 }
 
 /* Writes the surviving detection terms (Kalman-updated mean, weight
  * exp(lw - eta)) and birth terms of every parent, compacted in the
  * reference's pack order (updateKernel, src/kernels.cu:608-659: detection
- * terms measurement-major, then births). */
+ * terms measurement-major, then births).  The detection terms come from
+ * k_eta's list, one a thread, so that the gathers of their records are in
+ * flight together and the survivors are written as one stretch (11.9 ms over
+ * ten frames of 4096 parents, 200 landmarks, when a thread found and wrote
+ * its measurement's terms one after the other); a parent without a list has
+ * its map swept. */
 __global__ __launch_bounds__(NT) void k_survivors(SurvArgs a) {
     __shared__ int sh[8];
     const EtaArgs& e = a.e;
@@ -1269,52 +1473,49 @@ __global__ __launch_bounds__(NT) void k_survivors(SurvArgs a) {
     const int M = e.moff ? e.moff[rig + 1] - e.moff[rig] : e.M;
     const int64_t zb = e.moff ? e.moff[rig] : 0;
     const int rounds = (M + NT - 1) / NT;
-    for (int r = 0; r < rounds; ++r) {
-        const int m = r * NT + t;
-        const bool valid = m < M;
-        const double zu = valid ? e.zu[zb + m] : 0.0, zv = valid ? e.zv[zb + m] : 0.0;
-        const double eta = valid ? e.eta[(int64_t)p * e.M + m] : 0.0;
-        const int cnt = valid ? e.mcnt[(int64_t)p * e.M + m] : 0; /* detection terms kept, from k_eta */
-        int tot;
-        int o = run + block_exscan(cnt, sh, &tot);
-        if (valid && cnt > 0) {
-            const int64_t pm = (int64_t)p * e.M + m;
-            /* detection term of map entry j: kept when its normalised weight
-             * reaches min_weight (the gate first: exp(x) < min_weight below it) */
-            auto term = [&](int j, const double* rec) {
-                const double x = det_lw(rec, zu, zv) - eta;
-                if (!(x > e.lw_gate && rec[LK_OK] != 0.0)) return;
-                const double w = exp(x);
-                if (w < e.min_weight) return;
-                if (o < cap) {
-                    const int64_t gi = g0 + j;
-                    const int64_t so = base + o;
-                    const double i0 = zu - rec[LK_MUU], i1 = zv - rec[LK_MUV];
-                    a.sw[so] = w;
-                    a.sg[so] = (int32_t)gi;
-                    a.sm[so] = m;
-                    const double* mk = e.pre + PP_MK * e.Ng + gi * PP_MK_LEN;
+    /* survivor i: map entry j and measurement m (at zu, zv) with weight w */
+    auto put = [&](int i, int j, int m, double zu, double zv, double w) {
+        if (i >= cap) return;
+        const int64_t so = base + i, gi = g0 + j;
+        const double* mk = e.pre + PP_MK * e.Ng + gi * PP_MK_LEN;
+        const double i0 = zu - mk[0], i1 = zv - mk[1];
+        a.sw[so] = w;
+        a.sg[so] = (int32_t)gi;
+        a.sm[so] = m;
 #pragma unroll
-                    for (int c = 0; c < 6; ++c) a.smu[(so) * 6 + c] = mk[c] + i0 * mk[6 + c] + i1 * mk[12 + c];
-                }
-                ++o;
-            };
-            const int nc = e.mncand[pm];
-            if (nc <= e.ncand_cap) { /* the candidates k_eta listed, ascending */
-                for (int k = 0; k < nc; ++k) {
-                    const int j = e.mcand[pm * ETA_NCAND + k];
-                    term(j, e.lik + (g0 + j) * LK_COUNT);
-                }
-            } else {
+        for (int c = 0; c < 6; ++c) a.smu[so * 6 + c] = mk[c] + i0 * mk[6 + c] + i1 * mk[12 + c];
+    };
+    const int kn = e.knum[p];
+    if (kn >= 0) {
+        for (int i = t; i < kn; i += NT) {
+            const int2 jm = *(const int2*)(e.kjm + 2 * (p * e.kcap + i));
+            put(i, jm.x, jm.y, e.zu[zb + jm.y], e.zv[zb + jm.y], e.kw[p * e.kcap + i]);
+        }
+        run = kn;
+    } else {
+        for (int r = 0; r < rounds; ++r) {
+            const int m = r * NT + t;
+            const bool valid = m < M;
+            const double zu = valid ? e.zu[zb + m] : 0.0, zv = valid ? e.zv[zb + m] : 0.0;
+            const double eta = valid ? e.eta[(int64_t)p * e.M + m] : 0.0;
+            const int cnt = valid ? e.mcnt[(int64_t)p * e.M + m] : 0; /* detection terms kept, from k_eta */
+            int tot;
+            int o = run + block_exscan(cnt, sh, &tot);
+            if (valid && cnt > 0)
                 for (int j0 = 0; j0 < G; j0 += 4) {
                     const Lik4 R = load_lik4(e.lik, g0 + j0);
 #pragma unroll
-                    for (int q = 0; q < 4; ++q)
-                        if (j0 + q < G) term(j0 + q, R.v[q]);
+                    for (int q = 0; q < 4; ++q) {
+                        /* kept when its normalised weight reaches min_weight
+                         * (the gate first: exp(x) < min_weight below it) */
+                        const double x = det_lw(R.v[q], zu, zv) - eta;
+                        if (j0 + q >= G || !(x > e.lw_gate && R.v[q][LK_OK] != 0.0)) continue;
+                        const double w = exp(x);
+                        if (w >= e.min_weight) put(o++, j0 + q, m, zu, zv, w);
+                    }
                 }
-            }
+            run += tot;
         }
-        run += tot;
     }
     for (int r = 0; r < rounds; ++r) {
         const int m = r * NT + t;
@@ -2840,8 +3041,10 @@ hipError_t launch_precompute(hipStream_t s, const double* fit, const double* gw,
     LAUNCH_CHECK();
 }
 
-hipError_t launch_eta(hipStream_t s, const EtaArgs& a) {
-    k_eta<<<a.Np, NT, 0, s>>>(a);
+hipError_t launch_eta(hipStream_t s, EtaArgs a, int max_map) {
+    /* an odd stride: a word of all places lies in all banks */
+    a.mask_stride = ((std::min(max_map, ETA_CHUNK) + 31) / 32) | 1;
+    k_eta<<<a.Np, NT, (size_t)std::min(std::max(a.M, 1), NT) * a.mask_stride * sizeof(uint32_t), s>>>(a);
     LAUNCH_CHECK();
 }
 
