@@ -228,7 +228,8 @@ int scphd_get_phase_ms(scphd_t* f, double* ms8);
 /* Verification limits: lower the capacities at which the update falls back
  * to its general code paths, so that small inputs exercise them.
  *   merge_lds_cap       parents with more survivors merge in global scratch
- *                       (k_merge_groups<true>); default: what fits 60 KB LDS
+ *                       (k_merge_groups<true>, k_merge_rounds<true>);
+ *                       default: what fits the LDS
  *   eta_heavy_cap       0..2048: below 2048 the normaliser meets every pair
  *                       of a Gaussian and a measurement instead of those
  *                       within a window in v
@@ -236,8 +237,8 @@ int scphd_get_phase_ms(scphd_t* f, double* ms8);
  *                       this times its measurements -> the normaliser count
  *                       and the survivor pass sweep the map (0: always)
  *   merge_force_rounds  nonzero: every parent merges in the round loop
- *                       (k_merge_rounds), the path of candidate or
- *                       neighbour-list overflow
+ *                       (k_merge_rounds), the path of neighbour-list
+ *                       overflow
  *   merge_all_pairs     nonzero: merge candidates come from every pair of
  *                       survivors, the path of survivors whose (u, v)
  *                       covariance is ill-conditioned, instead of windows

@@ -275,7 +275,7 @@ struct scphd_filter {
     bool timing = false;
     hipEvent_t ev[10] = {};  /* 0..5 phase boundaries, 6..7 fit kernel, 8..9 sample kernel */
     double phase_ms[8] = {};
-    int lds_cap = 0;
+    int rounds_cap = 0;
     /* the open profiler range of the update's current phase (0: none) */
     roctx_range_id_t phase_range = 0;
     /* verification limits (scphd_debug_set_limits); -1 = the normal limit */
@@ -367,11 +367,11 @@ void set_models(scphd_filter* f) {
     f->models.feat = LinearCVMotionModel3D(p.feat_accel_std[0], p.feat_accel_std[1], p.feat_accel_std[2]);
     f->birth = birth_of(p);
     f->key = NoiseKey::from_seed(p.seed);
-    /* largest survivor count whose merge workspace fits 60 KB of LDS */
+    /* largest survivor count whose round-loop workspace fits 60 KB of LDS */
     int cap = 64;
     while (merge_lds_bytes(cap * 2) <= 61440) cap *= 2;
     while (merge_lds_bytes(cap + 64) <= 61440) cap += 64;
-    f->lds_cap = cap;
+    f->rounds_cap = cap;
 }
 
 /* Apply a deferred sample prediction into fresh, unshared blocks. */
@@ -597,11 +597,13 @@ int update_t(scphd_filter* f, int M, int fixed) {
     ma.births = f->dbirths.p;
     ma.min_separation = P.min_separation;
     ma.Np = Np;
-    const int lds_cap = f->dbg_lds_cap >= 0 ? std::min(f->dbg_lds_cap, f->lds_cap) : f->lds_cap;
-    ma.lds_cap = lds_cap;
+    ma.lds_cap = f->dbg_lds_cap >= 0 ? f->dbg_lds_cap : INT32_MAX;
+    ma.rounds_cap = std::min(ma.lds_cap, f->rounds_cap);
     ma.force_rounds = f->dbg_rounds;
     ma.all_pairs = f->dbg_all_pairs;
-    ma.scratch = nullptr;
+    ma.img_width = f->models.meas.img_width();
+    ma.rig_meas = f->ensemble ? f->dmeas.p : nullptr;
+    ma.prig = f->ensemble ? f->dprig.p : nullptr;
     ma.mw = f->mw.p;
     ma.mmu = f->mmu.p;
     ma.mP = f->mP.p;
@@ -617,21 +619,9 @@ int update_t(scphd_filter* f, int M, int fixed) {
     ma.gend = f->gend.p;
     ma.gmem = f->gmem.p;
     ma.Stot = Stot;
-    ma.big_lds_up = 0;
-    ma.big_lds_bytes = 0;
-    if (maxU > lds_cap) {
-        HIPTRY(f->mscratch.ensure(merge_scratch_bytes(Stot, Np)));
-        ma.scratch = f->mscratch.p;
-        /* the big parents' sort keys in LDS: 12 B per slot, at most 48 KB */
-        int up = 1;
-        while (up < maxU) up <<= 1;
-        ma.big_lds_up = up <= 4096 ? up : 0;
-        /* the sort keys (12 B per slot of next_pow2(U)), then, in the same
-         * LDS, 28 B per survivor for the walk's counts, offsets, labels,
-         * buckets and group records */
-        ma.big_lds_bytes = std::max(12 * ma.big_lds_up, ma.big_lds_up ? std::min(28 * maxU + 16, 65536) : 0);
-    }
-    HIPTRY(launch_merge(s, ma, merge_lds_bytes(std::max(1, std::min(maxU, lds_cap)))));
+    HIPTRY(f->mscratch.ensure(merge_scratch_bytes(Stot, Np, &ma, maxU > ma.rounds_cap)));
+    ma.scratch = f->mscratch.p;
+    HIPTRY(launch_merge(s, ma, maxU));
     if (!fixed)
         HIPTRY(launch_parent_weights(s, f->pw.p, f->loglik.p, Np, f->ensemble ? f->dpoff.p : nullptr, f->n_rigs,
                                      f->rig_fixed ? f->dfixed.p : nullptr));
@@ -1783,7 +1773,7 @@ int scphd_reserve(scphd_t* f, int64_t n_gaussians, int32_t max_meas) {
     for (DBuf<int32_t>* b : {&f->glead, &f->gsta, &f->gend, &f->gmem}) HIPTRY(b->ensure(G + 1));
     /* the global-scratch merge workspace, sized like the survivor lists (a
      * growth between frames would otherwise allocate in the update) */
-    HIPTRY(f->mscratch.ensure(merge_scratch_bytes(G + 1, (int)Np)));
+    HIPTRY(f->mscratch.ensure(merge_scratch_bytes(G + 1, (int)Np, nullptr, true)));
     /* per (parent, measurement) and the measurement sets */
     HIPTRY(f->eta.ensure(Np * M));
     HIPTRY(f->mcnt.ensure(Np * M));

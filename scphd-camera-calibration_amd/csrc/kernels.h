@@ -275,12 +275,15 @@ struct MergeArgs {
     const BirthModel* births; /* per rig, device memory: birth terms' covariance */
     double min_separation;
     int Np;
-    int32_t lds_cap;   /* parents with more survivors use global scratch */
+    int32_t lds_cap;   /* parents with more survivors form their groups in global scratch */
+    int32_t rounds_cap; /* and these run the round loop there */
     int32_t force_rounds; /* nonzero: every parent takes the round loop (verification of that path) */
     int32_t all_pairs;    /* nonzero: candidates from all pairs, as for ill-conditioned survivors (verification) */
-    int32_t big_lds_up;   /* big parents with next_pow2(U) <= this sort in the launch's LDS (12 B per slot) */
-    int32_t big_lds_bytes; /* the big launch's LDS: the sort keys, then the walk's per-survivor arrays (<= 64 KB) */
-    char* scratch;     /* global scratch for big parents: merge_scratch_bytes(Stot, Np) */
+    int32_t ws_slot, ws_parent; /* scratch bytes per survivor and per parent */
+    char* scratch;     /* merge_scratch_bytes(Stot, Np, ...) */
+    double img_width = 1.0;
+    const DisparityMeasurementModel* rig_meas = nullptr; /* per rig, in an ensemble */
+    const int32_t* prig = nullptr;
     double* mw;        /* merged outputs at survoff[p] + k */
     double* mmu;       /* 6 planes, stride scap */
     double* mP;        /* 21 planes, stride scap */
@@ -292,12 +295,14 @@ struct MergeArgs {
     int32_t* gmem;     /* per survivor slot: group members (survivor indices) */
     int64_t Stot;
 };
-/* Greedy merge of every parent's survivors: groups (sort, neighbour lists,
- * walk), moments per group, and the round loop for parents whose
+/* Greedy merge of every parent's survivors (at most max_surv): groups (neighbour
+ * lists, leaders), moments per group, and the round loop for parents whose
  * neighbour lists overflow the workspace. */
-hipError_t launch_merge(hipStream_t s, const MergeArgs& a, int lds_bytes);
+hipError_t launch_merge(hipStream_t s, const MergeArgs& a, int max_surv);
 int merge_lds_bytes(int cap);
-int64_t merge_scratch_bytes(int64_t Stot, int Np);
+/* scratch for the neighbour pairs, and with `big` for the workspaces of
+ * parents beyond the LDS; sets a's strides in it */
+int64_t merge_scratch_bytes(int64_t Stot, int Np, MergeArgs* a, bool big);
 hipError_t launch_iota(hipStream_t s, int32_t* x, int64_t n, int32_t start = 0);
 /* Removal of a rig's parents [P0, P0 + Nr) and their Gaussians [G0, G0 + Gr)
  * from an ensemble's map table: the entries after them move down, their

@@ -1541,17 +1541,11 @@ __global__ __launch_bounds__(NT) void k_survivors(SurvArgs a) {
 }
 
 /* -------------------------------------------------------------- merging */
-/* Workspace of one parent's merge, U survivor slots (Up = next power of two):
+/* Workspace of one parent's round loop, U survivor slots (Up = next power of two):
  *   key_w double[Up]  sort keys;            ord   int[Up]   (weight desc, index asc) order
  *   bu, bv double[U]  mean u, v;            bs    double[3U] (u,v) covariance block uu uv vv
  *   flag  uint8[U]    merged;               selfm uint8[U]  member of its own group
- *   nbo   int[U+1]    neighbour offsets;    cnt   int[U]    neighbour counts / fill cursors
- *   mem   int[U]      group members;
- *   nbr   int[ecap]   neighbour lists, ecap = 8 U + 64
- *   cand  uint32[ccap] candidate pairs i << 16 | j (i < j), ccap = 16 U + 64
- *   res   uint8[ccap] their membership
- * While the candidates are enumerated, ord holds the (u, index) order,
- * selfm the ill-conditioned flags and mem the list of those survivors. */
+ *   mem   int[U]      group members;        memb  uint8[U]  round membership */
 __host__ __device__ inline int next_pow2(int x) {
     int v = 1;
     while (v < x) v <<= 1;
@@ -1559,7 +1553,7 @@ __host__ __device__ inline int next_pow2(int x) {
 }
 
 struct MergeLayout {
-    int64_t ord, bu, bv, bs, flag, selfm, nbo, cnt, mem, nbr, ecap, cand, ccap, res, bytes;
+    int64_t ord, bu, bv, bs, flag, selfm, mem, memb, bytes;
     __host__ __device__ explicit MergeLayout(int U) {
         const int64_t Up = next_pow2(U > 0 ? U : 1);
         ord = Up * 8;
@@ -1568,26 +1562,65 @@ struct MergeLayout {
         bs = bv + (int64_t)U * 8;
         flag = bs + (int64_t)U * 24;
         selfm = flag + U;
-        nbo = (selfm + U + 7) & ~(int64_t)7;
-        cnt = nbo + ((int64_t)U + 1) * 4;
-        mem = cnt + (int64_t)U * 4;
-        nbr = mem + (int64_t)U * 4;
-        ecap = 8 * (int64_t)U + 64;
-        cand = nbr + ecap * 4;
-        ccap = 16 * (int64_t)U + 64;
-        res = cand + ccap * 4;
-        bytes = res + ccap;
+        mem = (selfm + U + 7) & ~(int64_t)7;
+        memb = mem + (int64_t)U * 4;
+        bytes = (memb + U + 7) & ~(int64_t)7;
     }
 };
 
 /* global scratch for parents that do not fit in LDS: MergeLayout(U).bytes
- * <= 190 U + 600 since Up < 2 U */
-static constexpr int64_t MERGE_WS_PER_SLOT = 240, MERGE_WS_PER_PARENT = 1024;
+ * <= 71 U + 32 since Up < 2 U, GroupsLayout's and the pairs 49 U + 344 */
+static constexpr int MERGE_WS_PER_SLOT = 72, MERGE_WS_PER_PARENT = 512;
+
+/* k_merge_groups' workspace of one parent, U survivor slots, in LDS or (BIG)
+ * in global scratch.  The survivors in bins of u, while the candidates are
+ * enumerated:
+ *   u, v  double[U]  mean;  s  float[3U]  (u, v) covariance uu uv vv (uu < 0:
+ *   ill-conditioned);  id  uint16[U]  survivor;  ill  uint16[U]  those ones
+ * and in the same place, from the weight sort on:
+ *   key   double[U]  weights; then nbr  uint16[ecap]  neighbour lists, ranks
+ *   nbo   int[U+1]   list offsets;      cnt  int[U]  fill cursors, then groups
+ *   ord   uint16[U]  survivor of a rank
+ *   own   uint16[U]  rank of a survivor; then rank of a rank's leader
+ *   st    uint8[U]   undecided, leader or member
+ * and over both self uint8[U] (member of its own group).  The neighbour pairs
+ * i << 16 | j, up to ecap / 2, go to global scratch. */
+struct GroupsLayout {
+    int64_t v, s, id, ill, bnbo, cnt, ord, own, st, self, bytes;
+    __host__ __device__ explicit GroupsLayout(int U) {
+        const int64_t n = U;
+        v = 8 * n;
+        s = 16 * n;
+        id = 28 * n;
+        ill = 30 * n;
+        bnbo = 2 * (8 * n + 64);
+        cnt = bnbo + 4 * (n + 1);
+        ord = cnt + 4 * n; /* the bitonic sort's 12 next_pow2(U) < 24 U bytes end before it */
+        own = ord + 2 * n;
+        st = own + 2 * n;
+        const int64_t b = st + n;
+        self = 32 * n > b ? 32 * n : b;
+        bytes = (self + n + 7) & ~(int64_t)7;
+    }
+};
+static constexpr int GROUPS_PAIRS_PER_SLOT = 16, GROUPS_PAIRS_PER_PARENT = 128;
+
+/* k_merge_groups' dynamic LDS for parents of up to U survivors, and the
+ * largest U of which two workgroups fit a CU and of which one does (160 KB,
+ * of which the kernel's own arrays take 13 each) */
+int groups_lds_bytes(int U) { return (int)GroupsLayout(std::max(U, 0)).bytes; }
+static constexpr int GROUPS_CAP2 = 2048, GROUPS_CAP1 = 4352;
 
 int merge_lds_bytes(int cap) { return (int)MergeLayout(cap).bytes; }
 
-int64_t merge_scratch_bytes(int64_t Stot, int Np) {
-    return Stot * MERGE_WS_PER_SLOT + (int64_t)Np * MERGE_WS_PER_PARENT + 256;
+int64_t merge_scratch_bytes(int64_t Stot, int Np, MergeArgs* a, bool big) {
+    const int slot = big ? MERGE_WS_PER_SLOT : GROUPS_PAIRS_PER_SLOT;
+    const int parent = big ? MERGE_WS_PER_PARENT : GROUPS_PAIRS_PER_PARENT;
+    if (a) {
+        a->ws_slot = slot;
+        a->ws_parent = parent;
+    }
+    return Stot * slot + (int64_t)Np * parent + 256;
 }
 
 /* Packed covariance entry e of a survivor's term: the updated covariance of
@@ -1598,10 +1631,15 @@ __device__ inline double term_P(const MergeArgs& a, int g, int e) {
     return g >= 0 ? a.pre[(int64_t)PP_PN * a.Ng + (int64_t)g * 21 + e] : a.births[-1 - g].P[e];
 }
 
+/* all of them (a pointer chosen once: 16-byte loads) */
+__device__ inline const double* term_P_all(const MergeArgs& a, int g) {
+    return g >= 0 ? a.pre + (int64_t)PP_PN * a.Ng + (int64_t)g * 21 : a.births[-1 - g].P;
+}
+
 __device__ inline void survivor_P(const MergeArgs& a, int64_t si, double* P) {
-    const int g = a.sg[si];
+    const double* o = term_P_all(a, a.sg[si]);
 #pragma unroll
-    for (int e = 0; e < 21; ++e) P[e] = term_P(a, g, e);
+    for (int e = 0; e < 21; ++e) P[e] = o[e];
 }
 
 __device__ inline void survivor_mu(const MergeArgs& a, int64_t si, double* mu) {
@@ -1609,7 +1647,7 @@ __device__ inline void survivor_mu(const MergeArgs& a, int64_t si, double* mu) {
     for (int c = 0; c < 6; ++c) mu[c] = a.smu[(si) * 6 + c];
 }
 
-/* Workspace pointers of one parent's merge. */
+/* Workspace pointers of one parent's round loop. */
 struct MergeWs {
     double* key_w;
     int* ord;
@@ -1618,13 +1656,8 @@ struct MergeWs {
     double* bs;
     uint8_t* flag;
     uint8_t* selfm;
-    int* nbo;
-    int* cnt;
     int* mem;
-    int* nbr;
-    uint32_t* cand;
-    uint8_t* res;
-    int64_t ecap, ccap;
+    uint8_t* memb;
     __device__ MergeWs(char* ws, int U) {
         const MergeLayout ly(U);
         key_w = (double*)ws;
@@ -1634,14 +1667,8 @@ struct MergeWs {
         bs = (double*)(ws + ly.bs);
         flag = (uint8_t*)(ws + ly.flag);
         selfm = (uint8_t*)(ws + ly.selfm);
-        nbo = (int*)(ws + ly.nbo);
-        cnt = (int*)(ws + ly.cnt);
         mem = (int*)(ws + ly.mem);
-        nbr = (int*)(ws + ly.nbr);
-        cand = (uint32_t*)(ws + ly.cand);
-        res = (uint8_t*)(ws + ly.res);
-        ecap = ly.ecap;
-        ccap = ly.ccap;
+        memb = (uint8_t*)(ws + ly.memb);
     }
 };
 
@@ -1679,10 +1706,8 @@ __device__ inline bool merge_pair(const MergeArgs& a, int64_t sbase, const Merge
     return merge_bound(w, i, j, thr) && merge_full(a, sbase, i, j, thr);
 }
 
-/* Bitonic sort of ord[0, Up) by key_w: ascending (key, index) when ASC,
- * else descending key with ascending index on ties.  Padding slots carry
- * keys that sort last.  Ends with a barrier. */
-template <bool ASC>
+/* Bitonic sort of ord[0, Up) by descending key with ascending index on
+ * ties.  Padding slots carry keys that sort last.  Ends with a barrier. */
 __device__ inline void merge_bitonic(double* key, int* ord, int Up) {
     const int t = threadIdx.x;
     __syncthreads();
@@ -1693,8 +1718,7 @@ __device__ inline void merge_bitonic(double* key, int* ord, int Up) {
                 if (l > i) {
                     const double wi = key[i], wl = key[l];
                     const int ii = ord[i], il = ord[l];
-                    const bool l_before_i = ASC ? ((wl < wi) || (wl == wi && il < ii))
-                                                : ((wl > wi) || (wl == wi && il < ii));
+                    const bool l_before_i = (wl > wi) || (wl == wi && il < ii);
                     const bool asc = (i & k) == 0;
                     if (asc == l_before_i) {
                         key[i] = wl;
@@ -1709,33 +1733,6 @@ __device__ inline void merge_bitonic(double* key, int* ord, int Up) {
     }
 }
 
-/* Load one parent's survivors' (u, v) marginals into the workspace, clear
- * the merged flags, and sort them by (u, index): key[r] is the u of rank r
- * (+inf for a u that is not finite, which sorts last), ord[r] its survivor.
- * key and ord hold next_pow2(U) entries. */
-__device__ inline void merge_load_sort_u(const MergeArgs& a, int64_t sbase, int U, MergeWs& w, double* key,
-                                         int* ord) {
-    const int t = threadIdx.x;
-    const int Up = next_pow2(U);
-    for (int i = t; i < Up; i += NT) {
-        if (i < U) {
-            w.bu[i] = a.smu[(sbase + i) * 6 + 0];
-            w.bv[i] = a.smu[(sbase + i) * 6 + 1];
-            const int g = a.sg[sbase + i];
-            w.bs[3 * i] = term_P(a, g, pidx(0, 0));
-            w.bs[3 * i + 1] = term_P(a, g, pidx(1, 0));
-            w.bs[3 * i + 2] = term_P(a, g, pidx(1, 1));
-            w.flag[i] = 0;
-            key[i] = isfinite(w.bu[i]) ? w.bu[i] : INFINITY;
-            ord[i] = i;
-        } else {
-            key[i] = INFINITY;
-            ord[i] = 0x7fffffff;
-        }
-    }
-    merge_bitonic<true>(key, ord, Up);
-}
-
 /* Sort one parent's survivors by (weight desc, index asc) into ord, the
  * order in which the reference's argmax loop picks leaders (ties: lowest
  * pack index). */
@@ -1747,12 +1744,21 @@ __device__ inline void merge_sort_w(const MergeArgs& a, int64_t sbase, int U, do
         key[i] = i < U ? a.sw[sbase + i] : -INFINITY;
         ord[i] = i < U ? i : 0x7fffffff;
     }
-    merge_bitonic<false>(key, ord, Up);
+    merge_bitonic(key, ord, Up);
 }
 
-/* Load and sort by weight (the round loop). */
+/* The round loop's start: the (u, v) marginals, no survivor merged, and the
+ * order by weight. */
 __device__ inline void merge_load_sort(const MergeArgs& a, int64_t sbase, int U, MergeWs& w) {
-    merge_load_sort_u(a, sbase, U, w, w.key_w, w.ord);
+    for (int i = threadIdx.x; i < U; i += NT) {
+        w.bu[i] = a.smu[(sbase + i) * 6 + 0];
+        w.bv[i] = a.smu[(sbase + i) * 6 + 1];
+        const int g = a.sg[sbase + i];
+        w.bs[3 * i] = term_P(a, g, pidx(0, 0));
+        w.bs[3 * i + 1] = term_P(a, g, pidx(1, 0));
+        w.bs[3 * i + 2] = term_P(a, g, pidx(1, 1));
+        w.flag[i] = 0;
+    }
     merge_sort_w(a, sbase, U, w.key_w, w.ord);
 }
 
@@ -1763,73 +1769,18 @@ __device__ inline bool merge_self(const MergeArgs& a, int64_t si, double thr) {
     return mahal6(m, P, m, P) < thr;
 }
 
-/* Step 2 of k_merge_groups: the merge candidates, from the survivors
- * sorted by (u, index) (key[r] = u of rank r, ord[r] its survivor; in LDS
- * when they fit, else in the workspace). */
-__device__ inline void merge_candidates(const MergeArgs& a, int U, MergeWs& w, double thr, const double* key,
-                                        const int* ord, int* s_nc, int* s_nill, double* s_red) {
-    const int t = threadIdx.x;
-    /* 2. candidates: the pairs that pass merge_bound, enumerated without
-     * visiting all U (U - 1) / 2 pairs.
-     *   A survivor is ill-conditioned when its (u, v) block is not PD with
-     *   det > 2e-6 puu pvv (or holds a non-finite value).  For two that are
-     *   not, the block of their sum has det > 1e-6 suu svv (the correlation
-     *   of a sum of PSD 2x2 blocks is at most the larger of theirs:
-     *   |auv + buv| <= r (sqrt(auu avv) + sqrt(buu bvv)) <= r sqrt(suu svv)
-     *   by Cauchy-Schwarz), so merge_bound decides by q <= 1.001 thr det,
-     *   and q suu - du^2 det = (suv du - suu dv)^2 >= 0 makes that imply
-     *   du^2 <= 1.001 thr suu.  Such pairs lie within
-     *   du^2 <= 1.002 thr (puu_i + max puu) of each other in u: each
-     *   survivor scans its successors in (u, index) order up to that
-     *   window.  (Every survivor of this filter has puu <= std_u^2: a
-     *   Kalman update with H = [I2 0] never raises the measured variance
-     *   above R, and births carry R; the windows span a few pixels.)
-     *   Pairs with an ill-conditioned survivor are tested against all
-     *   others.  The candidate set is the one the full U^2 sweep finds. */
-    for (int i = t; i < U; i += NT) w.cnt[i] = 0;
-    if (t == 0) *s_nill = 0;
-    __syncthreads();
-    double smax = 0.0;
-    for (int i = t; i < U; i += NT) {
-        const double suu = w.bs[3 * i], suv = w.bs[3 * i + 1], svv = w.bs[3 * i + 2];
-        const bool good = !a.all_pairs && isfinite(w.bu[i]) && isfinite(w.bv[i]) && isfinite(suu) && isfinite(suv) &&
-                          isfinite(svv) && suu > 0.0 && svv > 0.0 && suu * svv - suv * suv > 2e-6 * suu * svv;
-        w.selfm[i] = good ? 0 : 1;
-        if (good) {
-            smax = fmax(smax, suu);
-        } else {
-            w.mem[atomicAdd(s_nill, 1)] = i;
-        }
-    }
-    smax = block_max(smax, s_red); /* ends with a barrier after the flags */
-    {
-        auto add = [&](int i, int j) {
-            const int lo = min(i, j), hi = max(i, j);
-            if (merge_bound(w, lo, hi, thr)) {
-                const int c = atomicAdd(s_nc, 1);
-                if (c < w.ccap) w.cand[c] = ((uint32_t)lo << 16) | (uint32_t)hi;
-            }
-        };
-        for (int r = t; r < U; r += NT) {
-            const int i = ord[r];
-            if (w.selfm[i]) continue;
-            const double ui = key[r];
-            const double lim2 = 1.002 * thr * (w.bs[3 * i] + smax);
-            for (int r2 = r + 1; r2 < U; ++r2) {
-                const int j = ord[r2];
-                const double du = key[r2] - ui;
-                if (!(du * du <= lim2)) break;
-                if (!w.selfm[j]) add(i, j);
-            }
-        }
-        const int nill = *s_nill;
-        const int64_t nx = (int64_t)nill * U;
-        for (int64_t e = t; e < nx; e += NT) {
-            const int i = w.mem[e / U], j = (int)(e % U);
-            if (j == i || (w.selfm[j] && j < i)) continue; /* two ill survivors: once */
-            add(i, j);
-        }
-    }
+/* A pair's marginal bound from the stored means and covariances (merge_bound
+ * for the pairs of an ill-conditioned survivor). */
+__device__ inline bool merge_bound_at(const MergeArgs& a, int64_t si, int64_t sj, double thr) {
+    const double du = a.smu[sj * 6] - a.smu[si * 6], dv = a.smu[sj * 6 + 1] - a.smu[si * 6 + 1];
+    const int gi = a.sg[si], gj = a.sg[sj];
+    const double suu = term_P(a, gi, pidx(0, 0)) + term_P(a, gj, pidx(0, 0));
+    const double suv = term_P(a, gi, pidx(1, 0)) + term_P(a, gj, pidx(1, 0));
+    const double svv = term_P(a, gi, pidx(1, 1)) + term_P(a, gj, pidx(1, 1));
+    const double det = suu * svv - suv * suv;
+    if (!(det > 1e-6 * suu * svv)) return true;
+    const double q = svv * du * du - 2.0 * suv * du * dv + suu * dv * dv;
+    return !(q > 1.001 * thr * det);
 }
 
 /* Greedy Gaussian-mixture merge (phdUpdateMergeKernel, src/kernels.cu:662-874):
@@ -1840,30 +1791,46 @@ __device__ inline void merge_candidates(const MergeArgs& a, int U, MergeWs& w, d
  *
  * Evaluated in phases instead of the reference's barrier-bound rounds.
  * k_merge_groups (one workgroup per parent):
- *   1. sort by (u, index);
- *   2. candidate pairs i < j that pass merge_bound, found by scanning a
- *      window in u around each survivor (and every pair of an
- *      ill-conditioned survivor), compacted in the workspace; then sort by
- *      (weight desc, index asc);
- *   3. the full 6x6 test, one lane per candidate pair (and per self pair),
- *      so that lanes stay busy however sparse the candidates are;
- *   4. neighbour lists from the members, each sorted ascending;
- *   5. one lane walks the sorted order forming each leader's group from its
- *      unmerged neighbours -- the same groups as the round loop, since
- *      membership depends only on the pair.
+ *   1. the survivors in bins of u;
+ *   2. candidate pairs from each survivor's window of bins, those that pass
+ *      the (u, v) marginal's bound (single precision, with its rounding
+ *      errors on the safe side: it only chooses what is tested) into a
+ *      buffer; whenever it is full, the full 6x6 test, one lane per pair (and
+ *      per self pair), so that lanes stay busy however sparse the candidates
+ *      are;
+ *   3. ranks by (weight desc, index asc): buckets of the weight's leading
+ *      bits, then the order within a bucket (bitonic, should one hold more
+ *      than MERGE_BUCKET);
+ *   4. neighbour lists, by rank;
+ *   5. the greedy walk's outcome without the walk: membership depends only on
+ *      the pair, so a survivor leads a group when no heavier neighbour does,
+ *      and else belongs to the heaviest neighbour that does.  Decided in
+ *      rounds, each survivor as soon as its heavier neighbours are;
+ *   6. groups in rank order by two scans, members ascending by index.  A
+ *      leader that is not its own member ends the walk.
  * k_merge_moments (one thread per group): moments with members summed in
  * ascending index order.  k_merge_rounds: the round loop, for parents whose
- * candidate or neighbour lists overflow the workspace. */
+ * neighbour lists overflow the workspace.
+ *
+ * Bound: latency of short phases; three workgroups of 1200 survivors share a
+ * CU.  Ten frames of 4096 parents, 200 landmarks (1000 survivors and 4800
+ * candidates a parent): 27.6 ms with two bitonic sorts, the lists and a walk
+ * per connected component in global scratch; 12.0 so. */
+static constexpr int MERGE_BINS = 512, MERGE_CAND = 2048, MERGE_BUCKET = 1024;
+
 template <bool BIG>
-__global__ __launch_bounds__(NT) void k_merge_groups(MergeArgs a) {
+__global__ __launch_bounds__(NT) void k_merge_groups(MergeArgs a, int lo, int hi) {
     extern __shared__ char lds[];
-    __shared__ int s_nc, s_tot;
+    __shared__ int s_n, s_np, s_nill, s_stop;
     __shared__ int sh[8];
+    __shared__ double s_red[8];
+    __shared__ int s_off[MERGE_BINS + 1], s_cur[MERGE_BINS];
+    __shared__ uint32_t s_cand[MERGE_CAND];
     const int p = blockIdx.x;
     const int t = threadIdx.x;
     const int64_t sbase = a.survoff[p];
     const int U = a.survoff[p + 1] - a.survoff[p];
-    if (BIG != (U > a.lds_cap)) return; /* the other launch handles this parent (uniform) */
+    if (U <= lo || U > hi) return; /* another launch handles this parent (uniform) */
     if (U == 0) {
         if (t == 0) {
             a.ngroups[p] = 0;
@@ -1871,298 +1838,402 @@ __global__ __launch_bounds__(NT) void k_merge_groups(MergeArgs a) {
         }
         return;
     }
-    if (U >= 65536 || a.force_rounds) { /* candidate pairs pack two 16-bit indices: the round loop takes it */
+    if (U >= 65536 || a.force_rounds) { /* pairs pack two 16-bit indices: the round loop takes it */
         if (t == 0) {
             a.ngroups[p] = -1;
             a.nmerged[p] = 0;
         }
         return;
     }
+    char* const scratch = a.scratch + sbase * a.ws_slot + (int64_t)p * a.ws_parent;
+    uint32_t* const pairs = (uint32_t*)scratch;
+    const int pcap = 4 * U + 32;
     /* a compile-time choice of workspace, so that the LDS instantiation
      * addresses it with ds_* instructions rather than flat ones */
-    char* ws = BIG ? (a.scratch + sbase * MERGE_WS_PER_SLOT + (int64_t)p * MERGE_WS_PER_PARENT) : lds;
-    MergeWs w(ws, U);
+    char* const ws = BIG ? scratch + (int64_t)U * GROUPS_PAIRS_PER_SLOT + GROUPS_PAIRS_PER_PARENT : lds;
+    const GroupsLayout ly(U);
     const double thr = a.min_separation;
-    if (t == 0) s_nc = 0;
-    /* 1-2. sort by (u, index), candidates, sort by weight: the sort keys
-     * in LDS for a big parent whose keys fit the launch's LDS, else in the
-     * workspace */
-    __shared__ int s_nill;
-    __shared__ double s_red[8];
-    const int Up = next_pow2(U);
-    const bool keys_lds = BIG && Up <= a.big_lds_up;
-    /* once the keys are sorted, the LDS they held takes the walk's most
-     * accessed per-survivor arrays (global scratch otherwise): neighbour
-     * counts and offsets always, and when the launch's LDS allows (28 B per
-     * survivor) the component labels, bucket offsets and cursors and the
-     * per-rank group records */
-    int* lds_lab = nullptr;
-    int* lds_boff = nullptr;
-    int* lds_rinfo = nullptr;
-    if (keys_lds) {
-        double* key = (double*)lds;
-        int* ord = (int*)(lds + (size_t)8 * Up);
-        merge_load_sort_u(a, sbase, U, w, key, ord); /* ends with a barrier */
-        merge_candidates(a, U, w, thr, key, ord, &s_nc, &s_nill, s_red);
-        __syncthreads();
-        if (s_nc <= w.ccap) {
-            merge_sort_w(a, sbase, U, key, ord);
-            for (int i = t; i < U; i += NT) w.ord[i] = ord[i];
-            __syncthreads(); /* the sort keys are read */
-            /* U + (U + 1) ints within the keys' 12 Up bytes */
-            w.cnt = (int*)lds;
-            w.nbo = (int*)lds + U;
-            if ((int64_t)(7 * U + 2) * 4 <= a.big_lds_bytes) {
-                lds_lab = (int*)lds + 2 * U + 1;
-                lds_boff = lds_lab + U;
-                lds_rinfo = lds_boff + 2 * U + 1;
-            }
-            for (int i = t; i < U; i += NT) w.cnt[i] = 0;
-        }
-    } else {
-        merge_load_sort_u(a, sbase, U, w, w.key_w, w.ord);
-        merge_candidates(a, U, w, thr, w.key_w, w.ord, &s_nc, &s_nill, s_red);
-        __syncthreads();
-        if (s_nc <= w.ccap) merge_sort_w(a, sbase, U, w.key_w, w.ord);
-    }
+    uint8_t* const self = (uint8_t*)(ws + ly.self);
 
+    /* s_cur[0, MERGE_BINS) to exclusive offsets s_off and cursors */
+    auto offsets = [&]() {
+        constexpr int E = MERGE_BINS / NT;
+        int c[E], mine = 0;
+#pragma unroll
+        for (int e = 0; e < E; ++e) mine += c[e] = s_cur[E * t + e];
+        int tot;
+        int o = block_exscan(mine, sh, &tot);
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            s_off[E * t + e] = s_cur[E * t + e] = o;
+            o += c[e];
+        }
+        if (t == 0) s_off[MERGE_BINS] = tot;
+        __syncthreads();
+    };
+    auto clear = [&]() {
+        for (int b = t; b < MERGE_BINS; b += NT) s_cur[b] = 0;
+        __syncthreads();
+    };
+
+    /* 1. bins of u, monotone in u (a NaN's the first) */
+    const double bin_scale =
+        MERGE_BINS / fabs(a.rig_meas ? a.rig_meas[a.prig[p]].img_width() : a.img_width);
+    auto bin = [&](double u) { return (int)fmin(fmax(u * bin_scale, 0.0), (double)(MERGE_BINS - 1)); };
+    if (t == 0) s_n = s_np = s_nill = 0;
+    clear();
+    /* a survivor's (u, v) marginal; the first few of a thread are held in
+     * registers over the barriers, so that their loads wait once */
+    struct Marginal {
+        double u, v, suu, suv, svv;
+        int bin;
+    };
+    constexpr int HELD = 4;
+    auto load_mean = [&](int i, Marginal& m) {
+        m.u = a.smu[(sbase + i) * 6];
+        m.v = a.smu[(sbase + i) * 6 + 1];
+    };
+    auto load_cov = [&](int g, Marginal& m) {
+        const double* P = term_P_all(a, g);
+        m.suu = P[pidx(0, 0)];
+        m.suv = P[pidx(1, 0)];
+        m.svv = P[pidx(1, 1)];
+    };
+    Marginal held[HELD];
+    {
+        int g[HELD];
+#pragma unroll
+        for (int e = 0; e < HELD; ++e) {
+            const int i = min(t + e * NT, U - 1);
+            load_mean(i, held[e]);
+            g[e] = a.sg[sbase + i];
+        }
+#pragma unroll
+        for (int e = 0; e < HELD; ++e) load_cov(g[e], held[e]);
+    }
+#pragma unroll
+    for (int e = 0; e < HELD; ++e) {
+        held[e].bin = bin(held[e].u);
+        if (t + e * NT < U) atomicAdd(&s_cur[held[e].bin], 1);
+    }
+    for (int i = t + HELD * NT; i < U; i += NT) atomicAdd(&s_cur[bin(a.smu[(sbase + i) * 6])], 1);
     __syncthreads();
-    const int nc = s_nc;
-    if (nc > w.ccap) {
+    offsets();
+    {
+        double* const bu = (double*)ws;
+        double* const bv = (double*)(ws + ly.v);
+        float* const bs = (float*)(ws + ly.s);
+        uint16_t* const id = (uint16_t*)(ws + ly.id);
+        uint16_t* const ill = (uint16_t*)(ws + ly.ill);
+        double smax = 0.0, smax_v = 0.0;
+        auto good = [&](const Marginal& m) {
+            return !a.all_pairs && isfinite(m.u) && isfinite(m.v) && isfinite(m.suu) && isfinite(m.suv) &&
+                   isfinite(m.svv) && m.suu > 0.0 && m.svv > 0.0 &&
+                   m.suu * m.svv - m.suv * m.suv > 2e-6 * m.suu * m.svv;
+        };
+        auto place = [&](int i, const Marginal& m) {
+            const int q = atomicAdd(&s_cur[m.bin], 1);
+            const bool ok = good(m);
+            bu[q] = m.u;
+            bv[q] = m.v;
+            bs[3 * q] = ok ? (float)m.suu : -1.0f;
+            bs[3 * q + 1] = (float)m.suv;
+            bs[3 * q + 2] = (float)m.svv;
+            id[q] = (uint16_t)i;
+            if (ok) {
+                smax = fmax(smax, m.suu);
+                smax_v = fmax(smax_v, m.svv);
+            } else {
+                ill[atomicAdd(&s_nill, 1)] = (uint16_t)i;
+            }
+        };
+#pragma unroll
+        for (int e = 0; e < HELD; ++e)
+            if (t + e * NT < U) place(t + e * NT, held[e]);
+        for (int i = t + HELD * NT; i < U; i += NT) {
+            Marginal m;
+            load_mean(i, m);
+            load_cov(a.sg[sbase + i], m);
+            m.bin = bin(m.u);
+            place(i, m);
+        }
+        smax = block_max(smax, s_red);
+        smax_v = block_max(smax_v, s_red);
+        __syncthreads();
+        /* 2. candidates.
+         *   A survivor is ill-conditioned when its (u, v) block is not PD with
+         *   det > 2e-6 puu pvv (or holds a non-finite value).  For two that are
+         *   not, the block of their sum has det > 1e-6 suu svv (the correlation
+         *   of a sum of PSD 2x2 blocks is at most the larger of theirs:
+         *   |auv + buv| <= r (sqrt(auu avv) + sqrt(buu bvv)) <= r sqrt(suu svv)
+         *   by Cauchy-Schwarz), so the marginal's bound on the distance is
+         *   q / det with q = svv du^2 - 2 suv du dv + suu dv^2, and
+         *   q suu - du^2 det = (suv du - suu dv)^2 >= 0 makes q <= thr det
+         *   imply du^2 <= thr suu.  Such pairs lie within
+         *   du^2 <= 1.002 thr (puu_i + max puu) of each other in u: each
+         *   survivor meets those after it up to the bin that window ends in,
+         *   eight at a time for their v, which must lie within the same of it.
+         *   (Every survivor of this filter has puu <= std_u^2: a Kalman update
+         *   with H = [I2 0] never raises the measured variance above R, and
+         *   births carry R; the windows span a few pixels.)  q is rejected
+         *   when it exceeds thr det by 0.1 % and by the single-precision
+         *   errors of both (below 1e-6 of their terms).
+         *   Pairs with an ill-conditioned survivor are tested against all
+         *   others. */
+        const float thrf = (float)(1.0011 * thr);
+        int q = t, q2 = 0, qend = 0; /* survivor q, the next block of others */
+        uint32_t near = 0;           /* those of the last block near in v */
+        float suu = 0, suv = 0, svv = 0;
+        double u = 0, v = 0, vlim = 0;
+        auto open = [&]() { /* survivor q's window */
+            if (q >= U) return;
+            u = bu[q];
+            v = bv[q];
+            suu = bs[3 * q];
+            suv = bs[3 * q + 1];
+            svv = bs[3 * q + 2];
+            q2 = q + 1;
+            const double hw = sqrt(1.002 * thr * (1.000001 * (double)suu + smax)) * 1.000001 + 1e-12 * fabs(u);
+            vlim = 1.002 * thr * (1.000001 * (double)svv + smax_v);
+            qend = suu < 0.0f ? 0 : s_off[bin(u + hw) + 1];
+        };
+        open();
+        const int64_t nx = (int64_t)s_nill * U;
+        int64_t e = t; /* of the ill-conditioned survivors' pairs */
+        int selfs = U; /* self tests, with the first buffer */
+        for (;;) {
+            /* `pair` to the buffer; false when it is full */
+            auto push = [&](int i, int j) {
+                const int c = atomicAdd(&s_n, 1);
+                if (c >= MERGE_CAND) return false;
+                s_cand[c] = (uint32_t)min(i, j) << 16 | (uint32_t)max(i, j);
+                return true;
+            };
+            bool room = true;
+            while (room && q < U) {
+                if (!near) {
+                    if (q2 >= qend) {
+                        q += NT;
+                        open();
+                        continue;
+                    }
+                    double d[8];
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) d[k] = bv[min(q2 + k, U - 1)] - v;
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) near |= d[k] * d[k] <= vlim ? 1u << k : 0u;
+                    near &= (1u << min(qend - q2, 8)) - 1u;
+                    q2 += 8;
+                    continue;
+                }
+                const int q1 = q2 - 8 + __builtin_ctz(near);
+                const float auu = bs[3 * q1];
+                const float du = (float)(bu[q1] - u), dv = (float)(bv[q1] - v);
+                const float tuu = suu + auu, tuv = suv + bs[3 * q1 + 1], tvv = svv + bs[3 * q1 + 2];
+                const float x = tvv * du * du, y = tuu * dv * dv, w = tuu * tvv;
+                const bool far = x + y - 2.0f * tuv * du * dv - 1e-6f * (x + y) > thrf * (w - tuv * tuv + 1e-6f * w);
+                if (auu < 0.0f || far || (room = push(id[q], id[q1]))) near &= near - 1u;
+            }
+            while (room && e < nx) {
+                const int i = ill[e / U], j = (int)(e % U);
+                /* two ill survivors: once */
+                const bool other = j != i && (j > i || !a.all_pairs);
+                bool skip = !other;
+                if (other && j < i) { /* is j ill too? */
+                    Marginal m;
+                    load_mean(j, m);
+                    load_cov(a.sg[sbase + j], m);
+                    skip = !good(m);
+                }
+                if (skip || !merge_bound_at(a, sbase + min(i, j), sbase + max(i, j), thr) || (room = push(i, j))) e += NT;
+            }
+            __syncthreads();
+            const int nc = min(s_n, MERGE_CAND);
+            for (int c = t; c < nc + selfs; c += NT) {
+                const uint32_t pr = c < nc ? s_cand[c] : (uint32_t)(c - nc) * 0x10001u;
+                const bool in = merge_full(a, sbase, (int)(pr >> 16), (int)(pr & 0xFFFFu), thr);
+                if (c >= nc) {
+                    self[c - nc] = in ? 1 : 0;
+                } else if (in) {
+                    const int k = atomicAdd(&s_np, 1);
+                    if (k < pcap) pairs[k] = pr;
+                }
+            }
+            selfs = 0;
+            const int more = __syncthreads_or(!room);
+            if (!more) break;
+            if (t == 0) s_n = 0;
+            __syncthreads();
+        }
+    }
+    const int np = s_np;
+    if (np > pcap) {
         if (t == 0) {
             a.ngroups[p] = -1;
             a.nmerged[p] = 0;
         }
         return;
     }
-    /* 3. full tests: candidates, then every survivor against itself */
-    for (int c = t; c < nc + U; c += NT) {
-        if (c < nc) {
-            const int i = (int)(w.cand[c] >> 16), j = (int)(w.cand[c] & 0xFFFFu);
-            const bool m = merge_full(a, sbase, i, j, thr);
-            w.res[c] = m ? 1 : 0;
-            if (m) {
-                atomicAdd(&w.cnt[i], 1);
-                atomicAdd(&w.cnt[j], 1);
+    /* 3. ranks */
+    uint16_t* const ord = (uint16_t*)(ws + ly.ord);
+    uint16_t* const own = (uint16_t*)(ws + ly.own);
+    {
+        double* const key = (double*)ws;
+        uint16_t* const tmp = (uint16_t*)(ws + 8 * (int64_t)U);
+        /* five bits of the mantissa; weights below 2^-15 share a bucket */
+        auto bucket = [&](double w) {
+            return min(max((1024 << 5) - 1 - (__double2hiint(w) >> 15), 0), MERGE_BINS - 1);
+        };
+        clear();
+        for (int i = t; i < U; i += NT) {
+            const double w = a.sw[sbase + i];
+            key[i] = w;
+            atomicAdd(&s_cur[bucket(w)], 1);
+        }
+        __syncthreads();
+        int most = 0;
+        for (int b = t; b < MERGE_BINS; b += NT) most = max(most, s_cur[b]);
+        if (!__syncthreads_or(most > MERGE_BUCKET)) {
+            offsets();
+            for (int i = t; i < U; i += NT) tmp[atomicAdd(&s_cur[bucket(key[i])], 1)] = (uint16_t)i;
+            __syncthreads();
+            for (int x = t; x < U; x += NT) {
+                const int i = tmp[x];
+                const double w = key[i];
+                const int b = bucket(w), y0 = s_off[b], y1 = s_off[b + 1];
+                int r = y0;
+                for (int y = y0; y < y1; y += 4) { /* four reads wait together */
+                    int j[4];
+                    double o[4];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) j[k] = tmp[min(y + k, y1 - 1)];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) o[k] = key[j[k]];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k)
+                        r += y + k < y1 && (o[k] > w || (o[k] == w && j[k] < i)) ? 1 : 0;
+                }
+                ord[r] = (uint16_t)i;
+                own[i] = (uint16_t)r;
             }
         } else {
-            const int i = c - nc;
-            w.selfm[i] = merge_self(a, sbase + i, thr) ? 1 : 0;
+            int* const o = (int*)(ws + 8 * (int64_t)next_pow2(U));
+            merge_sort_w(a, sbase, U, key, o);
+            for (int r = t; r < U; r += NT) {
+                ord[r] = (uint16_t)o[r];
+                own[o[r]] = (uint16_t)r;
+            }
         }
+        __syncthreads();
     }
-    __syncthreads();
-    /* 4. neighbour lists: offsets (rows [r0, r1) per thread), fill, sort */
+    /* 4. neighbour lists: offsets (rows [r0, r1) per thread), fill */
+    uint16_t* const nbr = (uint16_t*)ws;
+    int* const nbo = (int*)(ws + ly.bnbo);
+    int* const cnt = (int*)(ws + ly.cnt);
+    uint8_t* const st = (uint8_t*)(ws + ly.st);
     const int rc = (U + NT - 1) / NT;
     const int r0 = min(U, t * rc), r1 = min(U, r0 + rc);
-    int mine = 0;
-    for (int i = r0; i < r1; ++i) mine += w.cnt[i];
-    int tot;
-    int base = block_exscan(mine, sh, &tot);
-    for (int i = r0; i < r1; ++i) {
-        w.nbo[i] = base;
-        base += w.cnt[i];
-        w.cnt[i] = 0;
-    }
-    if (t == 0) {
-        w.nbo[U] = tot;
-        s_tot = tot;
+    for (int i = t; i < U; i += NT) {
+        cnt[i] = 0;
+        st[i] = 0;
     }
     __syncthreads();
-    if (s_tot > w.ecap) {
-        if (t == 0) {
-            a.ngroups[p] = -1;
-            a.nmerged[p] = 0;
-        }
-        return;
-    }
-    for (int c = t; c < nc; c += NT)
-        if (w.res[c]) {
-            const int i = (int)(w.cand[c] >> 16), j = (int)(w.cand[c] & 0xFFFFu);
-            w.nbr[w.nbo[i] + atomicAdd(&w.cnt[i], 1)] = j;
-            w.nbr[w.nbo[j] + atomicAdd(&w.cnt[j], 1)] = i;
-        }
-    __syncthreads();
-    for (int i = t; i < U; i += NT) { /* insertion sort: lists are short */
-        const int e0 = w.nbo[i], e1 = w.nbo[i + 1];
-        for (int e = e0 + 1; e < e1; ++e) {
-            const int x = w.nbr[e];
-            int f = e - 1;
-            while (f >= e0 && w.nbr[f] > x) {
-                w.nbr[f + 1] = w.nbr[f];
-                --f;
-            }
-            w.nbr[f + 1] = x;
-        }
+    for (int c = t; c < np; c += NT) {
+        const uint32_t pr = pairs[c];
+        atomicAdd(&cnt[own[pr >> 16]], 1);
+        atomicAdd(&cnt[own[pr & 0xFFFFu]], 1);
     }
     __syncthreads();
-    /* 5. the greedy walk.  A survivor with an empty neighbour list is
-     * isolated: no leader takes it, so when the walk reaches it, it forms
-     * the group {itself}, or stops the walk when it is not its own member.
-     * The sequential walk therefore visits only the connected survivors, in
-     * rank order; every rank's outcome (group size, stop) is then placed in
-     * rank order by two scans.  Per rank r: rinfo[2 r] = group size | STOP,
-     * rinfo[2 r + 1] = start of the members in tmp (connected leaders). */
-    constexpr int STOP = 1 << 30;
-    int* rinfo = lds_rinfo ? lds_rinfo : (int*)w.bu; /* bu is free after the candidates: 8 bytes per slot */
-    int* nl = w.cnt;         /* connected ranks, ascending; free after the lists */
-    int* tmp = (int*)w.cand; /* members of connected groups; ccap >= U */
     {
         int mine = 0;
-        for (int r = r0; r < r1; ++r) mine += w.nbo[w.ord[r] + 1] != w.nbo[w.ord[r]];
-        int nn;
-        int k = block_exscan(mine, sh, &nn);
+        for (int r = r0; r < r1; ++r) mine += cnt[r];
+        int tot;
+        int base = block_exscan(mine, sh, &tot);
         for (int r = r0; r < r1; ++r) {
-            const int L = w.ord[r];
-            if (w.nbo[L + 1] != w.nbo[L]) {
-                nl[k++] = r;
-                rinfo[2 * r] = 0;
-            } else {
-                rinfo[2 * r] = w.selfm[L] ? 1 : STOP;
-            }
-        }
-        if (t == 0) s_tot = nn;
-    }
-    __syncthreads();
-    /* The walk per connected component.  A leader takes only unmerged
-     * neighbours, so the groups formed in one component of the neighbour
-     * graph depend only on that component's ranks and flags: each
-     * component is walked on its own, in rank order, by one lane.  (The
-     * reference's loop ends at the first leader that is not its own member;
-     * a component walked past that rank forms groups the rank-ordered
-     * placement below discards, exactly as if the walk had stopped.)
-     *   labels: the smallest survivor index of the component, by min
-     *           propagation along the neighbour lists;
-     *   buckets: the connected ranks grouped by label (counts, scan,
-     *           scatter), each bucket sorted by rank by its lane;
-     *   members of a group go to tmp inside its bucket's range, ascending
-     *           by survivor index with the leader in its place. */
-    {
-        const int nn = s_tot;
-        int* lab = lds_lab ? lds_lab : (int*)w.bv; /* label per survivor (bv is free after the candidates) */
-        int* gb = (int*)w.bs;            /* bs is free after the candidates */
-        int* boff = lds_boff ? lds_boff : gb; /* bucket offsets [U + 1] */
-        int* bcur = boff + (U + 1);      /* scatter cursors [U] */
-        int* bkt = gb + 2 * U + 1;       /* connected ranks by bucket [nn] */
-        int* seg = (int*)w.key_w;        /* non-empty buckets (key_w is free after the sorts) */
-        for (int i = t; i < U; i += NT) {
-            lab[i] = i;
-            boff[i] = 0;
+            nbo[r] = base;
+            base += cnt[r];
+            cnt[r] = nbo[r];
         }
         if (t == 0) {
-            boff[U] = 0;
-            s_nc = 0;
-        }
-        __syncthreads();
-        for (;;) {
-            int changed = 0;
-            for (int k = t; k < nn; k += NT) {
-                const int i = w.ord[nl[k]];
-                int m = lab[i];
-                for (int e = w.nbo[i]; e < w.nbo[i + 1]; ++e) m = min(m, lab[w.nbr[e]]);
-                if (m < lab[i]) {
-                    lab[i] = m;
-                    changed = 1;
-                }
-            }
-            if (!__syncthreads_or(changed)) break;
-        }
-        for (int k = t; k < nn; k += NT) atomicAdd(&boff[lab[w.ord[nl[k]]]], 1);
-        __syncthreads();
-        {
-            int mine = 0;
-            for (int i = r0; i < r1; ++i) mine += boff[i];
-            int tot;
-            int base = block_exscan(mine, sh, &tot);
-            for (int i = r0; i < r1; ++i) {
-                const int c = boff[i];
-                boff[i] = base;
-                bcur[i] = base;
-                if (c > 0) seg[atomicAdd(&s_nc, 1)] = i;
-                base += c;
-            }
-            if (t == 0) boff[U] = tot;
-        }
-        __syncthreads();
-        for (int k = t; k < nn; k += NT) {
-            const int r = nl[k];
-            bkt[atomicAdd(&bcur[lab[w.ord[r]]], 1)] = r;
-        }
-        __syncthreads();
-        const int nseg = s_nc;
-        for (int q = t; q < nseg; q += NT) {
-            const int b0 = seg[q];
-            const int k0 = boff[b0], k1 = bcur[b0]; /* the cursor ends at the bucket's end */
-            for (int k = k0 + 1; k < k1; ++k) { /* ranks ascending: buckets are small */
-                const int x = bkt[k];
-                int f = k - 1;
-                while (f >= k0 && bkt[f] > x) {
-                    bkt[f + 1] = bkt[f];
-                    --f;
-                }
-                bkt[f + 1] = x;
-            }
-            int tp = k0;
-            for (int k = k0; k < k1; ++k) {
-                const int r = bkt[k], L = w.ord[r];
-                if (w.flag[L]) continue; /* taken by an earlier leader */
-                const bool sm = w.selfm[L] != 0;
-                const int st = tp;
-                bool placed = !sm;
-                for (int e = w.nbo[L]; e < w.nbo[L + 1]; ++e) {
-                    const int j = w.nbr[e];
-                    if (w.flag[j]) continue;
-                    if (!placed && j > L) {
-                        tmp[tp++] = L;
-                        placed = true;
-                    }
-                    tmp[tp++] = j;
-                    w.flag[j] = 1;
-                }
-                if (!placed) tmp[tp++] = L;
-                if (sm) w.flag[L] = 1;
-                const int gsz = tp - st;
-                /* empty group: zero weight, the reference stops; a leader
-                 * outside its group is taken again, finds nothing and stops */
-                rinfo[2 * r] = gsz | (sm ? 0 : STOP);
-                rinfo[2 * r + 1] = st;
-                if (!sm || gsz == 0) break;
-            }
+            nbo[U] = tot;
+            s_stop = U;
         }
     }
     __syncthreads();
-    if (t == 0) s_nc = U; /* first stopping rank */
+    for (int c = t; c < np; c += NT) {
+        const uint32_t pr = pairs[c];
+        const int x = own[pr >> 16], y = own[pr & 0xFFFFu];
+        nbr[atomicAdd(&cnt[x], 1)] = (uint16_t)y;
+        nbr[atomicAdd(&cnt[y], 1)] = (uint16_t)x;
+    }
     __syncthreads();
-    for (int r = r0; r < r1; ++r)
-        if (rinfo[2 * r] & STOP) {
-            atomicMin(&s_nc, r);
-            break;
+    /* 5. leaders (1) and members (2).  A neighbour's state may change while
+     * it is read, to what it stays. */
+    for (;;) {
+        int left = 0;
+        for (int r = t; r < U; r += NT) {
+            if (st[r]) continue;
+            int s = 1;
+            const int e1 = nbo[r + 1];
+            for (int e = nbo[r]; e < e1 && s != 2; e += 4) { /* four reads wait together */
+                int x[4], sx[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) x[k] = nbr[min(e + k, e1 - 1)];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) sx[k] = *(volatile uint8_t*)(st + x[k]);
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    if (x[k] < r && sx[k] != 2) s = sx[k] == 1 || s == 2 ? 2 : 0;
+            }
+            *(volatile uint8_t*)(st + r) = (uint8_t)s;
+            left |= s == 0;
         }
+        if (!__syncthreads_or(left)) break;
+    }
+    /* each rank's leader; sizes; the first leader that is not its own
+     * member, after which no group forms */
+    for (int r = t; r < U; r += NT) cnt[r] = 0;
     __syncthreads();
+    for (int r = t; r < U; r += NT) {
+        int L = r;
+        bool counts = true;
+        if (st[r] == 2) {
+            for (int e = nbo[r]; e < nbo[r + 1]; ++e) {
+                const int x = nbr[e];
+                if (x < L && st[x] == 1) L = x;
+            }
+        } else if (!self[ord[r]]) {
+            atomicMin(&s_stop, r);
+            counts = false;
+        }
+        own[r] = (uint16_t)L;
+        if (counts) atomicAdd(&cnt[L], 1);
+    }
+    __syncthreads();
+    /* 6. groups in rank order */
     {
-        const int rstop = s_nc; /* ranks after it form no group */
+        const int re = min(r1, s_stop + 1);
         int mg = 0, mm = 0;
-        for (int r = r0; r < min(r1, rstop + 1); ++r) {
-            const int n = rinfo[2 * r] & (STOP - 1);
-            mg += n > 0;
-            mm += n;
+        for (int r = r0; r < re; ++r) {
+            if (st[r] != 1) continue;
+            mg += cnt[r] > 0;
+            mm += cnt[r];
         }
-        int ng;
+        int ng, mtot;
         int gi = block_exscan(mg, sh, &ng);
-        int mtot;
         int mp = block_exscan(mm, sh, &mtot);
-        for (int r = r0; r < min(r1, rstop + 1); ++r) {
-            const int n = rinfo[2 * r] & (STOP - 1);
+        for (int r = r0; r < r1; ++r) {
+            if (st[r] != 1) continue;
+            const int n = cnt[r];
+            if (r >= re) {
+                cnt[r] = -1; /* forms no group */
+                continue;
+            }
+            cnt[r] = mp;
             if (n == 0) continue;
-            const int L = w.ord[r];
-            a.glead[sbase + gi] = L;
+            a.glead[sbase + gi] = ord[r];
             a.gsta[sbase + gi] = mp;
             a.gend[sbase + gi] = mp + n;
-            if (w.nbo[L + 1] == w.nbo[L]) {
-                w.mem[mp] = L;
-            } else {
-                const int s0 = rinfo[2 * r + 1];
-                for (int q = 0; q < n; ++q) w.mem[mp + q] = tmp[s0 + q];
-            }
             ++gi;
             mp += n;
         }
@@ -2172,7 +2243,16 @@ __global__ __launch_bounds__(NT) void k_merge_groups(MergeArgs a) {
         }
     }
     __syncthreads();
-    for (int i = t; i < U; i += NT) a.gmem[sbase + i] = w.mem[i];
+    for (int r = t; r < U; r += NT) {
+        const int L = own[r], st0 = cnt[L], i = ord[r];
+        if (st0 < 0 || (L == r && !self[i])) continue;
+        int k = L != r && self[ord[L]] && ord[L] < i ? 1 : 0;
+        for (int e = nbo[L]; e < nbo[L + 1]; ++e) {
+            const int x = nbr[e];
+            k += own[x] == L && x != L && ord[x] < i ? 1 : 0;
+        }
+        a.gmem[sbase + st0 + k] = i;
+    }
 }
 
 __global__ __launch_bounds__(128) void k_merge_moments(MergeArgs a) {
@@ -2246,8 +2326,8 @@ __global__ __launch_bounds__(NT) void k_merge_rounds(MergeArgs a) {
     if (a.ngroups[p] != -1) return; /* uniform */
     const int64_t sbase = a.survoff[p];
     const int U = a.survoff[p + 1] - a.survoff[p];
-    if (BIG != (U > a.lds_cap)) return;
-    char* ws = BIG ? (a.scratch + sbase * MERGE_WS_PER_SLOT + (int64_t)p * MERGE_WS_PER_PARENT) : lds;
+    if (BIG != (U > a.rounds_cap)) return;
+    char* ws = BIG ? (a.scratch + sbase * a.ws_slot + (int64_t)p * a.ws_parent) : lds;
     MergeWs w(ws, U);
     const double thr = a.min_separation;
     merge_load_sort(a, sbase, U, w);
@@ -2257,7 +2337,7 @@ __global__ __launch_bounds__(NT) void k_merge_rounds(MergeArgs a) {
     const int lane = t & 63, wave = t >> 6;
     const int64_t mbase = sbase;
     int K = 0;
-    uint8_t* memb = (uint8_t*)w.nbr; /* round membership bits; the neighbour-list area is free here */
+    uint8_t* memb = w.memb; /* round membership */
     for (;;) {
         if (wave == 0) {
             int found = -1;
@@ -3053,12 +3133,18 @@ hipError_t launch_survivors(hipStream_t s, const SurvArgs& a) {
     LAUNCH_CHECK();
 }
 
-hipError_t launch_merge(hipStream_t s, const MergeArgs& a, int lds_bytes) {
-    k_merge_groups<false><<<a.Np, NT, lds_bytes, s>>>(a);
-    if (a.scratch) k_merge_groups<true><<<a.Np, NT, a.big_lds_bytes, s>>>(a);
+hipError_t launch_merge(hipStream_t s, const MergeArgs& a, int max_surv) {
+    /* a launch's LDS is that of its largest parent: one for those of which
+     * two share a CU, one for those that take a CU each, and the rest in
+     * global scratch */
+    const int cap2 = std::min(a.lds_cap, GROUPS_CAP2), cap1 = std::min(a.lds_cap, GROUPS_CAP1);
+    k_merge_groups<false><<<a.Np, NT, groups_lds_bytes(std::min(max_surv, cap2)), s>>>(a, -1, cap2);
+    if (max_surv > cap2 && cap1 > cap2)
+        k_merge_groups<false><<<a.Np, NT, groups_lds_bytes(std::min(max_surv, cap1)), s>>>(a, cap2, cap1);
+    if (max_surv > cap1) k_merge_groups<true><<<a.Np, NT, 0, s>>>(a, cap1, INT32_MAX);
     if (a.Stot > 0) k_merge_moments<<<nblocks(a.Stot, 128), 128, 0, s>>>(a);
-    k_merge_rounds<false><<<a.Np, NT, lds_bytes, s>>>(a);
-    if (a.scratch) k_merge_rounds<true><<<a.Np, NT, 0, s>>>(a);
+    k_merge_rounds<false><<<a.Np, NT, merge_lds_bytes(std::max(1, std::min(max_surv, a.rounds_cap))), s>>>(a);
+    if (max_surv > a.rounds_cap) k_merge_rounds<true><<<a.Np, NT, 0, s>>>(a);
     LAUNCH_CHECK();
 }
 
