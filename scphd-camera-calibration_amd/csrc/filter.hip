@@ -845,7 +845,7 @@ int create_filter(const scphd_params* p, int32_t n_rigs, bool ensemble, scphd_t*
     if (f->ext.ensure(12 * (int64_t)Np) || f->ext_tmp.ensure(12 * (int64_t)Np) || f->pw.ensure(Np) ||
         f->pose.ensure(12 * (int64_t)Np) || f->loglik.ensure(Np) || f->cum.ensure(Np) || f->anc.ensure(Np) ||
         f->newcnt.ensure(Np + 1) || f->goff.ensure(Np + 1) || f->goff2.ensure(Np + 1) || f->dneff.ensure(n_rigs) ||
-        f->drflag.ensure(n_rigs) || f->dflag.ensure(4) || f->gparent.ensure(1) || f->gblock.ensure(1) ||
+        f->drflag.ensure(2 * n_rigs) || f->dflag.ensure(4) || f->gparent.ensure(1) || f->gblock.ensure(1) ||
         f->gw.ensure(1))
         return bail(SCPHD_ERR_HIP);
     std::vector<BirthModel> births(n_rigs);
@@ -976,7 +976,7 @@ int scphd_ensemble_add_rig(scphd_t* f, const scphd_params* p, int32_t* rig_out) 
     HIPTRY(grow_keep(f->anc, Np_new, P0, s));
     HIPTRY(grow_keep(f->goff, Np_new + 1, (int64_t)P0 + 1, s));
     HIPTRY(grow_keep(f->dneff, R, R - 1, s));
-    HIPTRY(grow_keep(f->drflag, R, R - 1, s));
+    HIPTRY(grow_keep(f->drflag, 2 * R, R - 1, s));
     HIPTRY(f->ext_tmp.ensure(12 * Np_new));
     HIPTRY(f->pose.ensure(12 * Np_new));
     HIPTRY(f->cum.ensure(Np_new));
@@ -1241,6 +1241,7 @@ int scphd_resample(scphd_t* f, int32_t* resampled) {
     ra.goff = f->goff.p;
     ra.Np = Np;
     ra.poff = f->ensemble ? f->dpoff.p : nullptr;
+    ra.prig = f->ensemble ? f->dprig.p : nullptr;
     ra.nrigs = f->n_rigs;
     ra.min_neff = f->prm.min_neff;
     ra.key = f->key;
@@ -1249,6 +1250,7 @@ int scphd_resample(scphd_t* f, int32_t* resampled) {
     ra.rstep = (uint64_t)f->n_resample;
     ra.flag = f->dflag.p;
     ra.rflag = f->drflag.p;
+    ra.amax = f->drflag.p + f->n_rigs;
     ra.neff = f->dneff.p;
     HIPTRY(hipMemsetAsync(f->dflag.p, 0, sizeof(int32_t), s));
     HIPTRY(launch_resample(s, ra));
@@ -1261,6 +1263,7 @@ int scphd_resample(scphd_t* f, int32_t* resampled) {
     const int go = f->hmap[3];
     if (resampled) *resampled = go;
     if (!go) return SCPHD_OK;
+    std::swap(f->ext, f->ext_tmp); /* the gathered states */
     const int64_t Nnew = f->hmap[0];
     HIPTRY(f->gparent2.ensure(Nnew + 1));
     HIPTRY(f->gblock2.ensure(Nnew + 1));
@@ -1362,6 +1365,7 @@ int scphd_resample_noalloc(scphd_t* f, int32_t* resampled) {
     ra.rstep = (uint64_t)f->n_resample;
     ra.flag = (int32_t*)(base + ly.flag);
     ra.rflag = f->drflag.p;
+    ra.amax = f->drflag.p + f->n_rigs;
     ra.neff = f->dneff.p;
     ra.defer = 1;
     /* the scratch keeps the last call's contents: clear the flag */

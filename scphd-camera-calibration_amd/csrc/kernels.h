@@ -411,19 +411,23 @@ struct ResampleArgs {
     int32_t* anc;
     int32_t* newcnt;
     const int32_t* goff;
-    int Np;                /* parents of the one rig when poff is null */
+    int Np;                /* parents of all rigs */
     const int32_t* poff = nullptr; /* ensemble: rig r's parents [poff[r], poff[r + 1]) */
-    int nrigs = 1;         /* one workgroup per rig */
+    const int32_t* prig = nullptr; /* ensemble: a parent's rig */
+    int nrigs = 1;
     double min_neff;
     NoiseKey key;          /* one rig */
     const NoiseKey* keys = nullptr; /* ensemble: per rig, or nullptr */
     const uint32_t* sbase = nullptr; /* ensemble: per rig, the handle's step counts at joining (SC_COUNT each) */
     uint64_t rstep;
     int32_t* flag;  /* out: 1 if any rig resampled (zero before the launch) */
-    int32_t* rflag = nullptr; /* out: per rig, 1 if resampled (may be null) */
+    int32_t* rflag; /* out: per rig, 1 if resampled */
+    int32_t* amax;  /* scratch, per rig */
     double* neff;   /* out: per rig */
-    int defer = 0;  /* nonzero: leave ext and pw unchanged (k_resample_commit applies the gather) */
+    int defer = 0;  /* nonzero: leave pw unchanged too (k_resample_commit applies the gather) */
 };
+/* n_eff, the decision, ancestors and their map sizes, and when any rig
+ * resampled every parent's new state in ext_tmp and the rigs' new weights */
 hipError_t launch_resample(hipStream_t s, const ResampleArgs& a);
 /* Apply a deferred resampling of one rig's N parents: anc_out <- anc, and
  * when go, ext <- ext_tmp and pw <- 1/N. */

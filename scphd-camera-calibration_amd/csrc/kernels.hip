@@ -2739,53 +2739,46 @@ __global__ void k_table(TableArgs a) {
  * systematic resampling with points u + j/N against the sequential
  * cumulative sum of the weights (resample :2651-2702), the overrun fallback
  * to the first maximum of exp(w), gather of parent states, and weights 1/N.
- * One workgroup.  The cumulative sum keeps the reference's left-to-right
- * rounding: thread 0 accumulates chunks staged in LDS. */
-static constexpr int RS_CH = 2048;
+ *
+ * k_resample, one workgroup a rig: n_eff, the decision, the cumulative sum
+ * and the fallback.  The sum keeps the reference's left-to-right rounding,
+ * so it is a chain of N additions: the first wavefront adds sixteen weights
+ * at a time out of LDS in registers, while the others store the chunk before
+ * and load the next.  k_resample_draw, a parent a thread: its point's search
+ * (a chain of log2 N reads, so over the whole chip) and the gather.  16384
+ * parents: 620 us with the chain's sums stored one by one and the searches
+ * and gathers in the same workgroup; 100 so (a frame on average, half of
+ * which resample). */
+static constexpr int RS_CH = 2048, RS_STEP = 16;
 
 __global__ __launch_bounds__(1024) void k_resample(ResampleArgs a) {
     __shared__ double red[16];
-    __shared__ double s_u;
-    __shared__ double chunk[RS_CH];
+    __shared__ __attribute__((aligned(16))) double chunk[2][RS_CH];
     __shared__ double s_em[16];
     __shared__ int s_am[16];
-    /* one workgroup per rig: its Np parents from P0, ancestors within it */
     const int rig = blockIdx.x;
     const int N = a.poff ? a.poff[rig + 1] - a.poff[rig] : a.Np;
     const int64_t P0 = a.poff ? a.poff[rig] : 0;
-    a.pw += P0;
-    a.ext += P0 * 12;
-    a.ext_tmp += P0 * 12;
-    a.cum += P0;
-    a.anc += P0;
-    a.newcnt += P0;
-    a.goff += P0;
-    const NoiseKey key = a.keys ? a.keys[rig] : a.key;
-    /* the rig's own resample count: the handle's less its count at joining */
-    const uint64_t rstep = a.rstep - (a.sbase ? a.sbase[SC_COUNT * rig + SC_RESAMPLE] : 0u);
+    const double* const pw = a.pw + P0;
+    double* const cum = a.cum + P0;
     const int t = threadIdx.x;
     double ss = 0.0;
-    for (int p = t; p < N; p += blockDim.x) ss += a.pw[p] * a.pw[p];
+    for (int p = t; p < N; p += blockDim.x) ss += pw[p] * pw[p];
     ss = block_sum(ss, red);
     const double neff = 1.0 / (N * ss);
     const bool go = !(neff >= a.min_neff);
     if (t == 0) {
         a.neff[rig] = neff;
-        if (a.rflag) a.rflag[rig] = go ? 1 : 0;
+        a.rflag[rig] = go ? 1 : 0;
         if (go) atomicOr(a.flag, 1); /* any rig resampled; zero before the launch */
     }
-    if (!go) {
-        for (int p = t; p < N; p += blockDim.x) {
-            a.anc[p] = (int32_t)(P0 + p);
-            a.newcnt[p] = a.goff[p + 1] - a.goff[p];
-        }
-        return;
-    }
+    if (!go) return;
     /* first index of the maximum of exp(w) */
     double em = -1.0;
     int am = -1;
     for (int i = t; i < N; i += blockDim.x) {
-        const double e = exp(a.pw[i]);
+        const double w = pw[i], e = exp(w);
+        if (i < RS_CH) chunk[0][i] = w;
         if (e > em) {
             em = e;
             am = i;
@@ -2804,34 +2797,9 @@ __global__ __launch_bounds__(1024) void k_resample(ResampleArgs a) {
         s_em[t >> 6] = em;
         s_am[t >> 6] = am;
     }
-    if (t == 0) {
-        uint32_t x[4];
-        noise_block(key, NS_RESAMPLE, rstep, 0, 0, 0, 0, x);
-        s_u = uniform_co(x[0], x[1]) * (1.0 / N);
-    }
-    /* sequential cumulative sum */
-    double c = 0.0;
-    for (int c0 = 0; c0 < N; c0 += RS_CH) {
-        const int n = min(RS_CH, N - c0);
-        __syncthreads();
-        for (int i = t; i < n; i += blockDim.x) chunk[i] = a.pw[c0 + i];
-        __syncthreads();
-        if (t == 0) {
-            int i = 0;
-            if (c0 == 0) {
-                c = chunk[0];
-                a.cum[0] = c;
-                i = 1;
-            }
-            for (; i < n; ++i) {
-                c += chunk[i];
-                a.cum[c0 + i] = c;
-            }
-        }
-    }
     __syncthreads();
-    int amax = -1;
-    {
+    if (t == 0) {
+        int amax = -1;
         double bm = -1.0;
         for (int w = 0; w < (int)(blockDim.x >> 6); ++w) {
             if (s_am[w] >= 0 && (s_em[w] > bm || (s_em[w] == bm && s_am[w] < amax))) {
@@ -2839,29 +2807,90 @@ __global__ __launch_bounds__(1024) void k_resample(ResampleArgs a) {
                 amax = s_am[w];
             }
         }
+        a.amax[rig] = amax;
     }
-    const double interval = 1.0 / N;
-    for (int j = t; j < N; j += blockDim.x) {
-        const double r = s_u + j * interval;
-        int lo = 0, hi = N;
-        while (lo < hi) {
-            const int mid = (lo + hi) >> 1;
-            if (!(r > a.cum[mid]))
-                hi = mid;
-            else
-                lo = mid + 1;
+    /* sequential cumulative sum */
+    double c = 0.0;
+    int b = 0;
+    for (int c0 = 0; c0 < N; c0 += RS_CH, b ^= 1) {
+        if (t < 64) {
+            const int n = min(RS_CH, N - c0);
+            double* const x = chunk[b];
+            int i = 0;
+            double v[RS_STEP];
+            if (RS_STEP <= n) {
+#pragma unroll
+                for (int k = 0; k < RS_STEP; ++k) v[k] = x[k];
+            }
+            for (; i + RS_STEP <= n; i += RS_STEP) {
+                double w[RS_STEP]; /* the next, while this one's sums wait */
+                const int j = min(i + RS_STEP, RS_CH - RS_STEP);
+#pragma unroll
+                for (int k = 0; k < RS_STEP; ++k) w[k] = x[j + k];
+#pragma unroll
+                for (int k = 0; k < RS_STEP; ++k) v[k] = c += v[k];
+                if (t == 0) {
+#pragma unroll
+                    for (int k = 0; k < RS_STEP; ++k) x[i + k] = v[k];
+                }
+#pragma unroll
+                for (int k = 0; k < RS_STEP; ++k) v[k] = w[k];
+            }
+            for (; i < n; ++i) {
+                c += x[i];
+                if (t == 0) x[i] = c;
+            }
+        } else {
+            double* const x = chunk[b ^ 1];
+            for (int i = t - 64; i < RS_CH; i += blockDim.x - 64) {
+                const int at = c0 + i;
+                if (c0 > 0) cum[at - RS_CH] = x[i];
+                if (at + RS_CH < N) x[i] = pw[at + RS_CH];
+            }
         }
-        const int anc = lo < N ? lo : amax;
-        a.anc[j] = (int32_t)(P0 + anc);
-        for (int q = 0; q < 12; ++q) a.ext_tmp[(int64_t)j * 12 + q] = a.ext[(int64_t)anc * 12 + q];
-        a.newcnt[j] = a.goff[anc + 1] - a.goff[anc];
+        __syncthreads();
     }
-    if (a.defer) return; /* k_resample_commit applies the gather */
+    const int last = (N - 1) / RS_CH * RS_CH;
+    for (int i = t; last + i < N; i += blockDim.x) cum[last + i] = chunk[b ^ 1][i];
+}
+
+__global__ __launch_bounds__(256) void k_resample_draw(ResampleArgs a) {
+    __shared__ int s_anc[256];
+    const int t = threadIdx.x, j0 = blockIdx.x * 256, n = min(256, a.Np - j0);
+    const bool any = *a.flag != 0;
+    if (t < n) {
+        const int g = j0 + t;
+        const int rig = a.prig ? a.prig[g] : 0;
+        const int P0 = a.poff ? a.poff[rig] : 0, N = a.poff ? a.poff[rig + 1] - P0 : a.Np;
+        int anc = g;
+        if (a.rflag[rig]) {
+            const NoiseKey key = a.keys ? a.keys[rig] : a.key;
+            /* the rig's own resample count: the handle's less its count at joining */
+            const uint64_t rstep = a.rstep - (a.sbase ? a.sbase[SC_COUNT * rig + SC_RESAMPLE] : 0u);
+            uint32_t x[4];
+            noise_block(key, NS_RESAMPLE, rstep, 0, 0, 0, 0, x);
+            const double u = uniform_co(x[0], x[1]) * (1.0 / N);
+            const double interval = 1.0 / N;
+            const int j = g - P0;
+            const double r = u + j * interval;
+            int lo = 0, hi = N;
+            while (lo < hi) {
+                const int mid = (lo + hi) >> 1;
+                if (!(r > a.cum[P0 + mid]))
+                    hi = mid;
+                else
+                    lo = mid + 1;
+            }
+            anc = P0 + (lo < N ? lo : a.amax[rig]);
+            if (!a.defer) a.pw[g] = 1.0 / N;
+        }
+        a.anc[g] = anc;
+        a.newcnt[g] = a.goff[anc + 1] - a.goff[anc];
+        s_anc[t] = anc;
+    }
+    if (!any) return; /* uniform */
     __syncthreads();
-    for (int j = t; j < N; j += blockDim.x) {
-        for (int q = 0; q < 12; ++q) a.ext[(int64_t)j * 12 + q] = a.ext_tmp[(int64_t)j * 12 + q];
-        a.pw[j] = 1.0 / N;
-    }
+    for (int i = t; i < 12 * n; i += 256) a.ext_tmp[(int64_t)j0 * 12 + i] = a.ext[(int64_t)s_anc[i / 12] * 12 + i % 12];
 }
 
 __global__ void k_resample_commit(double* ext, const double* ext_tmp, double* pw, int32_t* anc_out,
@@ -3206,6 +3235,7 @@ hipError_t launch_table(hipStream_t s, const TableArgs& a) {
 
 hipError_t launch_resample(hipStream_t s, const ResampleArgs& a) {
     k_resample<<<a.poff ? a.nrigs : 1, 1024, 0, s>>>(a);
+    k_resample_draw<<<nblocks(a.Np, 256), 256, 0, s>>>(a);
     LAUNCH_CHECK();
 }
 
