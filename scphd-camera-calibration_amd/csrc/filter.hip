@@ -241,12 +241,12 @@ struct scphd_filter {
     int cur = 0;
     /* per-Gaussian intermediates */
     DBuf<double> fit, pre, lik;
-    DBuf<int32_t> keep, keepscan, ndlist, holes, redo, ndfill;
+    DBuf<int32_t> keep, ndlist, holes, redo, ndfill;
     DBuf<int32_t> wparent, wmerged; /* parent per wavefront of k_fit and of k_sample */
     /* measurements, normalisers, survivors, merge */
     DBuf<double> du, dv, eta;
     int capM = 0;
-    DBuf<int32_t> nsurv, survoff, nmerged, mergeoff, outcnt, scantmp, sg, sm, dflag, mcnt, knum, kjm;
+    DBuf<int32_t> nsurv, survoff, nmerged, mergeoff, nkeep, keepoff, scantmp, sg, sm, dflag, mcnt, knum, kjm;
     DBuf<int32_t> ngroups, glead, gsta, gend, gmem;
     DBuf<double> sw, smu, mw, mmu, mP, dneff, kw;
     DBuf<char> mscratch;
@@ -315,8 +315,8 @@ void for_each_buf(scphd_filter* f, Fn&& fn) {
     fn(f->dbirths); fn(f->dsbase); fn(f->dfixed); fn(f->ext); fn(f->pw); fn(f->pose); fn(f->loglik); fn(f->cum); fn(f->ext_tmp); fn(f->anc);
     fn(f->newcnt); fn(f->goff); fn(f->gparent); fn(f->gblock); fn(f->gw); fn(f->goff2); fn(f->gparent2);
     fn(f->gblock2); fn(f->gw2); fn(f->gpd); fn(f->gpd2); fn(f->fit); fn(f->pre); fn(f->lik); fn(f->keep);
-    fn(f->keepscan); fn(f->ndlist); fn(f->holes); fn(f->redo); fn(f->ndfill); fn(f->du); fn(f->dv); fn(f->eta); fn(f->nsurv);
-    fn(f->survoff); fn(f->nmerged); fn(f->mergeoff); fn(f->outcnt); fn(f->scantmp); fn(f->sg); fn(f->sm);
+    fn(f->nkeep); fn(f->keepoff); fn(f->ndlist); fn(f->holes); fn(f->redo); fn(f->ndfill); fn(f->du); fn(f->dv); fn(f->eta); fn(f->nsurv);
+    fn(f->survoff); fn(f->nmerged); fn(f->mergeoff); fn(f->scantmp); fn(f->sg); fn(f->sm);
     fn(f->dflag); fn(f->mcnt); fn(f->knum); fn(f->kjm); fn(f->kw); fn(f->ngroups); fn(f->glead); fn(f->gsta);
     fn(f->gend); fn(f->gmem); fn(f->sw); fn(f->smu); fn(f->mw); fn(f->mmu); fn(f->mP); fn(f->dneff);
     fn(f->mscratch); fn(f->wparent); fn(f->wmerged);
@@ -427,10 +427,10 @@ int update_t(scphd_filter* f, int M, int fixed) {
     record(f, 0);
 
     HIPTRY(f->wparent.ensure(wave_count(Ng, Np)));
+    HIPTRY(f->dflag.ensure(UC_COUNT));
     HIPTRY(launch_pose(s, f->ext.p, f->pose.p, Np, fixed, f->rig_fixed ? f->dprig.p : nullptr,
-                       f->rig_fixed ? f->dfixed.p : nullptr, f->goff.p, f->wparent.p));
-    HIPTRY(f->keepscan.ensure(Ng + 1));
-    HIPTRY(f->scantmp.ensure(scan_tmp_size(std::max<int64_t>(Ng, Np) + 1) + 16));
+                       f->rig_fixed ? f->dfixed.p : nullptr, f->goff.p, f->wparent.p, f->dflag.p));
+    HIPTRY(f->scantmp.ensure(scan_tmp_size(Np + 1) + 16));
     if (Ng > 0) {
         /* room for this step's posterior clouds too (the last step's count,
          * scaled by this step's measurement count, plus a quarter), so that
@@ -457,8 +457,8 @@ int update_t(scphd_filter* f, int M, int fixed) {
         HIPTRY(f->pre.ensure((int64_t)PP_COUNT * Ng));
         HIPTRY(f->lik.ensure((int64_t)LK_COUNT * (Ng + 3))); /* 3 records of padding: read four at a time */
         HIPTRY(f->keep.ensure(Ng));
-        HIPTRY(f->redo.ensure(Ng + 1)); /* [Ng]: the list length */
-        HIPTRY(f->ndfill.ensure(Ng + 1)); /* [Ng]: the list length */
+        HIPTRY(f->redo.ensure(Ng));
+        HIPTRY(f->ndfill.ensure(Ng));
         HIPTRY(f->ndlist.ensure(Ng));
         HIPTRY(f->holes.ensure(Ng));
         FitArgs fa;
@@ -483,11 +483,9 @@ int update_t(scphd_filter* f, int M, int fixed) {
         fa.fit = f->fit.p;
         fa.keep = f->keep.p;
         fa.redo = f->redo.p;
-        fa.redo_n = f->redo.p + Ng;
-        HIPTRY(hipMemsetAsync(fa.redo_n, 0, sizeof(int32_t), s));
+        fa.redo_n = f->dflag.p + UC_REDO;
         fa.ndfill = f->ndfill.p;
-        fa.ndfill_n = f->ndfill.p + Ng;
-        HIPTRY(hipMemsetAsync(fa.ndfill_n, 0, sizeof(int32_t), s));
+        fa.ndfill_n = f->dflag.p + UC_NDFILL;
         fa.nd_base = 0;
         fa.gpd = f->hint_ok ? f->gpd.p : nullptr;
         fa.arith32 = f->arith32 ? 1 : 0;
@@ -511,9 +509,9 @@ int update_t(scphd_filter* f, int M, int fixed) {
     HIPTRY(f->survoff.ensure(Np + 1));
     HIPTRY(f->nmerged.ensure(Np + 1));
     HIPTRY(f->mergeoff.ensure(Np + 1));
-    HIPTRY(f->outcnt.ensure(Np + 1));
+    HIPTRY(f->nkeep.ensure(Np + 1));
+    HIPTRY(f->keepoff.ensure(Np + 1));
     HIPTRY(f->goff2.ensure(Np + 1));
-    HIPTRY(f->dflag.ensure(4));
     EtaArgs ea;
     ea.goff = f->goff.p;
     ea.gw = f->gw.p;
@@ -537,6 +535,8 @@ int update_t(scphd_filter* f, int M, int fixed) {
     ea.eta = f->eta.p;
     ea.loglik = f->loglik.p;
     ea.nsurv = f->nsurv.p;
+    ea.keep = f->keep.p;
+    ea.nkeep = f->nkeep.p;
     HIPTRY(f->mcnt.ensure((int64_t)Np * std::max(M, 1)));
     /* room for the kept terms: ETA_NCAND a measurement, on average over a
      * parent's measurements */
@@ -554,8 +554,7 @@ int update_t(scphd_filter* f, int M, int fixed) {
     ea.img_height = f->models.meas.img_height();
     ea.rig_meas = f->ensemble ? f->dmeas.p : nullptr;
     HIPTRY(launch_eta(s, ea, f->max_map));
-    HIPTRY(launch_scan(s, f->nsurv.p, f->survoff.p, Np, f->scantmp.p));
-    HIPTRY(launch_readout(s, f->survoff.p, Np, 0, nullptr, nullptr, f->dmap));
+    HIPTRY(launch_scan_readout(s, f->nsurv.p, f->survoff.p, Np, f->scantmp.p, 0, nullptr, 0, nullptr, f->dmap));
     HIPTRY(hipStreamSynchronize(s));
     const int64_t Stot = f->hmap[0];
     const int maxU = f->hmap[1];
@@ -568,7 +567,6 @@ int update_t(scphd_filter* f, int M, int fixed) {
     HIPTRY(f->mw.ensure(scap));
     HIPTRY(f->mmu.ensure(6 * scap));
     HIPTRY(f->mP.ensure(21 * scap));
-    HIPTRY(hipMemsetAsync(f->dflag.p, 0, 4 * sizeof(int32_t), s));
     if (Stot > 0) {
         SurvArgs sa;
         sa.e = ea;
@@ -579,7 +577,7 @@ int update_t(scphd_filter* f, int M, int fixed) {
         sa.sm = f->sm.p;
         sa.smu = f->smu.p;
         sa.cap = scap;
-        sa.err = f->dflag.p;
+        sa.err = f->dflag.p + UC_ERR;
         HIPTRY(launch_survivors(s, sa));
     }
     record(f, 2);
@@ -628,19 +626,12 @@ int update_t(scphd_filter* f, int M, int fixed) {
     record(f, 3);
 
     /* output counts */
-    HIPTRY(launch_scan(s, f->nmerged.p, f->mergeoff.p, Np, f->scantmp.p));
-    if (Ng > 0)
-        HIPTRY(launch_scan(s, f->keep.p, f->keepscan.p, Ng, f->scantmp.p));
-    else
-        HIPTRY(hipMemsetAsync(f->keepscan.p, 0, sizeof(int32_t), s));
-    HIPTRY(f->wmerged.ensure(wave_count(Stot, Np)));
-    HIPTRY(launch_outcount(s, f->nmerged.p, f->goff.p, f->keepscan.p, Np, f->outcnt.p, f->mergeoff.p, f->wmerged.p));
-    HIPTRY(launch_scan(s, f->outcnt.p, f->goff2.p, Np, f->scantmp.p));
     /* the non-detection clouds in [0, Ng) of the next generation are
      * complete before any return or growth of the generation (which copies
      * them) */
     HIPTRY(hipStreamWaitEvent(s, f->ev_nd, 0));
-    HIPTRY(launch_readout(s, f->goff2.p, Np, P.max_gaussians, f->mergeoff.p + Np, f->dflag.p, f->dmap));
+    HIPTRY(launch_outputs(s, f->nmerged.p, f->nkeep.p, Np, f->scantmp.p, P.max_gaussians, f->dflag.p + UC_ERR,
+                          f->mergeoff.p, f->keepoff.p, f->goff2.p, f->dmap));
     HIPTRY(hipStreamSynchronize(s));
     flush_retired(f); /* both streams have drained */
     const int64_t Nout = f->hmap[0];
@@ -656,7 +647,9 @@ int update_t(scphd_filter* f, int M, int fixed) {
      * Ng on; the next generation holds Ng + max(0, Kt - holes) blocks */
     const int64_t nholes = Ng - (Nout - Kt);
     const int64_t over = std::max<int64_t>(0, Kt - nholes);
-    HIPTRY(launch_ndlist(s, f->keep.p, f->keepscan.p, Ng, f->ndlist.p, f->holes.p));
+    HIPTRY(f->wmerged.ensure(wave_count(Kt, Np)));
+    HIPTRY(launch_lists(s, f->keep.p, f->keepoff.p, f->goff.p, Np, f->ndlist.p, f->holes.p, f->mergeoff.p,
+                        f->wmerged.p));
     HIPTRY(f->gen[nxt].ensure(Ng + over, Ng, S, f->esz, s));
     SampleArgs pa;
     pa.mergeoff = f->mergeoff.p;
@@ -693,7 +686,7 @@ int update_t(scphd_filter* f, int M, int fixed) {
     ta.mergeoff = f->mergeoff.p;
     ta.survoff = f->survoff.p;
     ta.goff = f->goff.p;
-    ta.keepscan = f->keepscan.p;
+    ta.keepoff = f->keepoff.p;
     ta.ndlist = f->ndlist.p;
     ta.mw = f->mw.p;
     ta.gw = f->gw.p;
@@ -845,7 +838,7 @@ int create_filter(const scphd_params* p, int32_t n_rigs, bool ensemble, scphd_t*
     if (f->ext.ensure(12 * (int64_t)Np) || f->ext_tmp.ensure(12 * (int64_t)Np) || f->pw.ensure(Np) ||
         f->pose.ensure(12 * (int64_t)Np) || f->loglik.ensure(Np) || f->cum.ensure(Np) || f->anc.ensure(Np) ||
         f->newcnt.ensure(Np + 1) || f->goff.ensure(Np + 1) || f->goff2.ensure(Np + 1) || f->dneff.ensure(n_rigs) ||
-        f->drflag.ensure(2 * n_rigs) || f->dflag.ensure(4) || f->gparent.ensure(1) || f->gblock.ensure(1) ||
+        f->drflag.ensure(2 * n_rigs) || f->dflag.ensure(UC_COUNT) || f->gparent.ensure(1) || f->gblock.ensure(1) ||
         f->gw.ensure(1))
         return bail(SCPHD_ERR_HIP);
     std::vector<BirthModel> births(n_rigs);
@@ -1248,15 +1241,13 @@ int scphd_resample(scphd_t* f, int32_t* resampled) {
     ra.keys = f->ensemble ? f->dkeys.p : nullptr;
     ra.sbase = f->ensemble && f->sbase_used ? f->dsbase.p : nullptr;
     ra.rstep = (uint64_t)f->n_resample;
-    ra.flag = f->dflag.p;
     ra.rflag = f->drflag.p;
     ra.amax = f->drflag.p + f->n_rigs;
     ra.neff = f->dneff.p;
-    HIPTRY(hipMemsetAsync(f->dflag.p, 0, sizeof(int32_t), s));
     HIPTRY(launch_resample(s, ra));
     HIPTRY(f->scantmp.ensure(scan_tmp_size(Np + 1) + 16));
-    HIPTRY(launch_scan(s, f->newcnt.p, f->goff2.p, Np, f->scantmp.p));
-    HIPTRY(launch_readout(s, f->goff2.p, Np, 0, f->dflag.p, nullptr, f->dmap));
+    HIPTRY(launch_scan_readout(s, f->newcnt.p, f->goff2.p, Np, f->scantmp.p, 0, f->drflag.p, f->n_rigs, nullptr,
+                               f->dmap));
     HIPTRY(hipStreamSynchronize(s));
     flush_retired(f);
     f->n_resample++;
@@ -1316,9 +1307,9 @@ static hipError_t scratch_address(int dev, char** out) {
 }
 
 /* byte offsets into the scratch for n parents: cumulative weights,
- * gathered extrinsics, ancestors, new map sizes, scan partials, flags */
+ * gathered extrinsics, ancestors, new map sizes, scan partials, the fallback */
 struct NoAllocLayout {
-    size_t cum, ext_tmp, anc, newcnt, scantmp, flag, bytes;
+    size_t cum, ext_tmp, anc, newcnt, scantmp, amax, bytes;
     explicit NoAllocLayout(int n) {
         auto up = [](size_t x) { return (x + 255) & ~(size_t)255; };
         cum = 0;
@@ -1326,8 +1317,8 @@ struct NoAllocLayout {
         anc = up(ext_tmp + (size_t)n * 12 * sizeof(double));
         newcnt = up(anc + (size_t)n * sizeof(int32_t));
         scantmp = up(newcnt + ((size_t)n + 1) * sizeof(int32_t));
-        flag = up(scantmp + ((size_t)scan_tmp_size((int64_t)n + 1) + 16) * sizeof(int32_t));
-        bytes = up(flag + 4 * sizeof(int32_t));
+        amax = up(scantmp + ((size_t)scan_tmp_size((int64_t)n + 1) + 16) * sizeof(int32_t));
+        bytes = up(amax + 4 * sizeof(int32_t));
     }
 };
 
@@ -1363,16 +1354,13 @@ int scphd_resample_noalloc(scphd_t* f, int32_t* resampled) {
     ra.min_neff = f->prm.min_neff;
     ra.key = f->key;
     ra.rstep = (uint64_t)f->n_resample;
-    ra.flag = (int32_t*)(base + ly.flag);
     ra.rflag = f->drflag.p;
-    ra.amax = f->drflag.p + f->n_rigs;
+    ra.amax = (int32_t*)(base + ly.amax);
     ra.neff = f->dneff.p;
     ra.defer = 1;
-    /* the scratch keeps the last call's contents: clear the flag */
-    HIPTRY(launch_fill_i32(s, ra.flag, 0, 1));
     HIPTRY(launch_resample(s, ra));
-    HIPTRY(launch_scan(s, ra.newcnt, f->goff2.p, Np, (int32_t*)(base + ly.scantmp)));
-    HIPTRY(launch_readout(s, f->goff2.p, Np, 0, ra.flag, nullptr, f->dmap));
+    HIPTRY(launch_scan_readout(s, ra.newcnt, f->goff2.p, Np, (int32_t*)(base + ly.scantmp), 0, f->drflag.p, 1, nullptr,
+                               f->dmap));
     HIPTRY(hipStreamSynchronize(s));
     const int go = f->hmap[3];
     const int64_t Nnew = f->hmap[0];
@@ -1546,22 +1534,18 @@ int scphd_get_update_debug(scphd_t* f, double* eta, double* loglik, int32_t* nme
     const int Np = f->Np;
     /* an update of the current parents has run, and scphd_compact has not
      * released its outputs since */
-    if (!f->has_outputs || f->nmerged.n < Np || f->outcnt.n < Np || f->nsurv.n < Np ||
+    if (!f->has_outputs || f->nmerged.n < Np || f->nkeep.n < Np || f->nsurv.n < Np ||
         (f->last_M > 0 && f->eta.n < (int64_t)Np * f->last_M))
         return fail(f, SCPHD_ERR_STATE, "no update outputs for the current parents");
     if (eta && f->last_M > 0)
         HIPTRY(hipMemcpyAsync(eta, f->eta.p, (size_t)Np * f->last_M * sizeof(double), hipMemcpyDeviceToHost, s));
     if (loglik) HIPTRY(hipMemcpyAsync(loglik, f->loglik.p, (size_t)Np * sizeof(double), hipMemcpyDeviceToHost, s));
-    std::vector<int32_t> nm(Np), oc(Np);
-    HIPTRY(hipMemcpyAsync(nm.data(), f->nmerged.p, (size_t)Np * sizeof(int32_t), hipMemcpyDeviceToHost, s));
-    HIPTRY(hipMemcpyAsync(oc.data(), f->outcnt.p, (size_t)Np * sizeof(int32_t), hipMemcpyDeviceToHost, s));
+    if (nmerged) HIPTRY(hipMemcpyAsync(nmerged, f->nmerged.p, (size_t)Np * sizeof(int32_t), hipMemcpyDeviceToHost, s));
+    if (nnondetect)
+        HIPTRY(hipMemcpyAsync(nnondetect, f->nkeep.p, (size_t)Np * sizeof(int32_t), hipMemcpyDeviceToHost, s));
     if (nsurvivors)
         HIPTRY(hipMemcpyAsync(nsurvivors, f->nsurv.p, (size_t)Np * sizeof(int32_t), hipMemcpyDeviceToHost, s));
     HIPTRY(hipStreamSynchronize(s));
-    for (int p = 0; p < Np; ++p) {
-        if (nmerged) nmerged[p] = nm[p];
-        if (nnondetect) nnondetect[p] = oc[p] - nm[p];
-    }
     return SCPHD_OK;
 }
 
@@ -1719,9 +1703,9 @@ int scphd_compact(scphd_t* f) {
      * go with them */
     f->gen[1 - f->cur].release();
     for (auto* b : {&f->fit, &f->pre, &f->lik, &f->eta, &f->sw, &f->smu, &f->mw, &f->mmu, &f->mP, &f->kw}) b->release();
-    for (auto* b : {&f->keep, &f->keepscan, &f->ndlist, &f->holes, &f->redo, &f->ndfill, &f->mcnt, &f->knum, &f->kjm, &f->sg,
+    for (auto* b : {&f->keep, &f->ndlist, &f->holes, &f->redo, &f->ndfill, &f->mcnt, &f->knum, &f->kjm, &f->sg,
                     &f->sm, &f->glead, &f->gsta, &f->gend, &f->gmem, &f->gparent2, &f->gblock2, &f->nsurv,
-                    &f->survoff, &f->nmerged, &f->mergeoff, &f->outcnt, &f->ngroups, &f->wparent, &f->wmerged})
+                    &f->survoff, &f->nmerged, &f->mergeoff, &f->nkeep, &f->keepoff, &f->ngroups, &f->wparent, &f->wmerged})
         b->release();
     f->gw2.release();
     f->gpd2.release();
@@ -1747,14 +1731,13 @@ int scphd_reserve(scphd_t* f, int64_t n_gaussians, int32_t max_meas) {
     HIPTRY(f->pre.ensure((int64_t)PP_COUNT * G));
     HIPTRY(f->lik.ensure((int64_t)LK_COUNT * (G + 3)));
     HIPTRY(f->keep.ensure(G));
-    HIPTRY(f->keepscan.ensure(G + 1));
-    HIPTRY(f->redo.ensure(G + 1));
-    HIPTRY(f->ndfill.ensure(G + 1));
+    HIPTRY(f->redo.ensure(G));
+    HIPTRY(f->ndfill.ensure(G));
     HIPTRY(f->ndlist.ensure(G));
     HIPTRY(f->holes.ensure(G));
     HIPTRY(f->wparent.ensure(wave_count(G, (int)Np)));
     HIPTRY(f->wmerged.ensure(wave_count(G + 1, (int)Np)));
-    HIPTRY(f->scantmp.ensure(scan_tmp_size(std::max<int64_t>(G, Np) + 1) + 16));
+    HIPTRY(f->scantmp.ensure(scan_tmp_size(Np + 1) + 16));
     /* the successor table, and the current one keeping its entries, so that
      * the table swaps of later updates and resamplings find both sized */
     HIPTRY(f->gparent2.ensure(G + 1));

@@ -141,8 +141,11 @@ hipError_t launch_prior(hipStream_t s, double* ext, double* pw, int Np, const do
  * (rig of parent p: prig[p]); else `fixed` for every parent */
 /* goff, wave_parent (wave_count(goff[Np], Np) entries, written): the map
  * table's parent per wavefront of k_fit */
+/* an update's counters, zeroed by launch_pose: survivors miscounted, entries
+ * listed in FitArgs::redo and FitArgs::ndfill */
+enum { UC_ERR, UC_REDO, UC_NDFILL, UC_COUNT };
 hipError_t launch_pose(hipStream_t s, const double* ext, double* pose, int Np, int fixed, const int32_t* prig,
-                       const int32_t* rfixed, const int32_t* goff, int32_t* wave_parent);
+                       const int32_t* rfixed, const int32_t* goff, int32_t* wave_parent, int32_t* counters);
 /* wavefronts (of four rows) that take n table entries of Np parents, none of
  * them two parents' */
 int64_t wave_count(int64_t n, int Np);
@@ -230,6 +233,8 @@ struct EtaArgs {
     double* eta;       /* Np*M */
     double* loglik;    /* Np   */
     int32_t* nsurv;    /* Np   */
+    const int32_t* keep; /* per entry: its non-detection term is kept */
+    int32_t* nkeep;      /* Np their numbers */
     int32_t* mcnt;     /* Np*M detection terms kept per (parent, measurement) */
     /* the kept detection terms of a parent in pack order, at kcap p + i:
      * weight, (map index, measurement); knum[p] of them, -1 when there are
@@ -315,10 +320,6 @@ hipError_t launch_goff_remove(hipStream_t s, const int32_t* goff, int P0, int Nr
                               int32_t* goff_out);
 /* x[i] -= Nr where x[i] >= P1 (ancestor indices after a removal), n entries */
 hipError_t launch_index_shift(hipStream_t s, int32_t* x, int64_t n, int P1, int Nr);
-/* out[0..4] (device-visible host memory): off[n], the largest segment of
- * off, the number of segments above limit, *x0, *x1 */
-hipError_t launch_readout(hipStream_t s, const int32_t* off, int n, int32_t limit, const int32_t* x0,
-                          const int32_t* x1, int32_t* out);
 /* *out = the number of NaN entries of w[0, n) */
 hipError_t launch_nan_count(hipStream_t s, const double* w, int n, int32_t* out);
 /* *out = sum over rigs r of (goff[poff[r+1]] - goff[poff[r]]) (moff[r+1] - moff[r]) */
@@ -369,21 +370,17 @@ struct SampleArgs {
 template <typename T>
 hipError_t launch_sample(hipStream_t s, const SampleArgs& a, Clouds<T> dst);
 
-/* mergeoff, wave_parent (wave_count(mergeoff[Np], Np) entries, written): the
- * posterior terms' parent per wavefront of k_sample */
-hipError_t launch_outcount(hipStream_t s, const int32_t* nmerged, const int32_t* goff, const int32_t* keepscan,
-                           int Np, int32_t* outcnt, const int32_t* mergeoff, int32_t* wave_parent);
-/* ndlist[keepscan[g]] = g for the kept entries; with holes, also
- * holes[g - keepscan[g]] = g for the dropped ones */
-hipError_t launch_ndlist(hipStream_t s, const int32_t* keep, const int32_t* keepscan, int64_t Ng, int32_t* ndlist,
-                         int32_t* holes = nullptr);
+/* the kept entries (at keepoff[p] on for parent p) in ndlist, the blocks of the
+ * others in holes, and the posterior's wave_parent */
+hipError_t launch_lists(hipStream_t s, const int32_t* keep, const int32_t* keepoff, const int32_t* goff, int Np,
+                        int32_t* ndlist, int32_t* holes, const int32_t* mergeoff, int32_t* wave_parent);
 
 struct TableArgs {
     const int32_t* outoff;   /* Np+1 */
     const int32_t* mergeoff; /* Np+1 */
     const int32_t* survoff;  /* Np+1 */
     const int32_t* goff;     /* input table offsets */
-    const int32_t* keepscan; /* Ng+1 */
+    const int32_t* keepoff; /* Np+1 */
     const int32_t* ndlist;
     const double* mw;
     const double* gw;        /* input table weights */
@@ -420,7 +417,6 @@ struct ResampleArgs {
     const NoiseKey* keys = nullptr; /* ensemble: per rig, or nullptr */
     const uint32_t* sbase = nullptr; /* ensemble: per rig, the handle's step counts at joining (SC_COUNT each) */
     uint64_t rstep;
-    int32_t* flag;  /* out: 1 if any rig resampled (zero before the launch) */
     int32_t* rflag; /* out: per rig, 1 if resampled */
     int32_t* amax;  /* scratch, per rig */
     double* neff;   /* out: per rig */
@@ -449,10 +445,17 @@ template <typename T>
 hipError_t launch_inject(hipStream_t s, const double* in, int64_t Ng, int S, Clouds<T> dst);
 
 /* ---- scan ---- */
-/* out[0..n] = exclusive prefix sums of in[0..n), out[n] = total.
- * tmp needs scan_tmp_size(n) ints. */
-int64_t scan_tmp_size(int64_t n);
-hipError_t launch_scan(hipStream_t s, const int32_t* in, int32_t* out, int64_t n, int32_t* tmp);
+int64_t scan_tmp_size(int64_t n); /* ints of the scans' tmp */
+/* off[0, n] = exclusive sums of in[0, n) (tmp: scan_tmp_size(n)), and into host
+ * memory: out[0] their end, [1] the largest value, [2] the values over limit
+ * (when positive), [3] the largest of x0[0, n0), [4] x1 (may be null) */
+hipError_t launch_scan_readout(hipStream_t s, const int32_t* in, int32_t* off, int n, int32_t* tmp, int32_t limit,
+                               const int32_t* x0, int n0, const int32_t* x1, int32_t* out);
+/* the same of nmerged and nkeep into mergeoff and keepoff, of their sums into
+ * off and out; out[3]: the end of mergeoff */
+hipError_t launch_outputs(hipStream_t s, const int32_t* nmerged, const int32_t* nkeep, int n, int32_t* tmp,
+                          int32_t limit, const int32_t* x1, int32_t* mergeoff, int32_t* keepoff, int32_t* off,
+                          int32_t* out);
 
 }  // namespace scphd
 

@@ -187,10 +187,13 @@ __device__ inline void write_wave_parents(int off0, int off1, int p, int lane, i
 
 /* Camera used by an update: the parent's extrinsics, or all-zero extrinsics
  * for the fixed camera (src/scphdcameracalibration.cu:1167-1176); and the map
- * table's wave_parent.  One wavefront per parent. */
+ * table's wave_parent; and the update's counters zeroed.  One wavefront per
+ * parent. */
 __global__ __launch_bounds__(256) void k_pose(const double* ext, double* pose, int Np, int fixed, const int32_t* prig,
-                                              const int32_t* rfixed, const int32_t* goff, int32_t* wave_parent) {
+                                              const int32_t* rfixed, const int32_t* goff, int32_t* wave_parent,
+                                              int32_t* counters) {
     const int p = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (blockIdx.x == 0 && threadIdx.x < UC_COUNT) counters[threadIdx.x] = 0;
     if (p >= Np) return;
     write_wave_parents(goff[p], goff[p + 1], p, lane, wave_parent);
     if (lane != 0) return;
@@ -1438,13 +1441,19 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_
         }
     }
     double swg = 0.0;
-    for (int j = t; j < G; j += NT) swg += a.gw[g0 + j];
+    int nd = 0;
+    for (int j = t; j < G; j += NT) {
+        swg += a.gw[g0 + j];
+        nd += a.keep[g0 + j];
+    }
     const double se = block_sum(eta_sum, red);
     const double sg = block_sum(swg, red);
     const double sc = block_sum((double)cnt, red);
+    const double sn = block_sum((double)nd, red);
     if (t == 0) {
         a.loglik[p] = se + sg;
         a.nsurv[p] = (int32_t)sc;
+        a.nkeep[p] = (int32_t)sn;
         a.knum[p] = lists && kept <= a.kcap ? kept : -1;
     }
 }
@@ -2690,30 +2699,30 @@ __global__ __launch_bounds__(256) void k_sample(SampleKernArgs<T> ka) {
 /* -------------------------------------------------------- map assembly */
 /* Map sizes after the update, and the posterior terms' wave_parent.  One
  * wavefront per parent. */
-__global__ __launch_bounds__(256) void k_outcount(const int32_t* nmerged, const int32_t* goff, const int32_t* keepscan,
-                                                  int Np, int32_t* outcnt, const int32_t* mergeoff,
-                                                  int32_t* wave_parent) {
+/* The kept non-detection entries of a parent at keepoff[p] on, ndlist, the
+ * others' blocks in holes (at the entry's index less the kept ones before
+ * it), and the posterior's wave_parent.  One wavefront per parent. */
+__global__ __launch_bounds__(256) void k_lists(const int32_t* keep, const int32_t* keepoff, const int32_t* goff,
+                                               int Np, int32_t* ndlist, int32_t* holes, const int32_t* mergeoff,
+                                               int32_t* wave_parent) {
     const int p = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (p >= Np) return;
     write_wave_parents(mergeoff[p], mergeoff[p + 1], p, lane, wave_parent);
-    if (lane == 0) outcnt[p] = nmerged[p] + (keepscan[goff[p + 1]] - keepscan[goff[p]]);
+    const int g1 = goff[p + 1];
+    int k0 = keepoff[p];
+    for (int g0 = goff[p]; g0 < g1; g0 += 64) {
+        const int g = g0 + lane;
+        const bool in = g < g1, kept = in && keep[g] != 0;
+        const uint64_t b = __ballot(kept);
+        const int k = k0 + __popcll(b & ((1ull << lane) - 1ull));
+        if (kept)
+            ndlist[k] = g;
+        else if (in)
+            holes[g - k] = g;
+        k0 += __popcll(b);
+    }
 }
 
-__global__ void k_ndlist(const int32_t* keep, const int32_t* keepscan, int64_t Ng, int32_t* ndlist,
-                         int32_t* holes) {
-    const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= Ng) return;
-    if (keep[g])
-        ndlist[keepscan[g]] = (int32_t)g;
-    else if (holes)
-        holes[g - keepscan[g]] = (int32_t)g;
-}
-
-
-/* New map table per parent: [merged posterior Gaussians | kept
- * non-detection Gaussians in input order] (recombineNonDetections,
- * src/scphdcameracalibration.cu:1422-1574, weights w (1 - pd) for the
- * non-detection terms, :1314-1318). */
 __global__ void k_table(TableArgs a) {
     const int64_t o = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (o >= a.Nout) return;
@@ -2725,7 +2734,7 @@ __global__ void k_table(TableArgs a) {
         a.gwo[o] = a.mw[(int64_t)a.survoff[p] + j];
         a.gpd[o] = 1.0f;
     } else {
-        const int g = a.ndlist[a.keepscan[a.goff[p]] + (j - K)];
+        const int g = a.ndlist[a.keepoff[p] + (j - K)];
         const double pdg = a.fit[(int64_t)FP_PD * a.Ng_in + g];
         a.gblock[o] = (int32_t)(a.nd_base + g);
         a.gwo[o] = a.gw[g] * (1 - pdg);
@@ -2770,7 +2779,6 @@ __global__ __launch_bounds__(1024) void k_resample(ResampleArgs a) {
     if (t == 0) {
         a.neff[rig] = neff;
         a.rflag[rig] = go ? 1 : 0;
-        if (go) atomicOr(a.flag, 1); /* any rig resampled; zero before the launch */
     }
     if (!go) return;
     /* first index of the maximum of exp(w) */
@@ -2857,7 +2865,8 @@ __global__ __launch_bounds__(1024) void k_resample(ResampleArgs a) {
 __global__ __launch_bounds__(256) void k_resample_draw(ResampleArgs a) {
     __shared__ int s_anc[256];
     const int t = threadIdx.x, j0 = blockIdx.x * 256, n = min(256, a.Np - j0);
-    const bool any = *a.flag != 0;
+    int any = 0;
+    for (int r = t; r < a.nrigs; r += 256) any |= a.rflag[r];
     if (t < n) {
         const int g = j0 + t;
         const int rig = a.prig ? a.prig[g] : 0;
@@ -2888,8 +2897,7 @@ __global__ __launch_bounds__(256) void k_resample_draw(ResampleArgs a) {
         a.newcnt[g] = a.goff[anc + 1] - a.goff[anc];
         s_anc[t] = anc;
     }
-    if (!any) return; /* uniform */
-    __syncthreads();
+    if (!__syncthreads_or(any)) return;
     for (int i = t; i < 12 * n; i += 256) a.ext_tmp[(int64_t)j0 * 12 + i] = a.ext[(int64_t)s_anc[i / 12] * 12 + i % 12];
 }
 
@@ -2994,6 +3002,115 @@ __global__ void k_inject(const double* in, int64_t Ng, int S, Clouds<T> dst) {
 }
 
 /* ----------------------------------------------------------------- scan */
+/* Up to SCAN_ONE values in one workgroup: a launch instead of the three or
+ * four of the tiled scan and the read-out (256 values: 12.4 us in three
+ * launches, 7.4 in one; 4096: 22.8 in four, 9.7 in one; 16384: 23.6 and 21,
+ * and 45 for the update's two scans, the time of their eight launches). */
+static constexpr int SCAN_ONE_T = 1024, SCAN_ONE_I = 8, SCAN_ONE = SCAN_ONE_T * SCAN_ONE_I;
+
+/* SCAN_ONE_I consecutive values a thread, from base on */
+__device__ inline int scan_load(const int32_t* in, int n, int base, int (&v)[SCAN_ONE_I]) {
+    int s = 0;
+#pragma unroll
+    for (int i = 0; i < SCAN_ONE_I; ++i) {
+        v[i] = base + i < n ? in[base + i] : 0;
+        s += v[i];
+    }
+    return s;
+}
+
+/* what a read-out leaves in host memory: the offsets' end, the largest
+ * segment, the segments over limit, the largest of x0[0, n0) and x1 */
+__device__ inline void read_out(int total, int mx, int over, const int32_t* x0, int n0, const int32_t* x1,
+                                volatile int32_t* out) {
+    __shared__ int smax[16], scnt[16];
+    int any = 0;
+    for (int i = threadIdx.x; i < n0; i += blockDim.x) any = max(any, x0[i]);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        mx = max(mx, __shfl_xor(mx, o, 64));
+        over += __shfl_xor(over, o, 64);
+    }
+    if ((threadIdx.x & 63) == 0) {
+        smax[threadIdx.x >> 6] = mx;
+        scnt[threadIdx.x >> 6] = over;
+    }
+    __shared__ int s_any;
+    if (threadIdx.x == 0) s_any = 0;
+    __syncthreads();
+    if (any) atomicMax(&s_any, any);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < (int)(blockDim.x >> 6); ++w) {
+            mx = max(mx, smax[w]);
+            over += scnt[w];
+        }
+        out[0] = total;
+        out[1] = mx;
+        out[2] = over;
+        out[3] = s_any;
+        out[4] = x1 ? *x1 : 0;
+    }
+}
+
+__global__ __launch_bounds__(SCAN_ONE_T) void k_scan_readout(const int32_t* in, int32_t* off, int n, int32_t limit,
+                                                             const int32_t* x0, int n0, const int32_t* x1,
+                                                             volatile int32_t* out) {
+    __shared__ int sh[SCAN_ONE_T / 64];
+    const int items = (n + SCAN_ONE_T - 1) / SCAN_ONE_T; /* a thread */
+    const int base = threadIdx.x * items, end = min(n, base + items);
+    int v[SCAN_ONE_I], tot, mx = 0, over = 0;
+    int o = block_exscan(scan_load(in, end, base, v), sh, &tot);
+#pragma unroll
+    for (int i = 0; i < SCAN_ONE_I; ++i) {
+        if (base + i < end) off[base + i] = o;
+        o += v[i];
+        mx = max(mx, v[i]);
+        over += limit > 0 && v[i] > limit ? 1 : 0;
+    }
+    if (threadIdx.x == 0) off[n] = tot;
+    read_out(tot, mx, over, x0, n0, x1, out);
+}
+
+/* The update's output offsets: mergeoff of the merged terms' counts, keepoff
+ * of the kept non-detection terms', off of both. */
+__global__ __launch_bounds__(SCAN_ONE_T) void k_outputs(const int32_t* nmerged, const int32_t* nkeep, int n,
+                                                        int32_t limit, const int32_t* x1, int32_t* mergeoff,
+                                                        int32_t* keepoff, int32_t* off, volatile int32_t* out) {
+    __shared__ int sh[SCAN_ONE_T / 64];
+    __shared__ int s_merged;
+    const int items = (n + SCAN_ONE_T - 1) / SCAN_ONE_T;
+    const int base = threadIdx.x * items, end = min(n, base + items);
+    int v[SCAN_ONE_I], w[SCAN_ONE_I], tv, tw, mx = 0, over = 0;
+    int ov = block_exscan(scan_load(nmerged, end, base, v), sh, &tv);
+    int ow = block_exscan(scan_load(nkeep, end, base, w), sh, &tw);
+#pragma unroll
+    for (int i = 0; i < SCAN_ONE_I; ++i) {
+        if (base + i < end) {
+            mergeoff[base + i] = ov;
+            keepoff[base + i] = ow;
+            off[base + i] = ov + ow;
+        }
+        ov += v[i];
+        ow += w[i];
+        mx = max(mx, v[i] + w[i]);
+        over += limit > 0 && v[i] + w[i] > limit ? 1 : 0;
+    }
+    if (threadIdx.x == 0) {
+        mergeoff[n] = s_merged = tv;
+        keepoff[n] = tw;
+        off[n] = tv + tw;
+    }
+    __syncthreads();
+    read_out(tv + tw, mx, over, &s_merged, 1, x1, out);
+}
+
+/* off = mergeoff + keepoff, n + 1 of them */
+__global__ void k_add_offsets(const int32_t* mergeoff, const int32_t* keepoff, int n, int32_t* off) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i <= n) off[i] = mergeoff[i] + keepoff[i];
+}
+
 static constexpr int SCAN_T = 256, SCAN_I = 8, SCAN_TILE = SCAN_T * SCAN_I;
 
 __global__ __launch_bounds__(SCAN_T) void k_scan_tiles(const int32_t* in, int32_t* out, int64_t n, int32_t* sums) {
@@ -3066,9 +3183,9 @@ hipError_t launch_scale(hipStream_t s, double* x, int64_t n, double a) {
 int64_t wave_count(int64_t n, int Np) { return n / 4 + Np; }
 
 hipError_t launch_pose(hipStream_t s, const double* ext, double* pose, int Np, int fixed, const int32_t* prig,
-                       const int32_t* rfixed, const int32_t* goff, int32_t* wave_parent) {
+                       const int32_t* rfixed, const int32_t* goff, int32_t* wave_parent, int32_t* counters) {
     if (rfixed && !prig) return hipErrorInvalidValue;
-    k_pose<<<nblocks(Np, 4), 256, 0, s>>>(ext, pose, Np, fixed, prig, rfixed, goff, wave_parent);
+    k_pose<<<nblocks(Np, 4), 256, 0, s>>>(ext, pose, Np, fixed, prig, rfixed, goff, wave_parent, counters);
     LAUNCH_CHECK();
 }
 
@@ -3214,19 +3331,11 @@ hipError_t launch_sample(hipStream_t s, const SampleArgs& a, Clouds<T> dst) {
     LAUNCH_CHECK();
 }
 
-hipError_t launch_outcount(hipStream_t s, const int32_t* nmerged, const int32_t* goff, const int32_t* keepscan,
-                           int Np, int32_t* outcnt, const int32_t* mergeoff, int32_t* wave_parent) {
-    k_outcount<<<nblocks(Np, 4), 256, 0, s>>>(nmerged, goff, keepscan, Np, outcnt, mergeoff, wave_parent);
+hipError_t launch_lists(hipStream_t s, const int32_t* keep, const int32_t* keepoff, const int32_t* goff, int Np,
+                        int32_t* ndlist, int32_t* holes, const int32_t* mergeoff, int32_t* wave_parent) {
+    k_lists<<<nblocks(Np, 4), 256, 0, s>>>(keep, keepoff, goff, Np, ndlist, holes, mergeoff, wave_parent);
     LAUNCH_CHECK();
 }
-
-hipError_t launch_ndlist(hipStream_t s, const int32_t* keep, const int32_t* keepscan, int64_t Ng, int32_t* ndlist,
-                         int32_t* holes) {
-    if (Ng <= 0) return hipSuccess;
-    k_ndlist<<<nblocks(Ng, 256), 256, 0, s>>>(keep, keepscan, Ng, ndlist, holes);
-    LAUNCH_CHECK();
-}
-
 hipError_t launch_table(hipStream_t s, const TableArgs& a) {
     if (a.Nout <= 0) return hipSuccess;
     k_table<<<nblocks(a.Nout, 256), 256, 0, s>>>(a);
@@ -3244,41 +3353,17 @@ hipError_t launch_resample(hipStream_t s, const ResampleArgs& a) {
  * out[0] = off[n], out[1] = the largest segment off[p + 1] - off[p],
  * out[2] = the number of segments above `limit` (0 when limit <= 0),
  * out[3] = *x0 and out[4] = *x1 (0 for a null pointer).  One workgroup. */
-__global__ __launch_bounds__(1024) void k_readout(const int32_t* off, int n, int32_t limit, const int32_t* x0,
+__global__ __launch_bounds__(1024) void k_readout(const int32_t* off, int n, int32_t limit, const int32_t* x0, int n0,
                                                   const int32_t* x1, volatile int32_t* out) {
-    __shared__ int smax[16], scnt[16];
     int mx = 0, c = 0;
     for (int p = threadIdx.x; p < n; p += blockDim.x) {
         const int seg = off[p + 1] - off[p];
         mx = max(mx, seg);
         c += (limit > 0 && seg > limit) ? 1 : 0;
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        mx = max(mx, __shfl_xor(mx, o, 64));
-        c += __shfl_xor(c, o, 64);
-    }
-    if ((threadIdx.x & 63) == 0) {
-        smax[threadIdx.x >> 6] = mx;
-        scnt[threadIdx.x >> 6] = c;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int w = 1; w < (int)(blockDim.x >> 6); ++w) {
-            mx = max(mx, smax[w]);
-            c += scnt[w];
-        }
-        out[0] = off[n];
-        out[1] = mx;
-        out[2] = c;
-        out[3] = x0 ? *x0 : 0;
-        out[4] = x1 ? *x1 : 0;
-    }
+    read_out(off[n], mx, c, x0, n0, x1, out);
 }
 
-/* out = the number of NaN entries of w[0, n) (checkStuff,
- * src/scphdcameracalibration.cu:812-821, without the host copy).  One
- * workgroup. */
 __global__ __launch_bounds__(1024) void k_nan_count(const double* w, int n, volatile int32_t* out) {
     __shared__ int sc[16];
     int c = 0;
@@ -3317,11 +3402,6 @@ hipError_t launch_nan_count(hipStream_t s, const double* w, int n, int32_t* out)
     LAUNCH_CHECK();
 }
 
-hipError_t launch_readout(hipStream_t s, const int32_t* off, int n, int32_t limit, const int32_t* x0,
-                          const int32_t* x1, int32_t* out) {
-    k_readout<<<1, 1024, 0, s>>>(off, n, limit, x0, x1, out);
-    LAUNCH_CHECK();
-}
 
 hipError_t launch_resample_commit(hipStream_t s, double* ext, const double* ext_tmp, double* pw, int32_t* anc_out,
                                   const int32_t* anc, int N, int go) {
@@ -3397,11 +3477,35 @@ hipError_t launch_inject(hipStream_t s, const double* in, int64_t Ng, int S, Clo
 
 int64_t scan_tmp_size(int64_t n) { return (n + SCAN_TILE - 1) / SCAN_TILE + 1; }
 
-hipError_t launch_scan(hipStream_t s, const int32_t* in, int32_t* out, int64_t n, int32_t* tmp) {
+static void scan(hipStream_t s, const int32_t* in, int32_t* out, int64_t n, int32_t* tmp) {
     const int64_t nb = (n + SCAN_TILE - 1) / SCAN_TILE;
     if (nb > 0) k_scan_tiles<<<(unsigned)nb, SCAN_T, 0, s>>>(in, out, n, tmp);
     k_scan_sums<<<1, SCAN_T, 0, s>>>(tmp, nb, out + n);
     if (nb > 1) k_scan_add<<<nblocks(n, 256), 256, 0, s>>>(out, n, tmp);
+}
+
+hipError_t launch_scan_readout(hipStream_t s, const int32_t* in, int32_t* off, int n, int32_t* tmp, int32_t limit,
+                               const int32_t* x0, int n0, const int32_t* x1, int32_t* out) {
+    if (n <= SCAN_ONE) {
+        k_scan_readout<<<1, SCAN_ONE_T, 0, s>>>(in, off, n, limit, x0, n0, x1, out);
+    } else {
+        scan(s, in, off, n, tmp);
+        k_readout<<<1, 1024, 0, s>>>(off, n, limit, x0, n0, x1, out);
+    }
+    LAUNCH_CHECK();
+}
+
+hipError_t launch_outputs(hipStream_t s, const int32_t* nmerged, const int32_t* nkeep, int n, int32_t* tmp,
+                          int32_t limit, const int32_t* x1, int32_t* mergeoff, int32_t* keepoff, int32_t* off,
+                          int32_t* out) {
+    if (n <= SCAN_ONE) {
+        k_outputs<<<1, SCAN_ONE_T, 0, s>>>(nmerged, nkeep, n, limit, x1, mergeoff, keepoff, off, out);
+    } else {
+        scan(s, nmerged, mergeoff, n, tmp);
+        scan(s, nkeep, keepoff, n, tmp);
+        k_add_offsets<<<nblocks((int64_t)n + 1, 256), 256, 0, s>>>(mergeoff, keepoff, n, off);
+        k_readout<<<1, 1024, 0, s>>>(off, n, limit, mergeoff + n, 1, x1, out);
+    }
     LAUNCH_CHECK();
 }
 
