@@ -1463,12 +1463,14 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_
  * reference's pack order (updateKernel, src/kernels.cu:608-659: detection
  * terms measurement-major, then births).  The detection terms come from
  * k_eta's list, one a thread, so that the gathers of their records are in
- * flight together and the survivors are written as one stretch (11.9 ms over
- * ten frames of 4096 parents, 200 landmarks, when a thread found and wrote
- * its measurement's terms one after the other); a parent without a list has
- * its map swept. */
+ * flight together, and the means go through LDS to be stored as one stretch.
+ * Ten frames of 4096 parents, 200 landmarks: 11.9 ms when a thread found and
+ * wrote its measurement's terms one after the other, 4.4 from the list with
+ * each thread storing its 48 bytes, 1.9 so.  A parent without a list has its
+ * map swept. */
 __global__ __launch_bounds__(NT) void k_survivors(SurvArgs a) {
     __shared__ int sh[8];
+    __shared__ double s_mu[6 * NT]; /* means, stored as one stretch */
     const EtaArgs& e = a.e;
     const int p = blockIdx.x;
     const int t = threadIdx.x;
@@ -1496,9 +1498,22 @@ __global__ __launch_bounds__(NT) void k_survivors(SurvArgs a) {
     };
     const int kn = e.knum[p];
     if (kn >= 0) {
-        for (int i = t; i < kn; i += NT) {
-            const int2 jm = *(const int2*)(e.kjm + 2 * (p * e.kcap + i));
-            put(i, jm.x, jm.y, e.zu[zb + jm.y], e.zv[zb + jm.y], e.kw[p * e.kcap + i]);
+        for (int i0 = 0; i0 < kn; i0 += NT) {
+            const int i = i0 + t, n = min(min(NT, kn - i0), cap - i0);
+            if (t < n) {
+                const int2 jm = *(const int2*)(e.kjm + 2 * (p * e.kcap + i));
+                const int64_t gi = g0 + jm.x;
+                const double* mk = e.pre + PP_MK * e.Ng + gi * PP_MK_LEN;
+                const double i0u = e.zu[zb + jm.y] - mk[0], i1v = e.zv[zb + jm.y] - mk[1];
+                a.sw[base + i] = e.kw[p * e.kcap + i];
+                a.sg[base + i] = (int32_t)gi;
+                a.sm[base + i] = jm.y;
+#pragma unroll
+                for (int c = 0; c < 6; ++c) s_mu[6 * t + c] = mk[c] + i0u * mk[6 + c] + i1v * mk[12 + c];
+            }
+            __syncthreads();
+            for (int q = t; q < 6 * n; q += NT) a.smu[(base + i0) * 6 + q] = s_mu[q];
+            __syncthreads();
         }
         run = kn;
     } else {
@@ -2292,7 +2307,7 @@ __global__ __launch_bounds__(128) void k_merge_moments(MergeArgs a) {
     for (int e = st; e < en; ++e) {
         const int64_t si = sbase + a.gmem[sbase + e];
         const double w = a.sw[si];
-        const int g = a.sg[si];
+        const double* Pt = term_P_all(a, a.sg[si]);
         double dl[6];
 #pragma unroll
         for (int c = 0; c < 6; ++c) dl[c] = mu[c] - a.smu[(si) * 6 + c];
@@ -2300,8 +2315,7 @@ __global__ __launch_bounds__(128) void k_merge_moments(MergeArgs a) {
         for (int r = 0; r < 6; ++r)
 #pragma unroll
             for (int c = 0; c <= r; ++c) {
-                const double Pe = term_P(a, g, pidx(r, c));
-                P[pidx(r, c)] += w * (Pe + dl[c] * dl[r]);
+                P[pidx(r, c)] += w * (Pt[pidx(r, c)] + dl[c] * dl[r]);
             }
     }
 #pragma unroll
