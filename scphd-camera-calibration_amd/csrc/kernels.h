@@ -249,6 +249,7 @@ struct EtaArgs {
     const DisparityMeasurementModel* rig_meas = nullptr;
     int sweep = 0;     /* nonzero: every pair is evaluated, no windows (verification) */
     int mask_stride = 0; /* set by launch_eta */
+    int list;          /* terms of a list, a power of two; both set by launch_eta */
 };
 static constexpr int ETA_NCAND = 8; /* kept detection terms a measurement that the lists have room for */
 static constexpr int ETA_HEAVY = 2048; /* the normal value of scphd_debug_set_limits' eta_heavy_cap */

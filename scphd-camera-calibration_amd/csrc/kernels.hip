@@ -1130,8 +1130,9 @@ __device__ inline double max_val(unsigned long long k) {
  * Bound: latency (LDS and the records' gathers), which is why the lists
  * spread the uneven terms over all lanes.  Ten frames of 4096 parents, 200
  * landmarks: 18.0 ms when every pair was evaluated twice and measurements
- * with more than eight candidate terms (one in seven) swept the map again. */
-static constexpr int ETA_BINS = 128, ETA_CHUNK = 2048, ETA_LIST = 1024;
+ * with more than eight candidate terms (one in seven) swept the map again,
+ * 9.6 so. */
+static constexpr int ETA_BINS = 128, ETA_CHUNK = 2048;
 static constexpr double ETA_DROP = 60.0;
 
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_eta(EtaArgs a) {
@@ -1144,14 +1145,13 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_
     __shared__ unsigned long long s_any[NT]; /* per place: its mask's non-zero words */
     __shared__ int s_cnt[NT];                /* per measurement: terms kept */
     __shared__ int s_off[ETA_BINS + 1], s_cur[ETA_BINS];
-    __shared__ union {
-        double rec[NT / 64][32 * REC];       /* per wavefront: the records of a word of Gaussians */
-        struct {
-            double e[ETA_LIST];              /* a list's terms: exp(l - max) */
-            uint32_t pair[ETA_LIST];         /* place << 16 | map index in the chunk */
-        } l;
-    } u;
-    extern __shared__ uint32_t s_mask[];     /* per place, a.mask_stride words */
+    /* a.list terms of a list: place << 16 | map index in the chunk, and in the
+     * same place then exp(l - max); in step 2 the wavefronts' records of a
+     * word of Gaussians.  Then per place a.mask_stride words of its mask. */
+    extern __shared__ double s_dyn[];
+    double* const s_e = s_dyn;
+    uint32_t* const s_pair = (uint32_t*)s_dyn;
+    uint32_t* const s_mask = (uint32_t*)(s_dyn + a.list);
     const int p = blockIdx.x;
     const int t = threadIdx.x, lane = t & 63;
     const int64_t g0 = a.goff[p];
@@ -1249,7 +1249,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_
         double T = 0.0;
         const int nq = s_off[ETA_BINS];
         /* the terms in this thread's row of the masks from (words, bits) on,
-         * ascending: fills the list's places up to ETA_LIST from `pos` on */
+         * ascending: fills the list's places up to `end` from `pos` on */
         unsigned long long words_left = 0;
         uint32_t bits_left = 0;
         int word = 0;
@@ -1270,7 +1270,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_
                     bits_left = s_mask[place * a.mask_stride + word];
                     continue;
                 }
-                u.l.pair[pos & (ETA_LIST - 1)] =
+                s_pair[2 * (pos & (a.list - 1))] =
                     (uint32_t)place << 16 | (uint32_t)(32 * word + __builtin_ctz(bits_left));
                 bits_left &= bits_left - 1;
                 ++pos;
@@ -1296,7 +1296,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_
             __syncthreads();
             for (int w = __builtin_amdgcn_readfirstlane(t >> 6); w < words; w += NT / 64) {
                 const int jw = c0 + 32 * w, n = min(32, c0 + cn - jw);
-                double* const wr = u.rec[t >> 6];
+                double* const wr = s_dyn + (t >> 6) * (32 * REC);
                 /* the word's windows, a Gaussian a lane: blocks met */
                 int blocks = 0;
                 if (lane < n) {
@@ -1344,23 +1344,23 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_
             int total, n = row_begin();
             const int first = block_exscan(n, sh, &total);
             int pos = first;
-            for (int l0 = 0; l0 < total; l0 += ETA_LIST) {
-                row_list(pos, l0 + ETA_LIST);
+            for (int l0 = 0; l0 < total; l0 += a.list) {
+                row_list(pos, l0 + a.list);
                 __syncthreads();
-                const int ln = min(ETA_LIST, total - l0);
+                const int ln = min(a.list, total - l0);
                 for (int q = t; q < ln; q += NT) {
-                    const uint32_t pr = u.l.pair[q];
+                    const uint32_t pr = s_pair[2 * q];
                     const int pl = (int)(pr >> 16), j = (int)(pr & 0xFFFFu);
                     double rec[LK_COUNT];
                     load_rec(c0 + j, rec);
                     const double x = det_lw(rec, s_zu[pl], s_zv[pl]) - max_val(s_max[s_m[pl]]);
-                    u.l.e[q] = x > -746.0 ? exp_nonpos(x) : 0.0;
+                    s_e[q] = x > -746.0 ? exp_nonpos(x) : 0.0;
                     if (!(x > cgate)) atomicAnd(&s_mask[pl * a.mask_stride + (j >> 5)], ~(1u << (j & 31)));
                 }
                 __syncthreads();
                 const int q1 = min(first + n - l0, ln);
                 for (int q = max(first - l0, 0); q < q1; ++q) {
-                    const double e = u.l.e[q];
+                    const double e = s_e[q];
                     if (!met && e == 1.0)
                         met = true;
                     else
@@ -1382,43 +1382,46 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_
         if (lists && G > 0) {
             int total, n = row_begin();
             int pos = block_exscan(n, sh, &total);
-            for (int l0 = 0; l0 < total; l0 += ETA_LIST) {
-                row_list(pos, l0 + ETA_LIST);
+            for (int l0 = 0; l0 < total; l0 += a.list) {
+                row_list(pos, l0 + a.list);
                 __syncthreads();
-                constexpr int E = ETA_LIST / NT; /* consecutive terms of a thread */
-                double w[E];
-                int mine = 0;
+                constexpr int E = 4; /* consecutive terms of a thread */
+                for (int b0 = 0; b0 < min(a.list, total - l0); b0 += E * NT) {
+                    double w[E];
+                    uint32_t pr[E];
+                    int mine = 0;
 #pragma unroll
-                for (int i = 0; i < E; ++i) {
-                    const int q = E * t + i;
-                    w[i] = -1.0; /* not kept */
-                    if (l0 + q >= total) continue;
-                    const uint32_t pr = u.l.pair[q];
-                    const int pl = (int)(pr >> 16), sl = s_m[pl];
-                    double rec[LK_COUNT];
-                    load_rec((int)(pr & 0xFFFFu), rec);
-                    const double x = det_lw(rec, s_zu[pl], s_zv[pl]) - __longlong_as_double((long long)s_max[sl]);
-                    if (!(x > a.lw_gate)) continue;
-                    const double wx = exp(x);
-                    if (!(wx >= a.min_weight)) continue;
-                    w[i] = wx;
-                    ++mine;
-                    atomicAdd(&s_cnt[sl], 1);
-                }
-                int k, kn;
-                k = kept + block_exscan(mine, sh, &kn);
-#pragma unroll
-                for (int i = 0; i < E; ++i)
-                    if (w[i] >= 0.0) {
-                        if (k < a.kcap) {
-                            const uint32_t pr = u.l.pair[E * t + i];
-                            a.kw[p * a.kcap + k] = w[i];
-                            *(int2*)(a.kjm + 2 * (p * a.kcap + k)) =
-                                int2{(int)(pr & 0xFFFFu), r * NT + s_m[pr >> 16]};
-                        }
-                        ++k;
+                    for (int i = 0; i < E; ++i) {
+                        const int q = b0 + E * t + i;
+                        w[i] = -1.0; /* not kept */
+                        pr[i] = 0;
+                        if (l0 + q >= total) continue;
+                        pr[i] = s_pair[2 * q];
+                        const int pl = (int)(pr[i] >> 16), sl = s_m[pl];
+                        double rec[LK_COUNT];
+                        load_rec((int)(pr[i] & 0xFFFFu), rec);
+                        const double x = det_lw(rec, s_zu[pl], s_zv[pl]) - __longlong_as_double((long long)s_max[sl]);
+                        if (!(x > a.lw_gate)) continue;
+                        const double wx = exp(x);
+                        if (!(wx >= a.min_weight)) continue;
+                        w[i] = wx;
+                        ++mine;
+                        atomicAdd(&s_cnt[sl], 1);
                     }
-                kept += kn;
+                    int kn;
+                    int k = kept + block_exscan(mine, sh, &kn);
+#pragma unroll
+                    for (int i = 0; i < E; ++i)
+                        if (w[i] >= 0.0) {
+                            if (k < a.kcap) {
+                                a.kw[p * a.kcap + k] = w[i];
+                                *(int2*)(a.kjm + 2 * (p * a.kcap + k)) =
+                                    int2{(int)(pr[i] & 0xFFFFu), r * NT + s_m[pr[i] >> 16]};
+                            }
+                            ++k;
+                        }
+                    kept += kn;
+                }
                 __syncthreads();
             }
             __syncthreads();
@@ -3282,9 +3285,16 @@ hipError_t launch_precompute(hipStream_t s, const double* fit, const double* gw,
 }
 
 hipError_t launch_eta(hipStream_t s, EtaArgs a, int max_map) {
-    /* an odd stride: a word of all places lies in all banks */
+    /* an odd stride: a word of all places lies in all banks.  The list as
+     * long as two workgroups of a CU's 160 KB allow (the kernel's own arrays
+     * take 11 each): each round of a list costs the walk of its rows' masks by
+     * few lanes (ten frames of 4096 parents, 200 landmarks: 11.6 ms with 1024
+     * terms, 10.5 with 2048, 9.6 with 4096; a denser scene, where 4096 leave
+     * room for one: 10.7, 8.5, 10.8). */
     a.mask_stride = ((std::min(max_map, ETA_CHUNK) + 31) / 32) | 1;
-    k_eta<<<a.Np, NT, (size_t)std::min(std::max(a.M, 1), NT) * a.mask_stride * sizeof(uint32_t), s>>>(a);
+    const size_t mask = (size_t)std::min(std::max(a.M, 1), NT) * a.mask_stride * sizeof(uint32_t);
+    a.list = mask + 4096 * sizeof(double) <= 68 * 1024 ? 4096 : 2048;
+    k_eta<<<a.Np, NT, a.list * sizeof(double) + mask, s>>>(a);
     LAUNCH_CHECK();
 }
 
