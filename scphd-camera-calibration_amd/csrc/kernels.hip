@@ -2473,14 +2473,38 @@ __global__ __launch_bounds__(1024) void k_parent_weights(double* pw, const doubl
         loglik += poff[blockIdx.x];
         Np = poff[blockIdx.x + 1] - poff[blockIdx.x];
     }
+    /* the first few values of a thread are held over the passes (three
+     * logarithms and two exponentials a parent otherwise: 4096 parents 19 us,
+     * 10 held; sixteen held cost registers that a busy CU does not have) */
+    constexpr int HELD = 4;
+    double v[HELD];
     double mx = -INFINITY;
-    for (int p = threadIdx.x; p < Np; p += blockDim.x) mx = fmax(mx, safe_log(pw[p]) + loglik[p]);
+    const int p1 = threadIdx.x + HELD * blockDim.x;
+#pragma unroll
+    for (int k = 0; k < HELD; ++k) {
+        const int p = threadIdx.x + k * blockDim.x;
+        v[k] = p < Np ? safe_log(pw[p]) + loglik[p] : -INFINITY;
+        mx = fmax(mx, v[k]);
+    }
+    for (int p = p1; p < Np; p += blockDim.x) mx = fmax(mx, safe_log(pw[p]) + loglik[p]);
     mx = block_max(mx, red);
     double s = 0.0;
-    for (int p = threadIdx.x; p < Np; p += blockDim.x) s += exp(safe_log(pw[p]) + loglik[p] - mx);
+#pragma unroll
+    for (int k = 0; k < HELD; ++k) {
+        const int p = threadIdx.x + k * blockDim.x;
+        if (p >= Np) break;
+        v[k] = exp(v[k] - mx);
+        s += v[k];
+    }
+    for (int p = p1; p < Np; p += blockDim.x) s += exp(safe_log(pw[p]) + loglik[p] - mx);
     s = block_sum(s, red);
     __syncthreads();
-    for (int p = threadIdx.x; p < Np; p += blockDim.x) pw[p] = exp(safe_log(pw[p]) + loglik[p] - mx) / s;
+#pragma unroll
+    for (int k = 0; k < HELD; ++k) {
+        const int p = threadIdx.x + k * blockDim.x;
+        if (p < Np) pw[p] = v[k] / s;
+    }
+    for (int p = p1; p < Np; p += blockDim.x) pw[p] = exp(safe_log(pw[p]) + loglik[p] - mx) / s;
 }
 
 /* ------------------------------------------------------ noise check */
@@ -2518,24 +2542,31 @@ __device__ inline void block_sum_n(double (&v)[N], double* sh) {
     __syncthreads();
 }
 
-/* One 256-thread workgroup per rig of Np parents: weighted mean and
+/* Twelve 256-thread workgroups per rig of Np parents: weighted mean and
  * covariance of the parent extrinsics and the summed Gaussian weight of the
  * first highest-weight parent's map (exp_traj, cov_traj and cardinality of
  * load_disparity_results.m:27-34).  out per rig: mean[12], cov[144]
- * row-major, cardinality (EST_DOUBLES). */
+ * row-major, cardinality (EST_DOUBLES).
+ *
+ * Bound: latency, of one pass over the parents for the mean and one for a row
+ * of the covariance and of their reductions, so each workgroup forms the mean
+ * and then a row of its own (one workgroup a rig, row after row: 47 us for 256
+ * parents, 11 so; 16384: 260 and 51). */
 __global__ __launch_bounds__(256) void k_estimate(const double* ext, const double* pw, const int32_t* goff,
                                                    const double* gw, int Np, const int32_t* poff, double* out) {
-    __shared__ double sh[4 * 78];
-    if (poff) { /* one workgroup per rig */
-        const int64_t P0 = poff[blockIdx.x];
-        Np = poff[blockIdx.x + 1] - poff[blockIdx.x];
+    __shared__ double sh[4 * 13];
+    __shared__ double s_mu[12];
+    __shared__ double bws[4];
+    __shared__ int bis[4];
+    const int row = blockIdx.x; /* of the covariance */
+    if (poff) { /* the rig's */
+        const int64_t P0 = poff[blockIdx.y];
+        Np = poff[blockIdx.y + 1] - poff[blockIdx.y];
         ext += P0 * 12;
         pw += P0;
         goff += P0;
-        out += (int64_t)blockIdx.x * EST_DOUBLES;
+        out += (int64_t)blockIdx.y * EST_DOUBLES;
     }
-    __shared__ double bws[4];
-    __shared__ int bis[4];
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
     double s1[13];
 #pragma unroll
@@ -2567,6 +2598,32 @@ __global__ __launch_bounds__(256) void k_estimate(const double* ext, const doubl
         bis[wv] = bi;
     }
     block_sum_n<13>(s1, sh);
+    const double W = s1[12];
+    const double r = W > 0 ? 1.0 / W : 0.0;
+    double mu[12];
+#pragma unroll
+    for (int c = 0; c < 12; ++c) mu[c] = s1[c] * r;
+    if (t == 0) {
+#pragma unroll
+        for (int c = 0; c < 12; ++c) s_mu[c] = mu[c];
+    }
+    __syncthreads();
+    const double mi = s_mu[row];
+    double v[12];
+#pragma unroll
+    for (int j = 0; j < 12; ++j) v[j] = 0.0;
+    for (int p = t; p < Np; p += 256) {
+        const double* x = ext + (int64_t)p * 12;
+        const double wdi = pw[p] * (x[row] - mi);
+#pragma unroll
+        for (int j = 0; j < 12; ++j) v[j] += wdi * (x[j] - mu[j]);
+    }
+    block_sum_n<12>(v, sh);
+    if (t == 0) {
+#pragma unroll
+        for (int j = 0; j < 12; ++j) out[12 + row * 12 + j] = v[j] * r;
+    }
+    if (row != 0) return;
     int best = bis[0];
     double bestw = bws[0];
     for (int k = 1; k < 4; ++k)
@@ -2574,33 +2631,12 @@ __global__ __launch_bounds__(256) void k_estimate(const double* ext, const doubl
             bestw = bws[k];
             best = bis[k];
         }
-    const double W = s1[12];
-    const double r = W > 0 ? 1.0 / W : 0.0;
-    double mu[12];
-#pragma unroll
-    for (int c = 0; c < 12; ++c) mu[c] = s1[c] * r;
-    /* covariance one row per pass (12 running sums per thread) */
-    for (int i = 0; i < 12; ++i) {
-        double row[12];
-#pragma unroll
-        for (int j = 0; j < 12; ++j) row[j] = 0.0;
-        for (int p = t; p < Np; p += 256) {
-            const double* x = ext + (int64_t)p * 12;
-            const double wdi = pw[p] * (x[i] - mu[i]);
-#pragma unroll
-            for (int j = 0; j < 12; ++j) row[j] += wdi * (x[j] - mu[j]);
-        }
-        block_sum_n<12>(row, sh);
-        if (t < 12) out[12 + i * 12 + t] = row[t] * r;
-    }
     double card[1] = {0.0};
     if (best < Np)
         for (int64_t g = goff[best] + t; g < goff[best + 1]; g += 256) card[0] += gw[g];
     block_sum_n<1>(card, sh);
-    if (t < 12) out[t] = mu[t];
-    if (t == 0) {
-        out[156] = card[0];
-    }
+    if (t < 12) out[t] = s_mu[t];
+    if (t == 0) out[156] = card[0];
 }
 
 /* ---------------------------------------------------- posterior samples */
@@ -3335,7 +3371,7 @@ hipError_t launch_debug_normals(hipStream_t s, NoiseKey key, uint32_t stream, ui
 hipError_t launch_estimate(hipStream_t s, const double* ext, const double* pw, const int32_t* goff,
                            const double* gw, int Np, const int32_t* poff, int nrigs, double* out) {
     if (poff ? nrigs <= 0 : Np <= 0) return hipErrorInvalidValue;
-    k_estimate<<<poff ? nrigs : 1, 256, 0, s>>>(ext, pw, goff, gw, Np, poff, out);
+    k_estimate<<<dim3(12, poff ? nrigs : 1), 256, 0, s>>>(ext, pw, goff, gw, Np, poff, out);
     LAUNCH_CHECK();
 }
 
