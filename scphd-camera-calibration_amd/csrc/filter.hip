@@ -1490,6 +1490,9 @@ int scphd_set_state(scphd_t* f, const double* states, const double* weights, con
     f->hint_ok = false;
     HIPTRY(hipMemcpyAsync(f->ext.p, states, (size_t)Np * 12 * sizeof(double), hipMemcpyHostToDevice, s));
     HIPTRY(hipMemcpyAsync(f->pw.p, weights, (size_t)Np * sizeof(double), hipMemcpyHostToDevice, s));
+    /* a bound on the maps however the call ends: k_eta's masks are sized by it */
+    const int max_map = *std::max_element(gcount, gcount + Np);
+    f->max_map = std::max(f->max_map, max_map);
     HIPTRY(hipMemcpyAsync(f->goff.p, off.data(), (size_t)(Np + 1) * sizeof(int32_t), hipMemcpyHostToDevice, s));
     if (Ng > 0) {
         HIPTRY(hipMemcpyAsync(f->gparent.p, par.data(), (size_t)Ng * sizeof(int32_t), hipMemcpyHostToDevice, s));
@@ -1512,7 +1515,7 @@ int scphd_set_state(scphd_t* f, const double* states, const double* weights, con
     HIPTRY(hipStreamSynchronize(s));
     flush_retired(f);
     f->Ng = Ng;
-    f->max_map = *std::max_element(gcount, gcount + Np);
+    f->max_map = max_map;
     f->n_predict = n_predict;
     f->n_update = n_update;
     f->n_resample = n_resample;

@@ -15,8 +15,7 @@ a master seed (--workload small: workloads.small_ragged_rigs, parents in
   budget allows (scphd_batch_*), and a rig leaves when its frames are done.
 * ensemble: the rigs are packed, in order, into groups whose summed
   footprint (scphd_rig_footprint at --growth times the expected map size)
-  fits --ensemble-gb and whose sample planes stay below 4 GiB (the kernels'
-  32-bit offset form); each group is one ensemble (scphd_create_ensemble),
+  fits --ensemble-gb and whose samples stay below 4 GiB a value; each group is one ensemble (scphd_create_ensemble),
   its buffers reserved for that size before the first frame, whose
   frames step every rig of the group with one launch per kernel; the groups
   run one after the other.  The C2 maps keep growing over 100 frames (terms

@@ -450,9 +450,9 @@ def run_ensemble(rigs, progress=None, growth=1.0):
 def pack_ensembles(rigs, budget_gb, growth=2.0, alone_parents=None, plane_bytes=4 << 30):
     """Split prepared rigs into ensembles, in order: a group closes when the
     next rig would take its summed footprint (scphd_rig_footprint at `growth`
-    times the expected map size) past budget_gb, or its sample planes (at
-    that size, with the buffers' growth slack of 1.25) past plane_bytes, the
-    limit of the kernels' 32-bit offsets.  Rigs with at least alone_parents
+    times the expected map size) past budget_gb, or one of the seven values
+    of its samples (at that size, with the buffers' growth slack of 1.25) past
+    plane_bytes, which keeps a group's buffers to a few large ones.  Rigs with at least alone_parents
     parents (when given) are returned apart, to run alone.  Returns (groups,
     alone)."""
     alone = [r for r in rigs if alone_parents is not None and r["p"]["n_particles"] >= alone_parents]
