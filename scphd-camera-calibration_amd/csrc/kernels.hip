@@ -260,51 +260,53 @@ __device__ inline void load_sample(const T* block, int S, int s, T r[7]) {
 }
 
 template <typename T>
-__global__ void k_materialize(Clouds<T> src, Clouds<T> dst, const int32_t* gblock, const int32_t* gparent,
-                              const int32_t* goff, int64_t Ng, int S, LinearCVMotionModel3D feat, double dt,
-                              RigKeys rk, uint64_t step, int arith32) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= Ng * S) return;
-    const int64_t g = i / S;
-    const int s = (int)(i - g * S);
-    const int p = gparent[g];
-    const int k = (int)(g - goff[p]);
-    T r[7];
-    load_sample<T>(src.block(gblock[g]), S, s, r);
-    T* const db = dst.block(g);
-    auto put = [&](int c, T v) { db[cloud_at(S, s, c)] = v; };
-    if (arith32) { /* the single-precision prediction of the FP32-arithmetic variant */
-        float x[6], n[3];
+__global__ __launch_bounds__(256) void k_materialize(Clouds<T> src, Clouds<T> dst, const int32_t* gblock,
+                                                     const int32_t* gparent, const int32_t* goff, int64_t Ng, int S,
+                                                     LinearCVMotionModel3D feat, double dt, RigKeys rk, uint64_t step,
+                                                     int arith32) {
+    /* a grid stride: a map may have more samples than a launch threads */
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < Ng * S; i += (int64_t)gridDim.x * 256) {
+        const int64_t g = i / S;
+        const int s = (int)(i - g * S);
+        const int p = gparent[g];
+        const int k = (int)(g - goff[p]);
+        T r[7];
+        load_sample<T>(src.block(gblock[g]), S, s, r);
+        T* const db = dst.block(g);
+        auto put = [&](int c, T v) { db[cloud_at(S, s, c)] = v; };
+        if (arith32) { /* the single-precision prediction of the FP32-arithmetic variant */
+            float x[6], n[3];
 #pragma unroll
-        for (int c = 0; c < 6; ++c) x[c] = (float)r[c];
-        if (!rk.keys) {
-            feature_normals(rk.key, step, (uint32_t)p, (uint32_t)k, (uint32_t)s, n);
+            for (int c = 0; c < 6; ++c) x[c] = (float)r[c];
+            if (!rk.keys) {
+                feature_normals(rk.key, step, (uint32_t)p, (uint32_t)k, (uint32_t)s, n);
+            } else {
+                int pl;
+                const LaneKey key = rk.of(p, pl);
+                feature_normals(key, step, (uint32_t)pl, (uint32_t)k, (uint32_t)s, n);
+            }
+            predict_f(x, motion_f(feat, dt), n);
+#pragma unroll
+            for (int c = 0; c < 6; ++c) put(c, (T)x[c]);
+            put(6, r[6]);
+            continue;
+        }
+        EuclideanPoint x{(double)r[0], (double)r[1], (double)r[2], (double)r[3], (double)r[4], (double)r[5]};
+        if (!rk.keys) { /* one rig: the key stays in scalar registers */
+            x = predict_sample(x, NoisyMotion(feat, dt), rk.key, step, (uint32_t)p, (uint32_t)k, (uint32_t)s);
         } else {
             int pl;
             const LaneKey key = rk.of(p, pl);
-            feature_normals(key, step, (uint32_t)pl, (uint32_t)k, (uint32_t)s, n);
+            x = predict_sample(x, NoisyMotion(feat, dt), key, step, (uint32_t)pl, (uint32_t)k, (uint32_t)s);
         }
-        predict_f(x, motion_f(feat, dt), n);
-#pragma unroll
-        for (int c = 0; c < 6; ++c) put(c, (T)x[c]);
+        put(0, (T)x.x);
+        put(1, (T)x.y);
+        put(2, (T)x.z);
+        put(3, (T)x.vx);
+        put(4, (T)x.vy);
+        put(5, (T)x.vz);
         put(6, r[6]);
-        return;
     }
-    EuclideanPoint x{(double)r[0], (double)r[1], (double)r[2], (double)r[3], (double)r[4], (double)r[5]};
-    if (!rk.keys) { /* one rig: the key stays in scalar registers */
-        x = predict_sample(x, NoisyMotion(feat, dt), rk.key, step, (uint32_t)p, (uint32_t)k, (uint32_t)s);
-    } else {
-        int pl;
-        const LaneKey key = rk.of(p, pl);
-        x = predict_sample(x, NoisyMotion(feat, dt), key, step, (uint32_t)pl, (uint32_t)k, (uint32_t)s);
-    }
-    put(0, (T)x.x);
-    put(1, (T)x.y);
-    put(2, (T)x.z);
-    put(3, (T)x.vx);
-    put(4, (T)x.vy);
-    put(5, (T)x.vz);
-    put(6, r[6]);
 }
 
 /* ------------------------------------------------------- reproject + fit */
@@ -3019,15 +3021,17 @@ __global__ void k_table_resample(const int32_t* anc, const int32_t* goff_old, co
 
 /* ------------------------------------------------------------ read-back */
 /* The map's clouds into consecutive blocks: block g of dst <- block
- * gblock[g] of src. */
+ * gblock[g] of src.  A workgroup a cloud at a time: a map has more values
+ * than a launch may have threads. */
 template <typename T>
-__global__ void k_gather(Clouds<T> src, Clouds<T> dst, const int32_t* gblock, int64_t Ng, int S) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+__global__ __launch_bounds__(256) void k_gather(Clouds<T> src, Clouds<T> dst, const int32_t* gblock, int64_t Ng,
+                                                int S) {
     const int n = 7 * S;
-    if (i >= Ng * n) return;
-    const int64_t g = i / n;
-    const int e = (int)(i - g * n);
-    dst.block(g)[e] = src.block(gblock[g])[e];
+    for (int64_t g = blockIdx.x; g < Ng; g += gridDim.x) {
+        const T* const from = src.block(gblock[g]);
+        T* const to = dst.block(g);
+        for (int e = threadIdx.x; e < n; e += 256) to[e] = from[e];
+    }
 }
 
 template <typename T>
@@ -3208,6 +3212,13 @@ __global__ void k_scan_add(int32_t* out, int64_t n, const int32_t* sums) {
 /* ============================================================ launchers */
 static inline unsigned nblocks(int64_t n, int t) { return (unsigned)((n + t - 1) / t); }
 
+/* the same, of a kernel whose workgroups stride over what is left: no more
+ * than the 2^32 - 1 threads a launch may have (more are taken modulo 2^32,
+ * without an error) */
+static inline unsigned nblocks_strided(int64_t n, int t) {
+    return (unsigned)std::min<int64_t>((n + t - 1) / t, 0xFFFFFFFFll / t);
+}
+
 #define LAUNCH_CHECK() return hipGetLastError()
 
 hipError_t launch_prior(hipStream_t s, double* ext, double* pw, int Np, const double* a12, const double* b12,
@@ -3248,8 +3259,8 @@ hipError_t launch_materialize(hipStream_t s, Clouds<T> src, Clouds<T> dst, const
                               LinearCVMotionModel3D feat, double dt, RigKeys key, uint64_t step, bool arith32) {
     if (Ng <= 0) return hipSuccess;
     if (arith32 && !std::is_same_v<T, float>) return hipErrorInvalidValue;
-    k_materialize<T><<<nblocks(Ng * S, 256), 256, 0, s>>>(src, dst, gblock, gparent, goff, Ng, S, feat, dt, key,
-                                                          step, arith32 ? 1 : 0);
+    k_materialize<T><<<nblocks_strided(Ng * S, 256), 256, 0, s>>>(src, dst, gblock, gparent, goff, Ng, S, feat, dt,
+                                                                  key, step, arith32 ? 1 : 0);
     LAUNCH_CHECK();
 }
 
@@ -3517,7 +3528,7 @@ hipError_t launch_table_resample(hipStream_t s, const int32_t* anc, const int32_
 template <typename T>
 hipError_t launch_gather(hipStream_t s, Clouds<T> src, Clouds<T> dst, const int32_t* gblock, int64_t Ng, int S) {
     if (Ng <= 0) return hipSuccess;
-    k_gather<T><<<nblocks(Ng * 7 * S, 256), 256, 0, s>>>(src, dst, gblock, Ng, S);
+    k_gather<T><<<nblocks_strided(Ng * 256, 256), 256, 0, s>>>(src, dst, gblock, Ng, S);
     LAUNCH_CHECK();
 }
 
