@@ -1483,39 +1483,72 @@ int scphd_set_state(scphd_t* f, const double* states, const double* weights, con
     if (off[Np] != n_gaussians) return fail(f, SCPHD_ERR_ARG, "gcount does not sum to n_gaussians");
     hipStream_t s = f->stream;
     const int64_t Ng = n_gaussians;
-    HIPTRY(f->goff.ensure(Np + 1));
-    HIPTRY(f->gparent.ensure(Ng + 1));
-    HIPTRY(f->gblock.ensure(Ng + 1));
-    HIPTRY(f->gw.ensure(Ng + 1));
-    f->hint_ok = false;
-    HIPTRY(hipMemcpyAsync(f->ext.p, states, (size_t)Np * 12 * sizeof(double), hipMemcpyHostToDevice, s));
-    HIPTRY(hipMemcpyAsync(f->pw.p, weights, (size_t)Np * sizeof(double), hipMemcpyHostToDevice, s));
-    /* a bound on the maps however the call ends: k_eta's masks are sized by it */
-    const int max_map = *std::max_element(gcount, gcount + Np);
-    f->max_map = std::max(f->max_map, max_map);
-    HIPTRY(hipMemcpyAsync(f->goff.p, off.data(), (size_t)(Np + 1) * sizeof(int32_t), hipMemcpyHostToDevice, s));
-    if (Ng > 0) {
-        HIPTRY(hipMemcpyAsync(f->gparent.p, par.data(), (size_t)Ng * sizeof(int32_t), hipMemcpyHostToDevice, s));
-        HIPTRY(hipMemcpyAsync(f->gw.p, wg, (size_t)Ng * sizeof(double), hipMemcpyHostToDevice, s));
-        HIPTRY(launch_iota(s, f->gblock.p, Ng));
-        HIPTRY(f->gen[f->cur].ensure(Ng, 0, S, f->esz, s));
-        const int64_t n = Ng * S;
-        void* dv = nullptr;
-        size_t db = (size_t)n * 7 * sizeof(double);
-        HIPTRY(cache_alloc(&dv, &db));
-        double* d = (double*)dv;
-        hipError_t e = hipMemcpyAsync(d, samples, (size_t)n * 7 * sizeof(double), hipMemcpyHostToDevice, s);
-        if (e == hipSuccess)
-            e = f->esz == 8 ? launch_inject<double>(s, d, Ng, S, f->gen[f->cur].clouds<double>(f->S))
-                            : launch_inject<float>(s, d, Ng, S, f->gen[f->cur].clouds<float>(f->S));
-        if (e == hipSuccess) e = hipStreamSynchronize(s);
+    /* Memory first, beside the current state, which a refusal leaves as it
+     * was: the new table goes into the successor's arrays, and the clouds
+     * into a generation of their own where the current one is too small (its
+     * slabs would be held until the call's end all the same). */
+    Generation& cur = f->gen[f->cur];
+    Generation grown;
+    grown.retired = &f->retired;
+    const int64_t n = Ng * S;
+    size_t db = (size_t)n * 7 * sizeof(double);
+    void* dv = nullptr;
+    auto drop = [&]() {
+        (void)hipStreamSynchronize(s);
+        (void)hipStreamSynchronize(f->side);
         retire(&f->retired, dv, db);
-        if (e != hipSuccess) return hipfail(f, e, "set_state");
+        grown.release();
+        flush_retired(f);
+    };
+    hipError_t e = f->goff2.ensure(Np + 1);
+    if (e == hipSuccess) e = f->gparent2.ensure(Ng + 1);
+    if (e == hipSuccess) e = f->gblock2.ensure(Ng + 1);
+    if (e == hipSuccess) e = f->gw2.ensure(Ng + 1);
+    if (e == hipSuccess && Ng > 0) e = cache_alloc(&dv, &db);
+    if (e == hipSuccess && Ng > cur.cap_blocks) e = grown.ensure(Ng, 0, S, f->esz, s);
+    if (e != hipSuccess) {
+        drop();
+        return hipfail(f, e, "set_state: memory");
     }
-    HIPTRY(hipStreamSynchronize(s));
+    const Generation& to = Ng > cur.cap_blocks ? grown : cur;
+    double* const d = (double*)dv;
+    auto copy = [&](void* dst, const void* src, size_t bytes) {
+        if (e == hipSuccess) e = hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s);
+    };
+    copy(f->goff2.p, off.data(), (size_t)(Np + 1) * sizeof(int32_t));
+    if (Ng > 0) {
+        copy(f->gparent2.p, par.data(), (size_t)Ng * sizeof(int32_t));
+        copy(f->gw2.p, wg, (size_t)Ng * sizeof(double));
+        copy(d, samples, (size_t)n * 7 * sizeof(double));
+        if (e == hipSuccess) e = launch_iota(s, f->gblock2.p, Ng);
+        if (e == hipSuccess)
+            e = f->esz == 8 ? launch_inject<double>(s, d, Ng, S, to.clouds<double>(S))
+                            : launch_inject<float>(s, d, Ng, S, to.clouds<float>(S));
+    }
+    copy(f->ext.p, states, (size_t)Np * 12 * sizeof(double));
+    copy(f->pw.p, weights, (size_t)Np * sizeof(double));
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    if (e != hipSuccess) {
+        /* the device failed part-way: what it holds is not known, the map is
+         * an empty one */
+        (void)hipMemsetAsync(f->goff.p, 0, (size_t)(Np + 1) * sizeof(int32_t), s);
+        drop();
+        f->Ng = 0;
+        f->max_map = 0;
+        f->hint_ok = f->pending = false;
+        return hipfail(f, e, "set_state");
+    }
+    std::swap(f->goff, f->goff2);
+    std::swap(f->gparent, f->gparent2);
+    std::swap(f->gblock, f->gblock2);
+    std::swap(f->gw, f->gw2);
+    if (Ng > cur.cap_blocks) std::swap(cur, grown);
+    retire(&f->retired, dv, db);
+    grown.release();
     flush_retired(f);
+    f->hint_ok = false;
     f->Ng = Ng;
-    f->max_map = max_map;
+    f->max_map = *std::max_element(gcount, gcount + Np);
     f->n_predict = n_predict;
     f->n_update = n_update;
     f->n_resample = n_resample;
