@@ -485,7 +485,7 @@ __device__ inline EuclideanPoint world_to_camera(const CameraPose& c, const Eucl
  * camera c, with the three quotients fx/z, fy/z, 1/z^2 taken from one
  * reciprocal 1/z (within a few ulps of the divisions). */
 __device__ inline DisparityPoint disparity_fast(const DisparityMeasurementModel& m, const CameraPose& c,
-                                                const EuclideanPoint& pw, bool xy = false) {
+                                                const EuclideanPoint& pw, bool xy) {
     const EuclideanPoint p = world_to_camera(c, pw, xy);
     const double iz = rcp_nr(p.z);
     const double fz = m.fx() * iz, gz = m.fy() * iz, iz2 = iz * iz;

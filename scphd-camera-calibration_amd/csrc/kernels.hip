@@ -349,12 +349,21 @@ __device__ inline void load_step(const T* p, int w, int lane, T r[7]) {
     }
 }
 
+/* The order of the sums of the samples s0 .. s0 + 15 of a cloud
+ * (world_to_camera): x, y, z in the second step of each triple of whole
+ * steps, whose end is whole_triples(S), y, x, z in the others.  Every kernel
+ * that judges whether the camera sees a sample goes by it, so that one on
+ * the image's edge is judged alike. */
+__device__ inline int whole_triples(int S) { return S - S % 48; }
+__device__ inline bool sums_xy(int s0, int triples) { return (uint32_t)s0 / 16 % 3 == 1 && s0 < triples; }
+
 /* One sample of a Gaussian's cloud: the deferred prediction applied, its
  * disparity-space point, its field-of-view flag and stored weight. */
 template <typename T, typename Key>
 __device__ inline void eval_sample(const FitArgs& a, const DisparityMeasurementModel& meas, const T r[7], Key kk,
-                                   int pl, int k, int s, const CameraPose& pose, EuclideanPoint& x, DisparityPoint& d,
-                                   bool& in, double& w, FeatureCarry* fc = nullptr, uint32_t phase = 0) {
+                                   int pl, int k, int s, const CameraPose& pose, bool xy, EuclideanPoint& x,
+                                   DisparityPoint& d, bool& in, double& w, FeatureCarry* fc = nullptr,
+                                   uint32_t phase = 0) {
     x = EuclideanPoint{(double)r[0], (double)r[1], (double)r[2], (double)r[3], (double)r[4], (double)r[5]};
     w = (double)r[6];
     if (a.pending) {
@@ -363,7 +372,7 @@ __device__ inline void eval_sample(const FitArgs& a, const DisparityMeasurementM
         else
             x = predict_sample(x, a.motion, kk, a.pstep, (uint32_t)pl, (uint32_t)k, (uint32_t)s);
     }
-    d = disparity_fast(meas, pose, x);
+    d = disparity_fast(meas, pose, x, xy);
     in = meas.inRange(d);
 }
 
@@ -616,7 +625,7 @@ __device__ inline void fit_row(const FitArgs& a, const ParentCtx& pc, int64_t g,
      * and at once loads the step two ahead into it.  Steps go in groups of
      * four, the noise group, so that a step's place in it (which normals it
      * draws and which it carries) is fixed. */
-    [[maybe_unused]] const int triples = S - S % 48;
+    [[maybe_unused]] const int triples = whole_triples(S);
     T buf[2][7];
     load_step(from, S, lane, buf[0]);
     load_step(from + 112, S - 16, lane, buf[1]);
@@ -668,11 +677,8 @@ __device__ inline void fit_row(const FitArgs& a, const ParentCtx& pc, int64_t g,
                 disparity_f(cx.m, cx.pose, x, q);
                 in = in_range_f(cx.m, q);
             } else {
-                /* the order of a point's sums by its place in triples of
-                 * whole steps */
-                const bool xy = (uint32_t)s0 / 16 % 3 == 1 && s0 < triples;
-                const DisparityPoint d =
-                    disparity_fast(meas, pose, EuclideanPoint{x[0], x[1], x[2], x[3], x[4], x[5]}, xy);
+                const DisparityPoint d = disparity_fast(
+                    meas, pose, EuclideanPoint{x[0], x[1], x[2], x[3], x[4], x[5]}, sums_xy(s0, triples));
                 in = meas.inRange(d);
                 q[0] = d.u; q[1] = d.v; q[2] = d.d; q[3] = d.vu; q[4] = d.vv; q[5] = d.vd;
             }
@@ -824,7 +830,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SCPHD_FIT_W
 
 /* The non-detection clouds of the terms k_fit decided only after its sweep
  * and kept, listed in ndfill[0, *ndfill_n): the predicted samples and the
- * weights 1 - pd_i, computed by the same code as in the sweep.  One 16-lane
+ * weights 1 - pd_i, the same bits as in the sweep.  One 16-lane
  * row per listed term; workgroups stride over the list (its length is read
  * on the device). */
 template <typename T, bool RG, typename A = double>
@@ -869,7 +875,8 @@ __global__ __launch_bounds__(256) void k_nd_fill(FitArgs a, Clouds<T> src, Cloud
                         EuclideanPoint x;
                         DisparityPoint d;
                         double sw;
-                        eval_sample(a, meas, r[j], kk, pl, k, s, pose, x, d, in, sw, &fc, (uint32_t)j);
+                        eval_sample(a, meas, r[j], kk, pl, k, s, pose, sums_xy(s0 + 16 * j, whole_triples(a.S)), x, d,
+                                    in, sw, &fc, (uint32_t)j);
                         const double xs[6] = {x.x, x.y, x.z, x.vx, x.vy, x.vz};
 #pragma unroll
                         for (int c = 0; c < 6; ++c) o[c * w] = (T)xs[c];
@@ -917,7 +924,7 @@ __global__ __launch_bounds__(256) void k_fit_fix(FitArgs a, Clouds<T> src, Cloud
                 DisparityPoint d;
                 bool in;
                 double w;
-                eval_sample(a, meas, r, kk, pl, k, s, pose, x, d, in, w);
+                eval_sample(a, meas, r, kk, pl, k, s, pose, false, x, d, in, w); /* a fit of its own: one order */
                 q[0] = d.u; q[1] = d.v; q[2] = d.d; q[3] = d.vu; q[4] = d.vv; q[5] = d.vd;
             }
         };
