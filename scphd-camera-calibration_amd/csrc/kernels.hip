@@ -2562,19 +2562,21 @@ __device__ inline void block_sum_n(double (&v)[N], double* sh) {
  * and then a row of its own (one workgroup a rig, row after row: 47 us for 256
  * parents, 11 so; 16384: 260 and 51). */
 __global__ __launch_bounds__(256) void k_estimate(const double* ext, const double* pw, const int32_t* goff,
-                                                   const double* gw, int Np, const int32_t* poff, double* out) {
+                                                   const double* gw, int Np, const int32_t* poff, int rig0,
+                                                   double* out) {
     __shared__ double sh[4 * 13];
     __shared__ double s_mu[12];
     __shared__ double bws[4];
     __shared__ int bis[4];
     const int row = blockIdx.x; /* of the covariance */
     if (poff) { /* the rig's */
-        const int64_t P0 = poff[blockIdx.y];
-        Np = poff[blockIdx.y + 1] - poff[blockIdx.y];
+        const int rig = rig0 + blockIdx.y;
+        const int64_t P0 = poff[rig];
+        Np = poff[rig + 1] - poff[rig];
         ext += P0 * 12;
         pw += P0;
         goff += P0;
-        out += (int64_t)blockIdx.y * EST_DOUBLES;
+        out += (int64_t)rig * EST_DOUBLES;
     }
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
     double s1[13];
@@ -3389,7 +3391,9 @@ hipError_t launch_debug_normals(hipStream_t s, NoiseKey key, uint32_t stream, ui
 hipError_t launch_estimate(hipStream_t s, const double* ext, const double* pw, const int32_t* goff,
                            const double* gw, int Np, const int32_t* poff, int nrigs, double* out) {
     if (poff ? nrigs <= 0 : Np <= 0) return hipErrorInvalidValue;
-    k_estimate<<<dim3(12, poff ? nrigs : 1), 256, 0, s>>>(ext, pw, goff, gw, Np, poff, out);
+    constexpr int SLICE = 65535; /* a grid's y has at most 65536 */
+    for (int r = 0; r < (poff ? nrigs : 1); r += SLICE)
+        k_estimate<<<dim3(12, poff ? std::min(nrigs - r, SLICE) : 1), 256, 0, s>>>(ext, pw, goff, gw, Np, poff, r, out);
     LAUNCH_CHECK();
 }
 
