@@ -238,7 +238,7 @@ struct EtaArgs {
     int32_t* mcnt;     /* Np*M detection terms kept per (parent, measurement) */
     /* the kept detection terms of a parent in pack order, at kcap p + i:
      * weight, (map index, measurement); knum[p] of them, -1 when there are
-     * more than kcap or k_eta made no list */
+     * more than kcap or no list was made */
     int32_t* knum;
     double* kw;
     int32_t* kjm;

@@ -1104,6 +1104,66 @@ __device__ inline double max_val(unsigned long long k) {
     return __longlong_as_double((long long)(k >> 63 ? k & ~(1ull << 63) : ~k));
 }
 
+/* A round's measurements by bin of v: the places of bin b are off[b] ..
+ * off[b + 1] - 1. */
+static constexpr int ETA_BINS = 128, ETA_CHUNK = 2048;
+struct EtaBins {
+    double scale;
+    int* off; /* ETA_BINS + 1, LDS */
+    int* cur; /* ETA_BINS, LDS */
+    __device__ EtaBins(const EtaArgs& a, int rig, int* o, int* c)
+        : scale(ETA_BINS / fabs(a.rig_meas ? a.rig_meas[rig].img_height() : a.img_height)), off(o), cur(c) {}
+    /* monotone in v, a NaN's the first */
+    __device__ int of(double v) const { return (int)fmin(fmax(v * scale, 0.0), (double)(ETA_BINS - 1)); }
+    /* fills the bins; returns the place of this thread's measurement (at v,
+     * when `valid`).  Begins with a barrier; off is whole after it. */
+    __device__ int fill(bool valid, double v) const {
+        const int t = threadIdx.x, b = of(v);
+        __syncthreads();
+        if (t < ETA_BINS) cur[t] = 0;
+        __syncthreads();
+        if (valid) atomicAdd(&cur[b], 1);
+        __syncthreads();
+        if (t < 64) { /* exclusive offsets, two bins a lane */
+            const int c0 = cur[2 * t], c1 = cur[2 * t + 1];
+            int x = c0 + c1;
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                const int y = __shfl_up(x, o, 64);
+                if (t >= o) x += y;
+            }
+            off[2 * t] = cur[2 * t] = x - c0 - c1;
+            off[2 * t + 1] = cur[2 * t + 1] = x - c1;
+            if (t == 63) off[ETA_BINS] = x;
+        }
+        __syncthreads();
+        return valid ? atomicAdd(&cur[b], 1) : 0;
+    }
+    /* the places [q0, q1) of the measurements that Gaussian record r may give
+     * l > L, or with `all` every one it may give any; the margins cover the
+     * rounding of l and of the window */
+    __device__ void window(const double* r, double L, bool all, int& q0, int& q1) const {
+        q0 = q1 = 0;
+        if (r[LK_OK] == 0.0) return;
+        const double ub = r[LK_C] - LOG_2PI - r[LK_H], over = ub - L + 1e-6 * (1.0 + fabs(ub));
+        if (!(over > 0.0)) return;
+        const double c = 0.5 * r[LK_S12], det = r[LK_S0] * r[LK_S3] - c * c;
+        const double hw = sqrt(2.000002 * over * (r[LK_S0] / det)) * 1.000001 + 1e-12 * fabs(r[LK_MUV]);
+        if (all || !(det > 1e-9 * r[LK_S0] * r[LK_S3]) || !(hw < 1e300) || r[LK_MUV] != r[LK_MUV]) {
+            q1 = off[ETA_BINS]; /* near singular: every measurement */
+        } else {
+            q0 = off[of(r[LK_MUV] - hw)];
+            q1 = off[of(r[LK_MUV] + hw) + 1];
+        }
+    }
+};
+
+__device__ inline void load_rec(const EtaArgs& a, int64_t g, double* r) {
+    const double* rec = a.lik + g * LK_COUNT;
+#pragma unroll
+    for (int q = 0; q < LK_COUNT; ++q) r[q] = rec[q];
+}
+
 /* Per parent: eta_{p,m} = log( sum_g exp(lw_{g,m}) + M w0 + kappa ) for
  * every measurement (normaliser reduce_by_key + log_sum_exp,
  * src/scphdcameracalibration.cu:1729-1768, exact per-parent segments), the
@@ -1133,15 +1193,14 @@ __device__ inline double max_val(unsigned long long k) {
  *      can no longer be kept leave the mask;
  *   4. the rest are listed, evaluated against eta, and those kept written
  *      in list order, which is the pack order.
- * Gaussians go in chunks of the mask's 2048 bits in 2 and 3; a map of more
- * than one chunk makes no list (4), and k_survivors sweeps it.
+ * Gaussians go in chunks of the mask's 2048 bits in 2 and 3; the list (4) of
+ * a map of more than one chunk is k_eta_list's.
  *
  * Bound: latency (LDS and the records' gathers), which is why the lists
  * spread the uneven terms over all lanes.  Ten frames of 4096 parents, 200
  * landmarks: 18.0 ms when every pair was evaluated twice and measurements
  * with more than eight candidate terms (one in seven) swept the map again,
  * 9.6 so. */
-static constexpr int ETA_BINS = 128, ETA_CHUNK = 2048;
 static constexpr double ETA_DROP = 60.0;
 
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_eta(EtaArgs a) {
@@ -1176,64 +1235,20 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_
     const double logw0 = a.births[rig].logw0;
     const bool birth_ok = a.births[rig].pd_ok != 0;
     const int rounds = (M + NT - 1) / NT;
-    const double bin_scale = ETA_BINS / fabs(a.rig_meas ? a.rig_meas[rig].img_height() : a.img_height);
+    const EtaBins bins(a, rig, s_off, s_cur);
     /* candidates: terms with l - max above the gate (less 1e-6), the only
      * ones that can pass it against eta >= max */
     const double cgate = a.lw_gate - 1e-6;
     const double drop = fmax(ETA_DROP, -cgate); /* no candidate is dropped */
-    /* monotone in v, a NaN's the first */
-    auto bin = [&](double v) { return (int)fmin(fmax(v * bin_scale, 0.0), (double)(ETA_BINS - 1)); };
-    /* the places [q0, q1) of the measurements that Gaussian record r may give
-     * l > L; the margins cover the rounding of l and of the window */
-    auto window = [&](const double* r, double L, int& q0, int& q1) {
-        q0 = q1 = 0;
-        if (r[LK_OK] == 0.0) return;
-        const double ub = r[LK_C] - LOG_2PI - r[LK_H], over = ub - L + 1e-6 * (1.0 + fabs(ub));
-        if (!(over > 0.0)) return;
-        const double c = 0.5 * r[LK_S12], det = r[LK_S0] * r[LK_S3] - c * c;
-        const double hw = sqrt(2.000002 * over * (r[LK_S0] / det)) * 1.000001 + 1e-12 * fabs(r[LK_MUV]);
-        if (a.sweep || !(det > 1e-9 * r[LK_S0] * r[LK_S3]) || !(hw < 1e300) || r[LK_MUV] != r[LK_MUV]) {
-            q1 = s_off[ETA_BINS]; /* near singular: every measurement */
-        } else {
-            q0 = s_off[bin(r[LK_MUV] - hw)];
-            q1 = s_off[bin(r[LK_MUV] + hw) + 1];
-        }
-    };
-    auto load_rec = [&](int j, double* r) {
-        const double* rec = a.lik + (g0 + j) * LK_COUNT;
-#pragma unroll
-        for (int q = 0; q < LK_COUNT; ++q) r[q] = rec[q];
-    };
     for (int r = 0; r < rounds; ++r) {
         const int m = r * NT + t;
         const bool valid = m < M;
         const double zu = valid ? a.zu[zb + m] : 0.0, zv = valid ? a.zv[zb + m] : 0.0;
         const int64_t pm = (int64_t)p * a.M + m;
-        /* the round's measurements by bin */
-        __syncthreads();
-        if (t < ETA_BINS) s_cur[t] = 0;
+        const int place = bins.fill(valid, zv);
         s_max[t] = max_key(bpc);
         s_cnt[t] = 0;
-        __syncthreads();
-        const int mb = bin(zv);
-        int place = 0;
-        if (valid) atomicAdd(&s_cur[mb], 1);
-        __syncthreads();
-        if (t < 64) { /* exclusive offsets, two bins a lane */
-            const int c0 = s_cur[2 * t], c1 = s_cur[2 * t + 1];
-            int x = c0 + c1;
-#pragma unroll
-            for (int o = 1; o < 64; o <<= 1) {
-                const int y = __shfl_up(x, o, 64);
-                if (t >= o) x += y;
-            }
-            s_off[2 * t] = s_cur[2 * t] = x - c0 - c1;
-            s_off[2 * t + 1] = s_cur[2 * t + 1] = x - c1;
-            if (t == 63) s_off[ETA_BINS] = x;
-        }
-        __syncthreads();
         if (valid) {
-            place = atomicAdd(&s_cur[mb], 1);
             s_zu[place] = zu;
             s_zv[place] = zv;
             s_m[place] = (uint16_t)t;
@@ -1242,9 +1257,9 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_
         /* 1. maxima */
         for (int j = t; j < G; j += NT) {
             double rec[LK_COUNT];
-            load_rec(j, rec);
+            load_rec(a, g0 + j, rec);
             int q, q1;
-            for (window(rec, bpc, q, q1); q < q1; ++q) {
+            for (bins.window(rec, bpc, a.sweep != 0, q, q1); q < q1; ++q) {
                 const double l = det_lw(rec, s_zu[q], s_zv[q]);
                 if (l > bpc) atomicMax(&s_max[s_m[q]], max_key(l));
             }
@@ -1310,9 +1325,9 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_
                 int blocks = 0;
                 if (lane < n) {
                     double rec[LK_COUNT];
-                    load_rec(jw + lane, rec);
+                    load_rec(a, g0 + jw + lane, rec);
                     int q0, q1;
-                    window(rec, bpc - drop, q0, q1);
+                    bins.window(rec, bpc - drop, a.sweep != 0, q0, q1);
                     if (q0 < q1) blocks = (2 << ((q1 - 1) >> 6)) - (1 << (q0 >> 6));
                     const double ub = rec[LK_C] - LOG_2PI - rec[LK_H];
                     wr[lane * REC] = rec[LK_MUU];
@@ -1361,7 +1376,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_
                     const uint32_t pr = s_pair[2 * q];
                     const int pl = (int)(pr >> 16), j = (int)(pr & 0xFFFFu);
                     double rec[LK_COUNT];
-                    load_rec(c0 + j, rec);
+                    load_rec(a, g0 + c0 + j, rec);
                     const double x = det_lw(rec, s_zu[pl], s_zv[pl]) - max_val(s_max[s_m[pl]]);
                     s_e[q] = x > -746.0 ? exp_nonpos(x) : 0.0;
                     if (!(x > cgate)) atomicAnd(&s_mask[pl * a.mask_stride + (j >> 5)], ~(1u << (j & 31)));
@@ -1408,7 +1423,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_
                         pr[i] = s_pair[2 * q];
                         const int pl = (int)(pr[i] >> 16), sl = s_m[pl];
                         double rec[LK_COUNT];
-                        load_rec((int)(pr[i] & 0xFFFFu), rec);
+                        load_rec(a, g0 + (int)(pr[i] & 0xFFFFu), rec);
                         const double x = det_lw(rec, s_zu[pl], s_zv[pl]) - __longlong_as_double((long long)s_max[sl]);
                         if (!(x > a.lw_gate)) continue;
                         const double wx = exp(x);
@@ -1438,7 +1453,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_
                 a.mcnt[pm] = s_cnt[t];
                 cnt += s_cnt[t];
             }
-        } else if (valid) { /* no list: sweep the map */
+        } else if (valid && (a.no_lists || G == 0)) { /* no list: sweep the map */
             int mcnt = 0;
             for (int j0 = 0; j0 < G; j0 += 4) {
                 const Lik4 R = load_lik4(a.lik, g0 + j0);
@@ -1467,6 +1482,108 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_
         a.nsurv[p] = (int32_t)sc;
         a.nkeep[p] = (int32_t)sn;
         a.knum[p] = lists && kept <= a.kcap ? kept : -1;
+    }
+}
+
+/* The kept detection terms of the parents with more Gaussians than k_eta's
+ * masks take (it has left their normalisers and birth terms), listed and
+ * counted as it does.  One workgroup per parent, 256 measurements a round: a
+ * Gaussian a lane meets the measurements that its window for the smallest
+ * weight covers, and the terms kept go into LDS as they are found; then they
+ * are put in pack order, by measurement (counts and offsets) and within one by
+ * their rank in map index.  A round of more than LATE_LIST terms makes no
+ * list, and k_survivors sweeps the map.
+ *
+ * Bound: latency of the few terms a lane meets.  Why a kernel of its own: the
+ * terms wait for eta, by when k_eta's masks hold the last chunk only.
+ * Normalisers and survivors of 256 parents, 2100 Gaussians and 200
+ * measurements: 0.96 ms when k_eta's count and k_survivors each evaluated
+ * every pair, 0.21 so; 64 parents, 8000 and 400: 5.9 and 1.1 ms. */
+static constexpr int LATE_LIST = 4096;
+struct LateList {
+    double w[LATE_LIST];
+    int32_t j[LATE_LIST];
+    uint16_t slot[LATE_LIST]; /* measurement in the round */
+    uint16_t by_m[LATE_LIST]; /* the terms, measurements ascending */
+};
+
+__global__ __launch_bounds__(NT) void k_eta_list(EtaArgs a) {
+    __shared__ int sh[8];
+    __shared__ double s_zu[NT], s_zv[NT], s_eta[NT]; /* by place */
+    __shared__ uint16_t s_m[NT];
+    __shared__ int s_cnt[NT], s_base[NT], s_fill[NT]; /* per measurement: terms kept, their offsets */
+    __shared__ int s_off[ETA_BINS + 1], s_cur[ETA_BINS], s_n;
+    extern __shared__ double s_dyn[];
+    LateList& l = *(LateList*)s_dyn;
+    const int p = blockIdx.x, t = threadIdx.x;
+    const int64_t g0 = a.goff[p];
+    const int G = a.goff[p + 1] - a.goff[p];
+    if (G <= ETA_CHUNK) return;
+    const int rig = a.moff ? a.prig[p] : 0;
+    const int M = a.moff ? a.moff[rig + 1] - a.moff[rig] : a.M;
+    const int64_t zb = a.moff ? a.moff[rig] : 0;
+    const double bpc = a.bpcs ? a.bpcs[rig] : a.bpc;
+    const EtaBins bins(a, rig, s_off, s_cur);
+    const double L = bpc + a.lw_gate - 1e-6; /* eta >= bpc */
+    int kept = 0;
+    bool listed = true;
+    for (int r = 0; r < (M + NT - 1) / NT; ++r) {
+        const int m = r * NT + t;
+        const bool valid = m < M;
+        const int64_t pm = (int64_t)p * a.M + m;
+        const double zv = valid ? a.zv[zb + m] : 0.0;
+        const int place = bins.fill(valid, zv);
+        s_cnt[t] = 0;
+        if (t == 0) s_n = 0;
+        if (valid) {
+            s_zu[place] = a.zu[zb + m];
+            s_zv[place] = zv;
+            s_eta[place] = a.eta[pm];
+            s_m[place] = (uint16_t)t;
+        }
+        __syncthreads();
+        for (int j = t; j < G; j += NT) {
+            double rec[LK_COUNT];
+            load_rec(a, g0 + j, rec);
+            int q, q1;
+            for (bins.window(rec, L, a.sweep != 0, q, q1); q < q1; ++q) {
+                const double x = det_lw(rec, s_zu[q], s_zv[q]) - s_eta[q];
+                if (!(x > a.lw_gate)) continue;
+                const double w = exp(x);
+                if (!(w >= a.min_weight)) continue;
+                const int sl = s_m[q], i = atomicAdd(&s_n, 1);
+                atomicAdd(&s_cnt[sl], 1);
+                if (i < LATE_LIST) {
+                    l.w[i] = w;
+                    l.j[i] = j;
+                    l.slot[i] = (uint16_t)sl;
+                }
+            }
+        }
+        __syncthreads();
+        const int n = s_n;
+        int tot;
+        s_base[t] = s_fill[t] = block_exscan(s_cnt[t], sh, &tot);
+        if (valid) a.mcnt[pm] = s_cnt[t];
+        listed = listed && n <= LATE_LIST && kept + n <= a.kcap;
+        if (listed) { /* uniform */
+            __syncthreads();
+            for (int i = t; i < n; i += NT) l.by_m[atomicAdd(&s_fill[l.slot[i]], 1)] = (uint16_t)i;
+            __syncthreads();
+            for (int i = t; i < n; i += NT) {
+                const int sl = l.slot[i], j = l.j[i], e0 = s_base[sl], e1 = e0 + s_cnt[sl];
+                int k = e0;
+                for (int e = e0; e < e1; ++e) k += l.j[l.by_m[e]] < j ? 1 : 0;
+                const int64_t o = p * a.kcap + kept + k;
+                a.kw[o] = l.w[i];
+                *(int2*)(a.kjm + 2 * o) = int2{j, r * NT + sl};
+            }
+        }
+        kept += n;
+    }
+    if (t == 0) {
+        a.nsurv[p] += kept;
+        a.knum[p] = listed ? kept : -1;
     }
 }
 
@@ -3351,6 +3468,7 @@ hipError_t launch_eta(hipStream_t s, EtaArgs a, int max_map) {
     const size_t mask = (size_t)std::min(std::max(a.M, 1), NT) * a.mask_stride * sizeof(uint32_t);
     a.list = mask + 4096 * sizeof(double) <= 68 * 1024 ? 4096 : 2048;
     k_eta<<<a.Np, NT, a.list * sizeof(double) + mask, s>>>(a);
+    if (max_map > ETA_CHUNK && !a.no_lists) k_eta_list<<<a.Np, NT, sizeof(LateList), s>>>(a);
     LAUNCH_CHECK();
 }
 
