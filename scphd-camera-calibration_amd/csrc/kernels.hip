@@ -2130,7 +2130,10 @@ __global__ __launch_bounds__(NT) void k_merge_groups(MergeArgs a, int lo, int hi
          *   with H = [I2 0] never raises the measured variance above R, and
          *   births carry R; the windows span a few pixels.)  q is rejected
          *   when it exceeds thr det by 0.1 % and by the single-precision
-         *   errors of both (below 1e-6 of their terms).
+         *   errors of both.  Those add up to at most 17 roundings of 2^-24 of
+         *   svv du^2 + suu dv^2 and 12 of suu svv (1.02e-6 and 0.72e-6; |suv|
+         *   of a sum is at most sqrt(suu svv), by Cauchy-Schwarz), so 2e-6 of
+         *   each covers them.
          *   Pairs with an ill-conditioned survivor are tested against all
          *   others. */
         const float thrf = (float)(1.0011 * thr);
@@ -2184,7 +2187,7 @@ __global__ __launch_bounds__(NT) void k_merge_groups(MergeArgs a, int lo, int hi
                 const float du = (float)(bu[q1] - u), dv = (float)(bv[q1] - v);
                 const float tuu = suu + auu, tuv = suv + bs[3 * q1 + 1], tvv = svv + bs[3 * q1 + 2];
                 const float x = tvv * du * du, y = tuu * dv * dv, w = tuu * tvv;
-                const bool far = x + y - 2.0f * tuv * du * dv - 1e-6f * (x + y) > thrf * (w - tuv * tuv + 1e-6f * w);
+                const bool far = x + y - 2.0f * tuv * du * dv - 2e-6f * (x + y) > thrf * (w - tuv * tuv + 2e-6f * w);
                 if (auu < 0.0f || far || (room = push(id[q], id[q1]))) near &= near - 1u;
             }
             while (room && e < nx) {
