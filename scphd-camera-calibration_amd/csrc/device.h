@@ -130,8 +130,9 @@ SCPHD_HD inline double uniform_oc(uint32_t lo, uint32_t hi) { /* (0, 1] */
  *
  * The kernels that draw normals are bound by VALU issue, and this is half of
  * their instructions, so its integer work is kept short: 51 instructions a
- * pair instead of 64 for the same bits (checked for every x0 and every
- * x1 >> 8).
+ * pair instead of 64.  The bits are those of the longer form, which counted
+ * leading zeros and moved the hardware's square root by an ulp where the
+ * residual said so (compared on the card for every x0 and every x1 >> 8).
  *   - x0 + 1 in double is exact, x0 = 2^32 - 1 included; its exponent and
  *     leading 23 fraction bits are one alignbit away from the layout of a
  *     float (the exponent modulo 256), and one add of 1.0's bits less those
@@ -142,11 +143,13 @@ SCPHD_HD inline double uniform_oc(uint32_t lo, uint32_t hi) { /* (0, 1] */
  *   - The quadrant's signs and the exchange of sin and cos are bits 31 and
  *     30 of x1 and of y = x1 ^ 2 x1. */
 
-/* The correctly rounded single-precision square root of x = -0 or x in
- * [2^-23, 89), the values of -2 log a: the hardware's 1/sqrt (within 1 ulp)
- * and one Goldschmidt step, whose residual x - g^2 is exact.  Checked
- * against the correctly rounded root for every a.  (x = -0 gives -0: its
- * reciprocal root is taken of a small positive number instead.) */
+/* The single-precision square root of x = -0 or x in [2^-23, 89), the values
+ * of -2 log a: the hardware's 1/sqrt (within 1 ulp) and one Goldschmidt step.
+ * From a correctly rounded 1/sqrt the result is the correctly rounded root of
+ * every x; from its neighbours it is an ulp off for 5 of 3e7 values, so that
+ * it rests on the hardware's choice: for every a it gave the bits of the
+ * corrected root.  (x = -0 gives -0: its reciprocal root is taken of a small
+ * positive number instead.) */
 __device__ inline float sqrt_rn_log(float x) {
     const float r = __builtin_amdgcn_rsqf(__builtin_fmaxf(x, 0x1p-64f));
     const float g = x * r, h = 0.5f * r;

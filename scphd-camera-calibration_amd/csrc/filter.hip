@@ -523,7 +523,7 @@ int update_t(scphd_filter* f, int M, int fixed) {
     ea.M = M;
     ea.Np = Np;
     ea.bpc = safe_log(M * P.birth_w0 + f->models.meas.kappa());
-    if (f->ensemble) { /* M is the largest rig's count, the stride of eta, mcnt, mncand and mcand */
+    if (f->ensemble) { /* M is the largest rig's count, the stride of eta and mcnt */
         ea.moff = f->dmoff.p;
         ea.bpcs = f->dbpcs.p;
         ea.prig = f->dprig.p;

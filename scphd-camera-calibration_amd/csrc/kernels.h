@@ -137,13 +137,13 @@ hipError_t launch_scale(hipStream_t s, double* x, int64_t n, double a);
 /* one rig's Np parents (weights 1 / Np) */
 hipError_t launch_prior(hipStream_t s, double* ext, double* pw, int Np, const double* a12, const double* b12,
                         NoiseKey key);
-/* rfixed (ensembles, may be null): per rig, the fixed camera for that rig
- * (rig of parent p: prig[p]); else `fixed` for every parent */
-/* goff, wave_parent (wave_count(goff[Np], Np) entries, written): the map
- * table's parent per wavefront of k_fit */
 /* an update's counters, zeroed by launch_pose: survivors miscounted, entries
  * listed in FitArgs::redo and FitArgs::ndfill */
 enum { UC_ERR, UC_REDO, UC_NDFILL, UC_COUNT };
+/* The update's cameras.  rfixed (ensembles, may be null): per rig, the fixed
+ * camera for that rig (rig of parent p: prig[p]); else `fixed` for every
+ * parent.  Of goff, wave_parent (wave_count(goff[Np], Np) entries, written):
+ * the map table's parent per wavefront of k_fit. */
 hipError_t launch_pose(hipStream_t s, const double* ext, double* pose, int Np, int fixed, const int32_t* prig,
                        const int32_t* rfixed, const int32_t* goff, int32_t* wave_parent, int32_t* counters);
 /* wavefronts (of four rows) that take n table entries of Np parents, none of

@@ -420,32 +420,6 @@ __device__ inline void write_fit(const FitArgs& a, int64_t g, int lane, const do
     }
 }
 
-/* Sixteen lanes (one row of a wavefront) per Gaussian, four Gaussians per
- * wavefront: deferred prediction, world -> disparity with the parent's
- * camera and the field-of-view Pd (worldToDisparityKernel,
- * src/kernels.cu:6-47), per-Gaussian Pd (computePdKernel :82-99), sample
- * reweighting by pd and normalisation (src/scphdcameracalibration.cu:1602-1608,
- * normalizeWeightsKernel src/kernels.cu:996-1018), and the weighted moment
- * fit (fitGaussiansKernel :102-438, covariance normaliser (W^2 + sum w^2) / W).
- *
- * Samples stream through once: each lane accumulates, with weights
- * w' = w pd, the sums of w', w'^2, w' (q - K) and w' (q - K)(q - K)^T about
- * a shift K, from which the normalised mean and centred covariance follow;
- * 30 row sums by DPP.  K is the first sample with w' > 0 (the first sample
- * when there is none).
- *
- * The non-detection cloud (kept when w_g (1 - pd_g) >= min_weight,
- * computeNonDetections src/scphdcameracalibration.cu:1290-1420; sample
- * weights 1 - pd_i; the samples themselves are the predicted cloud, which
- * the reference's world -> disparity -> world round trip reproduces to
- * rounding) is written during the sweep when the term is kept for certain,
- * w_g (1 - Pd) >= min_weight (pd_g <= Pd).  A term that may go either way
- * is decided after the sweep and, when kept, listed for k_nd_fill, which
- * writes its cloud; most such terms are dropped, and their clouds are never
- * written.  A cloud whose weights are all zero, which the reference
- * normalises to weight 1 per sample, is listed in redo[] and refitted by
- * k_fit_fix when pd_g > 0; with pd_g = 0 its fit cannot reach any output and
- * is the first sample with zero covariance. */
 /* The noise key of parent p and p's index in its rig: the kernel argument
  * (in scalar registers) for one rig, the rig's key per lane in an ensemble. */
 template <bool RG>
@@ -586,7 +560,34 @@ __device__ inline double row_total(A* part, const A (&v)[16], int lane) {
     return (double)x[0];
 }
 
-/* One row of k_fit, its Gaussian g of parent p (the same for every row of
+/* Sixteen lanes (one row of a wavefront) per Gaussian, four Gaussians per
+ * wavefront: deferred prediction, world -> disparity with the parent's
+ * camera and the field-of-view Pd (worldToDisparityKernel,
+ * src/kernels.cu:6-47), per-Gaussian Pd (computePdKernel :82-99), sample
+ * reweighting by pd and normalisation (src/scphdcameracalibration.cu:1602-1608,
+ * normalizeWeightsKernel src/kernels.cu:996-1018), and the weighted moment
+ * fit (fitGaussiansKernel :102-438, covariance normaliser (W^2 + sum w^2) / W).
+ *
+ * Samples stream through once: each lane accumulates, with weights
+ * w' = w pd, the sums of w', w'^2, w' (q - K) and w' (q - K)(q - K)^T about
+ * a shift K, from which the normalised mean and centred covariance follow;
+ * 30 row sums through LDS.  K is the first sample with w' > 0 (the first
+ * sample when there is none).
+ *
+ * The non-detection cloud (kept when w_g (1 - pd_g) >= min_weight,
+ * computeNonDetections src/scphdcameracalibration.cu:1290-1420; sample
+ * weights 1 - pd_i; the samples themselves are the predicted cloud, which
+ * the reference's world -> disparity -> world round trip reproduces to
+ * rounding) is written during the sweep when the term is kept for certain,
+ * w_g (1 - Pd) >= min_weight (pd_g <= Pd).  A term that may go either way
+ * is decided after the sweep and, when kept, listed for k_nd_fill, which
+ * writes its cloud; most such terms are dropped, and their clouds are never
+ * written.  A cloud whose weights are all zero, which the reference
+ * normalises to weight 1 per sample, is listed in redo[] and refitted by
+ * k_fit_fix when pd_g > 0; with pd_g = 0 its fit cannot reach any output and
+ * is the first sample with zero covariance.
+ *
+ * One row of k_fit, its Gaussian g of parent p (the same for every row of
  * the wavefront).
  * A, the arithmetic type of the per-sample work: double, or float for the
  * FP32-arithmetic variant (FP32 storage), whose moment sums are single
@@ -1182,7 +1183,9 @@ __device__ inline void load_rec(const EtaArgs& a, int64_t g, double* r) {
  *      Gaussians and few measurements each, a Gaussian a lane, an atomic
  *      maximum per measurement;
  *   2. l > max - 60 (L = bpc - 60; all terms below exp(-60) of the largest
- *      together are 1e-7 of an ulp of eta): about 30 measurements a
+ *      add up to 1.8e-23 at most, for 2048 of them: less than a quarter of an
+ *      ulp of eta where |eta| > 4e-7, and nearer to 0 far below the rounding
+ *      of max itself, a sum of terms about 1 to 10): about 30 measurements a
  *      Gaussian, but all of them for a few, so a wavefront takes a Gaussian
  *      at a time against its measurements in blocks of 64, held in registers,
  *      and collects a word of the measurements' masks, 32 Gaussians, in
@@ -2881,8 +2884,6 @@ __global__ __launch_bounds__(256) void k_sample(SampleKernArgs<T> ka) {
 }
 
 /* -------------------------------------------------------- map assembly */
-/* Map sizes after the update, and the posterior terms' wave_parent.  One
- * wavefront per parent. */
 /* The kept non-detection entries of a parent at keepoff[p] on, ndlist, the
  * others' blocks in holes (at the entry's index less the kept ones before
  * it), and the posterior's wave_parent.  One wavefront per parent. */
@@ -2907,6 +2908,10 @@ __global__ __launch_bounds__(256) void k_lists(const int32_t* keep, const int32_
     }
 }
 
+/* New map table per parent: [merged posterior Gaussians | kept
+ * non-detection Gaussians in input order] (recombineNonDetections,
+ * src/scphdcameracalibration.cu:1422-1574, weights w (1 - pd) for the
+ * non-detection terms, :1314-1318). */
 __global__ void k_table(TableArgs a) {
     const int64_t o = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (o >= a.Nout) return;
@@ -3541,6 +3546,7 @@ hipError_t launch_lists(hipStream_t s, const int32_t* keep, const int32_t* keepo
     k_lists<<<nblocks(Np, 4), 256, 0, s>>>(keep, keepoff, goff, Np, ndlist, holes, mergeoff, wave_parent);
     LAUNCH_CHECK();
 }
+
 hipError_t launch_table(hipStream_t s, const TableArgs& a) {
     if (a.Nout <= 0) return hipSuccess;
     k_table<<<nblocks(a.Nout, 256), 256, 0, s>>>(a);
@@ -3557,7 +3563,8 @@ hipError_t launch_resample(hipStream_t s, const ResampleArgs& a) {
  * mapped host memory, so that a read-back costs no copy-engine transfer:
  * out[0] = off[n], out[1] = the largest segment off[p + 1] - off[p],
  * out[2] = the number of segments above `limit` (0 when limit <= 0),
- * out[3] = *x0 and out[4] = *x1 (0 for a null pointer).  One workgroup. */
+ * out[3] = the largest of x0[0, n0) (0 when n0 = 0) and out[4] = *x1 (0 for a
+ * null pointer).  One workgroup. */
 __global__ __launch_bounds__(1024) void k_readout(const int32_t* off, int n, int32_t limit, const int32_t* x0, int n0,
                                                   const int32_t* x1, volatile int32_t* out) {
     int mx = 0, c = 0;
@@ -3569,6 +3576,9 @@ __global__ __launch_bounds__(1024) void k_readout(const int32_t* off, int n, int
     read_out(off[n], mx, c, x0, n0, x1, out);
 }
 
+/* out = the number of NaN entries of w[0, n) (checkStuff,
+ * src/scphdcameracalibration.cu:812-821, without the host copy).  One
+ * workgroup. */
 __global__ __launch_bounds__(1024) void k_nan_count(const double* w, int n, volatile int32_t* out) {
     __shared__ int sc[16];
     int c = 0;
@@ -3606,7 +3616,6 @@ hipError_t launch_nan_count(hipStream_t s, const double* w, int n, int32_t* out)
     k_nan_count<<<1, 1024, 0, s>>>(w, n, out);
     LAUNCH_CHECK();
 }
-
 
 hipError_t launch_resample_commit(hipStream_t s, double* ext, const double* ext_tmp, double* pw, int32_t* anc_out,
                                   const int32_t* anc, int N, int go) {
