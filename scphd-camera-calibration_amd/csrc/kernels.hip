@@ -1159,8 +1159,9 @@ struct EtaBins {
     }
 };
 
-__device__ inline void load_rec(const EtaArgs& a, int64_t g, double* r) {
-    const double* rec = a.lik + g * LK_COUNT;
+/* the record of entry j of the map from g0 on */
+__device__ inline void load_rec(const EtaArgs& a, int64_t g0, int j, double* r) {
+    const double* rec = a.lik + (g0 + j) * LK_COUNT;
 #pragma unroll
     for (int q = 0; q < LK_COUNT; ++q) r[q] = rec[q];
 }
@@ -1260,7 +1261,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_
         /* 1. maxima */
         for (int j = t; j < G; j += NT) {
             double rec[LK_COUNT];
-            load_rec(a, g0 + j, rec);
+            load_rec(a, g0, j, rec);
             int q, q1;
             for (bins.window(rec, bpc, a.sweep != 0, q, q1); q < q1; ++q) {
                 const double l = det_lw(rec, s_zu[q], s_zv[q]);
@@ -1328,7 +1329,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_
                 int blocks = 0;
                 if (lane < n) {
                     double rec[LK_COUNT];
-                    load_rec(a, g0 + jw + lane, rec);
+                    load_rec(a, g0, jw + lane, rec);
                     int q0, q1;
                     bins.window(rec, bpc - drop, a.sweep != 0, q0, q1);
                     if (q0 < q1) blocks = (2 << ((q1 - 1) >> 6)) - (1 << (q0 >> 6));
@@ -1379,7 +1380,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_
                     const uint32_t pr = s_pair[2 * q];
                     const int pl = (int)(pr >> 16), j = (int)(pr & 0xFFFFu);
                     double rec[LK_COUNT];
-                    load_rec(a, g0 + c0 + j, rec);
+                    load_rec(a, g0, c0 + j, rec);
                     const double x = det_lw(rec, s_zu[pl], s_zv[pl]) - max_val(s_max[s_m[pl]]);
                     s_e[q] = x > -746.0 ? exp_nonpos(x) : 0.0;
                     if (!(x > cgate)) atomicAnd(&s_mask[pl * a.mask_stride + (j >> 5)], ~(1u << (j & 31)));
@@ -1426,7 +1427,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_
                         pr[i] = s_pair[2 * q];
                         const int pl = (int)(pr[i] >> 16), sl = s_m[pl];
                         double rec[LK_COUNT];
-                        load_rec(a, g0 + (int)(pr[i] & 0xFFFFu), rec);
+                        load_rec(a, g0, (int)(pr[i] & 0xFFFFu), rec);
                         const double x = det_lw(rec, s_zu[pl], s_zv[pl]) - __longlong_as_double((long long)s_max[sl]);
                         if (!(x > a.lw_gate)) continue;
                         const double wx = exp(x);
@@ -1547,7 +1548,7 @@ __global__ __launch_bounds__(NT) void k_eta_list(EtaArgs a) {
         __syncthreads();
         for (int j = t; j < G; j += NT) {
             double rec[LK_COUNT];
-            load_rec(a, g0 + j, rec);
+            load_rec(a, g0, j, rec);
             int q, q1;
             for (bins.window(rec, L, a.sweep != 0, q, q1); q < q1; ++q) {
                 const double x = det_lw(rec, s_zu[q], s_zv[q]) - s_eta[q];
