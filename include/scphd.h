@@ -171,8 +171,9 @@ int scphd_get_maps(scphd_t* f, int32_t* gcount, double* wg, double* samples);
 
 /* Replace the whole filter state (parents, weights, maps, noise counters).
  * Arrays as in scphd_get_parents / scphd_get_maps; n_gaussians must equal the
- * sum of gcount.  No counterpart in the reference (its state is private);
- * used for lock-step comparison and rig snapshot/resume. */
+ * sum of gcount.  A snapshot that is refused, for its arguments or for memory,
+ * leaves the state as it was.  No counterpart in the reference (its state is
+ * private); used for lock-step comparison and rig snapshot/resume. */
 int scphd_set_state(scphd_t* f, const double* states, const double* weights,
                     const int32_t* gcount, int64_t n_gaussians, const double* wg,
                     const double* samples, int64_t n_predict, int64_t n_update,
