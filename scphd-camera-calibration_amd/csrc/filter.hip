@@ -747,7 +747,11 @@ int update_t(scphd_filter* f, int M, int fixed) {
 }
 
 int update_common(scphd_filter* f, int M, int fixed) {
-    int rc = f->esz == 8 ? update_t<double>(f, M, fixed) : update_t<float>(f, M, fixed);
+    const int rc = f->esz == 8 ? update_t<double>(f, M, fixed) : update_t<float>(f, M, fixed);
+    /* an update that failed before it joined the second stream (for memory)
+     * may have left k_nd_fill there, which reads and writes what the next
+     * call may hand back or overwrite */
+    if (rc != SCPHD_OK) (void)hipStreamSynchronize(f->side);
     return rc;
 }
 
