@@ -1488,12 +1488,14 @@ int scphd_set_state(scphd_t* f, const double* states, const double* weights, con
     hipStream_t s = f->stream;
     const int64_t Ng = n_gaussians;
     /* Memory first, beside the current state, which a refusal leaves as it
-     * was: the new table goes into the successor's arrays, and the clouds
-     * into a generation of their own where the current one is too small (its
-     * slabs would be held until the call's end all the same). */
+     * was: larger table arrays and a larger generation where the current ones
+     * are too small (which would be held until the call's end all the same),
+     * and the staging buffer. */
     Generation& cur = f->gen[f->cur];
-    Generation grown;
-    grown.retired = &f->retired;
+    Generation gen;
+    DBuf<int32_t> gparent, gblock;
+    DBuf<double> gw;
+    gen.retired = gparent.retired = gblock.retired = gw.retired = &f->retired;
     const int64_t n = Ng * S;
     size_t db = (size_t)n * 7 * sizeof(double);
     void* dv = nullptr;
@@ -1501,33 +1503,39 @@ int scphd_set_state(scphd_t* f, const double* states, const double* weights, con
         (void)hipStreamSynchronize(s);
         (void)hipStreamSynchronize(f->side);
         retire(&f->retired, dv, db);
-        grown.release();
+        gen.release();
+        gparent.release();
+        gblock.release();
+        gw.release();
         flush_retired(f);
     };
-    hipError_t e = f->goff2.ensure(Np + 1);
-    if (e == hipSuccess) e = f->gparent2.ensure(Ng + 1);
-    if (e == hipSuccess) e = f->gblock2.ensure(Ng + 1);
-    if (e == hipSuccess) e = f->gw2.ensure(Ng + 1);
+    hipError_t e = hipSuccess;
+    if (f->gparent.n < Ng + 1) e = gparent.ensure(Ng + 1);
+    if (e == hipSuccess && f->gblock.n < Ng + 1) e = gblock.ensure(Ng + 1);
+    if (e == hipSuccess && f->gw.n < Ng + 1) e = gw.ensure(Ng + 1);
     if (e == hipSuccess && Ng > 0) e = cache_alloc(&dv, &db);
-    if (e == hipSuccess && Ng > cur.cap_blocks) e = grown.ensure(Ng, 0, S, f->esz, s);
+    if (e == hipSuccess && Ng > cur.cap_blocks) e = gen.ensure(Ng, 0, S, f->esz, s);
     if (e != hipSuccess) {
         drop();
         return hipfail(f, e, "set_state: memory");
     }
-    const Generation& to = Ng > cur.cap_blocks ? grown : cur;
+    if (gparent.p) std::swap(f->gparent, gparent);
+    if (gblock.p) std::swap(f->gblock, gblock);
+    if (gw.p) std::swap(f->gw, gw);
+    if (Ng > cur.cap_blocks) std::swap(cur, gen);
     double* const d = (double*)dv;
     auto copy = [&](void* dst, const void* src, size_t bytes) {
         if (e == hipSuccess) e = hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s);
     };
-    copy(f->goff2.p, off.data(), (size_t)(Np + 1) * sizeof(int32_t));
+    copy(f->goff.p, off.data(), (size_t)(Np + 1) * sizeof(int32_t));
     if (Ng > 0) {
-        copy(f->gparent2.p, par.data(), (size_t)Ng * sizeof(int32_t));
-        copy(f->gw2.p, wg, (size_t)Ng * sizeof(double));
+        copy(f->gparent.p, par.data(), (size_t)Ng * sizeof(int32_t));
+        copy(f->gw.p, wg, (size_t)Ng * sizeof(double));
         copy(d, samples, (size_t)n * 7 * sizeof(double));
-        if (e == hipSuccess) e = launch_iota(s, f->gblock2.p, Ng);
+        if (e == hipSuccess) e = launch_iota(s, f->gblock.p, Ng);
         if (e == hipSuccess)
-            e = f->esz == 8 ? launch_inject<double>(s, d, Ng, S, to.clouds<double>(S))
-                            : launch_inject<float>(s, d, Ng, S, to.clouds<float>(S));
+            e = f->esz == 8 ? launch_inject<double>(s, d, Ng, S, cur.clouds<double>(S))
+                            : launch_inject<float>(s, d, Ng, S, cur.clouds<float>(S));
     }
     copy(f->ext.p, states, (size_t)Np * 12 * sizeof(double));
     copy(f->pw.p, weights, (size_t)Np * sizeof(double));
@@ -1542,14 +1550,7 @@ int scphd_set_state(scphd_t* f, const double* states, const double* weights, con
         f->hint_ok = f->pending = false;
         return hipfail(f, e, "set_state");
     }
-    std::swap(f->goff, f->goff2);
-    std::swap(f->gparent, f->gparent2);
-    std::swap(f->gblock, f->gblock2);
-    std::swap(f->gw, f->gw2);
-    if (Ng > cur.cap_blocks) std::swap(cur, grown);
-    retire(&f->retired, dv, db);
-    grown.release();
-    flush_retired(f);
+    drop();
     f->hint_ok = false;
     f->Ng = Ng;
     f->max_map = *std::max_element(gcount, gcount + Np);
